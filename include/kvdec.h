@@ -81,9 +81,11 @@ size_t kvdec_workspace_bytes(int kind, int64_t B, int32_t H, int32_t KVH,
  *   q, o : [B, H, D] dtype        k, v : [B, KVH, L, D] dtype
  *   head h reads KV head h / (H / KVH); H / KVH <= 16; D == 128.
  *   o = softmax(q k^T * sm_scale) v, fp32 softmax and accumulation.
- *   dtype KVDEC_F16 runs the MFMA kernels; KVDEC_BF16 and KVDEC_F32 (which
- *   the reference kernel also loads, dense_kernel.py:37,48-49) a generic
- *   kernel in fp32 arithmetic, output rounded once to dtype.
+ *   dtype KVDEC_F16 and KVDEC_BF16 run the MFMA kernels (bf16 from tensors
+ *   on 16-byte boundaries); KVDEC_F32 (which the reference kernel also loads,
+ *   dense_kernel.py:37,48-49) and other bf16 tensors a generic kernel in fp32
+ *   arithmetic, output rounded once to dtype.  bf16 and fp32 calls take any
+ *   workspace: a smaller one (or none) means fewer splits.
  */
 int kvdec_dense_decode(const void* q, const void* k, const void* v, void* o,
                        int dtype, int64_t B, int32_t H, int32_t KVH, int64_t L,
@@ -111,8 +113,7 @@ int kvdec_dense_decode_noalloc(const void* q, const void* k, const void* v, void
  * cache.  Replaces sparse_kernel.py:105-118 (sparse_decode_attention) and
  * sparse_kernel.py:67-102; slot validity follows _kv_indices
  * (sparse_kernel.py:15-46) for KVDEC_LAYOUT_LINEAR.  q, o and the caches
- * are all of dtype (KVDEC_F16: MFMA kernels; KVDEC_BF16 / KVDEC_F32: the
- * generic fp32 kernel, as for kvdec_dense_decode).
+ * are all of dtype (kernels and workspace as for kvdec_dense_decode).
  */
 int kvdec_sparse_decode(const void* q, const void* k_cache, const void* v_cache,
                         void* o, int dtype, int64_t B, int32_t H, int32_t KVH,

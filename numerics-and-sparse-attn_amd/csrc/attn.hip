@@ -116,9 +116,10 @@ __device__ __forceinline__ int grab(int* ctr, int lane) {
   return __builtin_amdgcn_readfirstlane(v);
 }
 
-// fp16 tiles [tile0, tile0 + n) of one region of one KV head; region row r
-// is slot slot_base + r.
-struct F16Items {
+// Tiles [tile0, tile0 + n) of 16-bit rows (element type E) of one region of
+// one KV head; region row r is slot slot_base + r.
+template <int E>
+struct RowItems {
   typedef F16Raw Raw;
   rsrc_t rk, rv;
   int tile0, n, slot_base;
@@ -134,16 +135,17 @@ struct F16Items {
   }
   typedef WaveState State;
   __device__ __forceinline__ void step(int i, const Raw& X, State& st, const StepCtx& c) const {
-    f16_tile_step(X, c.slot, c.qB, slot_base + kTile * tile(i), c.R, c.scale_log2, st, c.lane);
+    f16_tile_step<E>(X, c.slot, c.qB, slot_base + kTile * tile(i), c.R, c.scale_log2, st, c.lane);
   }
   // The same, in a wave whose quantized-tile accumulators qs share st.m.
   __device__ __forceinline__ void step(int i, const Raw& X, State& st, QState& qs,
                                        const StepCtx& c) const {
     const int lane = c.lane;
-    f16_tile_step(X, c.slot, c.qB, slot_base + kTile * tile(i), c.R, c.scale_log2, st, lane,
-                  [&](float alpha) { q_state_rescale(qs, alpha, lane); });
+    f16_tile_step<E>(X, c.slot, c.qB, slot_base + kTile * tile(i), c.R, c.scale_log2, st, lane,
+                     [&](float alpha) { q_state_rescale(qs, alpha, lane); });
   }
 };
+typedef RowItems<kEltF16> F16Items;
 
 // The accumulators a quantized tile updates.
 struct QRef {
@@ -233,12 +235,13 @@ __device__ __forceinline__ uint32_t row_off(int head, int chunk) {
   return (uint32_t)head * 512u + 16u * (uint32_t)(chunk ^ head);
 }
 
-// The fp16 output of 4 channels, stored non-temporally (written once and
+// The 16-bit output of 4 channels, stored non-temporally (written once and
 // not read in this kernel: no L2 line is left dirty for the end-of-kernel
 // release; KIVI W=256 5.83 -> 5.79 us, W=32 4.24 -> 4.20, sparse W=256
 // 7.51 -> 7.48).
-__device__ __forceinline__ void store_out4(_Float16* p, half4v h) {
-  __builtin_nontemporal_store(__builtin_bit_cast(u32x2, h), reinterpret_cast<u32x2*>(p));
+template <int E = kEltF16>
+__device__ __forceinline__ void store_out4(_Float16* p, float4v v) {
+  __builtin_nontemporal_store(round_elt4<E>(v), reinterpret_cast<u32x2*>(p));
 }
 
 __device__ __forceinline__ void publish_ml(const AttnCommon& P, WaveState& st, char* lds, int lane,
@@ -360,6 +363,7 @@ __device__ __forceinline__ void publish_q(const QState& qs, char* slot, int lane
 
 // Barrier, then combine the waves' published partials into the output (one
 // split) or the split's fp32 partial.
+template <int E>
 __device__ __forceinline__ void merge_out(const AttnCommon& P, char* lds, int64_t pair, int split) {
   __syncthreads();
   const float* sh_m = reinterpret_cast<const float*>(lds + kLdsM);
@@ -393,9 +397,7 @@ __device__ __forceinline__ void merge_out(const AttnCommon& P, char* lds, int64_
   }
   if (P.n_splits == 1) {
     const float inv = L > 0.f ? 1.0f / L : 0.f;   // L == 0: a sequence of length 0
-    half4v h = {(_Float16)(acc[0] * inv), (_Float16)(acc[1] * inv), (_Float16)(acc[2] * inv),
-                (_Float16)(acc[3] * inv)};
-    store_out4(P.o + ((size_t)b * P.H + (size_t)kvh * P.G + hn) * kHeadDim + 4 * ch, h);
+    store_out4<E>(P.o + ((size_t)b * P.H + (size_t)kvh * P.G + hn) * kHeadDim + 4 * ch, acc * inv);
   } else {
     const size_t idx = ((size_t)pair * P.n_splits + split) * P.G + hn;
     *reinterpret_cast<float4v*>(P.ws + idx * kHeadDim + 4 * ch) = acc;
@@ -438,9 +440,11 @@ __device__ __forceinline__ void f16_queue(const AttnCommon& P, const Items& it, 
   publish_f(P, st, c.slot, lane);
 }
 
-// fp16 rows: the dense cache [B, KVH, L, 128] or the compacted sparse cache
+// 16-bit rows: the dense cache [B, KVH, L, 128] or the compacted sparse cache
 // [B, KVH, sink+window, 128]; slot == row.
-struct F16Src {
+template <int E>
+struct RowsSrc {
+  static constexpr int kElt = E;
   const _Float16* k;
   const _Float16* v;
   int rows;
@@ -452,7 +456,7 @@ struct F16Src {
   template <class Sync>
   __device__ __forceinline__ void process(int64_t pair, int split, const AttnCommon& P, int wave,
                                           int lane, int* ctr, Sync&& sync, WaveState& st) const {
-    F16Items it;
+    RowItems<E> it;
     const size_t off = (size_t)pair * rows * kHeadDim;
     const uint32_t bytes = (uint32_t)rows * kRowBytes;
     it.rk = make_rsrc(k + off, bytes);
@@ -483,6 +487,7 @@ struct F16Src {
 // load zeros without touching memory).
 typedef __attribute__((address_space(4))) const int32_t cint32;
 
+template <int E>
 struct PagedItems {
   typedef F16Raw Raw;
   const char* kb;      // this KV head's origin (+ the sequence's when untabled)
@@ -531,14 +536,16 @@ struct PagedItems {
   }
   typedef WaveState State;
   __device__ __forceinline__ void step(int i, const Raw& X, State& st, const StepCtx& c) const {
-    f16_tile_step(X, c.slot, c.qB, kTile * (tile0 + i), c.R, c.scale_log2, st, c.lane);
+    f16_tile_step<E>(X, c.slot, c.qB, kTile * (tile0 + i), c.R, c.scale_log2, st, c.lane);
   }
 };
 
 // Per-sequence lengths over a paged or strided cache: dense attention over
 // the first len(b) tokens, or (sparse) the sink + window rule over a
 // compacted [sink + window] cache at position len(b).
+template <int E>
 struct PagedSrc {
+  static constexpr int kElt = E;
   const char* k;
   const char* v;
   const int32_t* bt;     // [B, max_blocks] or null
@@ -564,7 +571,7 @@ struct PagedSrc {
     const SlotRanges R = sparse ? sparse_ranges(len, window, sink, layout) : SlotRanges{len, 0, 0};
     const int n_slots = sparse ? sink + window : len;
     const int tiles = (n_slots + kTile - 1) / kTile;
-    PagedItems it;
+    PagedItems<E> it;
     it.kb = k + (int64_t)kvh * head_bytes + (bt ? 0 : b * page_bytes);
     it.vb = v + (int64_t)kvh * head_bytes + (bt ? 0 : b * page_bytes);
     it.bt = bt ? (cint32*)bt + b * max_blocks : nullptr;
@@ -885,6 +892,16 @@ struct has_qtiles : std::false_type {};
 template <class Src>
 struct has_qtiles<Src, decltype((void)Src::kPackQ)> : std::true_type {};
 
+// The element type of a source's rows, Q and output (fp16 unless it says).
+template <class Src, class = void>
+struct src_elt {
+  static constexpr int value = kEltF16;
+};
+template <class Src>
+struct src_elt<Src, decltype((void)Src::kElt)> {
+  static constexpr int value = Src::kElt;
+};
+
 template <class Src>
 __global__ __launch_bounds__(kThreads, 1) void attn_kernel(AttnCommon P, Src S) {
   extern __shared__ __align__(16) char lds[];
@@ -955,7 +972,7 @@ __global__ __launch_bounds__(kThreads, 1) void attn_kernel(AttnCommon P, Src S) 
   WaveState st;
   wave_state_init(st);
   S.process(pair, split, P, wave, lane, ctr, sync, st);
-  merge_out(P, lds, pair, split);
+  merge_out<src_elt<Src>::value>(P, lds, pair, split);
   if constexpr (has_arrive<Src>::value) S.arrive(pair, P);
 }
 
@@ -1083,7 +1100,7 @@ static_assert(LeanLds<kWaves>::kL == kLdsL && LeanLds<kWaves>::kSlots == kLdsSlo
 // published partials into the fp16 output rows of this KV head.  The waves
 // of bit mask SKIP (never wave 0) have had their partials combined into
 // another's.
-template <int NW = kWaves, unsigned SKIP = 0>
+template <int NW = kWaves, unsigned SKIP = 0, int E = kEltF16>
 __device__ __forceinline__ void lean_merge(const LeanCommon& C, const char* lds, uint32_t head) {
   typedef LeanLds<NW> Lds;
   static_assert((SKIP & 1u) == 0, "wave 0's partial is always read");
@@ -1116,9 +1133,7 @@ __device__ __forceinline__ void lean_merge(const LeanCommon& C, const char* lds,
     acc += ow[w] * f;
   }
   const float inv = L > 0.f ? 1.0f / L : 0.f;
-  half4v h = {(_Float16)(acc[0] * inv), (_Float16)(acc[1] * inv), (_Float16)(acc[2] * inv),
-              (_Float16)(acc[3] * inv)};
-  store_out4(C.o + ((size_t)head * C.G + hn) * kHeadDim + 4 * ch, h);
+  store_out4<E>(C.o + ((size_t)head * C.G + hn) * kHeadDim + 4 * ch, acc * inv);
   CLOCK_STAMP(C, 1);
 }
 
@@ -1189,7 +1204,7 @@ __device__ __forceinline__ void quad_premerge(int G, char* lds, int* count, int 
   }
 }
 
-// fp16 rows [heads][rows][128] (the compacted sink + window cache, or a
+// 16-bit rows [heads][rows][128] (the compacted sink + window cache, or a
 // short dense cache): wave w steps tiles w and w + 8 (at most 16 tiles).
 struct F16LeanArgs {
   LeanCommon c;
@@ -1198,7 +1213,7 @@ struct F16LeanArgs {
   int rows;
 };
 
-template <bool TAIL>
+template <bool TAIL, int E = kEltF16>
 __global__ __launch_bounds__(kThreads, 1) void f16_lean_kernel(F16LeanArgs A) {
   extern __shared__ __align__(16) char lds[];
   CLOCK_STAMP(A.c, 0);
@@ -1269,10 +1284,10 @@ __global__ __launch_bounds__(kThreads, 1) void f16_lean_kernel(F16LeanArgs A) {
         XT.k[i] = i == 0 ? tk : u32x4{0u, 0u, 0u, 0u};
         XT.v[i] = i < 4 ? tv[i] : u32x4{0u, 0u, 0u, 0u};
       }
-      f16_tile_step(XT, slot, qB, rows(2 * kWaves), A.c.R, A.c.scale_log2, st, lane);
+      f16_tile_step<E>(XT, slot, qB, rows(2 * kWaves), A.c.R, A.c.scale_log2, st, lane);
     }
-    f16_tile_step(X0, slot, qB, rows(wave), A.c.R, A.c.scale_log2, st, lane);
-    f16_tile_step(X1, slot, qB, rows(wave + kWaves), A.c.R, A.c.scale_log2, st, lane);
+    f16_tile_step<E>(X0, slot, qB, rows(wave), A.c.R, A.c.scale_log2, st, lane);
+    f16_tile_step<E>(X1, slot, qB, rows(wave + kWaves), A.c.R, A.c.scale_log2, st, lane);
   } else if (wave < n_tiles) {
     // a single tile in two phases: its V loads are issued once QK and the
     // softmax are done, so only the PV follows the last bytes to arrive
@@ -1282,15 +1297,15 @@ __global__ __launch_bounds__(kThreads, 1) void f16_lean_kernel(F16LeanArgs A) {
     load_f16_k(rk, T, lv, 0u, lane, X);
     q_in(true);
     uint32_t valid;
-    const TileProbs P = f16_tile_probs(X, slot, qB, T, A.c.R, A.c.scale_log2, st, lane, valid);
-    load_f16_v(rv, T, after_probs(lv, P), 0u, lane, X);
-    f16_tile_pv(X, P, valid, st);
+    const TileProbs<E> P = f16_tile_probs<E>(X, slot, qB, T, A.c.R, A.c.scale_log2, st, lane, valid);
+    load_f16_v(rv, T, after_probs<E>(lv, P), 0u, lane, X);
+    f16_tile_pv<E>(X, P, valid, st);
   } else {
     q_in(false);   // no tile, but waves 0..3 still provide their quarter
   }
   lean_publish_ml(A.c.G, st, lds, lane, wave);
   lean_publish_f(A.c.G, st, slot, lane);
-  lean_merge(A.c, lds, head);
+  lean_merge<kWaves, 0u, E>(A.c, lds, head);
 }
 
 // The fused KIVI decode with an fp16 residual of at most 128 rows (4 tiles;
@@ -1964,9 +1979,7 @@ __global__ __launch_bounds__(kWideThreads, 1) void kivi_wide_kernel(KiviLeanArgs
     }
   }
   const float inv = L > 0.f ? 1.0f / L : 0.f;
-  half4v h = {(_Float16)(acc[0] * inv), (_Float16)(acc[1] * inv), (_Float16)(acc[2] * inv),
-              (_Float16)(acc[3] * inv)};
-  store_out4(A.c.o + ((size_t)head * A.c.G + hn) * kHeadDim + 4 * ch, h);
+  store_out4(A.c.o + ((size_t)head * A.c.G + hn) * kHeadDim + 4 * ch, acc * inv);
   CLOCK_STAMP(A.c, 1);
 }
 
@@ -2066,6 +2079,7 @@ void launch_probe2_kind(int kind, bool upfront, unsigned blocks, size_t lds, hip
 }
 
 // Log-sum-exp merge of the split partials: one thread per output element.
+template <int E>
 __global__ __launch_bounds__(256) void merge_kernel(AttnCommon P) {
   const int64_t e = (int64_t)blockIdx.x * 256 + threadIdx.x;
   if (e >= P.pairs * P.G * kHeadDim) return;
@@ -2089,8 +2103,9 @@ __global__ __launch_bounds__(256) void merge_kernel(AttnCommon P) {
     L += wl[idx] * f;
     acc += wo[idx * kHeadDim + d] * f;
   }
-  __builtin_nontemporal_store((_Float16)(L > 0.f ? acc / L : 0.f),
-                              P.o + ((size_t)b * P.H + (size_t)kvh * P.G + hn) * kHeadDim + d);
+  const uint32_t bits = round_elt4<E>(float4v{L > 0.f ? acc / L : 0.f, 0.f, 0.f, 0.f})[0];
+  __builtin_nontemporal_store((uint16_t)bits, reinterpret_cast<uint16_t*>(P.o) +
+                                                  ((size_t)b * P.H + (size_t)kvh * P.G + hn) * kHeadDim + d);
 }
 
 // ---------------------------------------------------------------------------
@@ -2163,11 +2178,23 @@ ClockRef next_clock() {
 #define SET_CLOCK(args) ((void)0)
 #endif
 
+// A plan of at most as many splits as the workspace holds (bf16 callers may
+// pass none: one pass, slower for few KV heads).
+Plan fit_plan(Plan plan, int64_t pairs, int64_t n_tiles, int G, const void* ws, size_t ws_bytes) {
+  const size_t per_split = (size_t)pairs * G * (kHeadDim + 2) * sizeof(float);
+  const int64_t most = ws == nullptr ? 1 : (int64_t)(ws_bytes / per_split);
+  if (plan.splits <= most) return plan;
+  const int64_t s = most < 1 ? 1 : most, t = (n_tiles + s - 1) / s;
+  return Plan{(int)((n_tiles + t - 1) / t), (int)t};
+}
+
 template <class Src>
 int launch_attn(AttnCommon P, const Src& S, bool kivi, size_t ws_bytes, hipStream_t stream) {
+  constexpr int E = src_elt<Src>::value;
   // The KIVI plan never splits: its quantized and residual regions are
   // addressed per KV head, and the windows it serves are short.
-  const Plan plan = kivi ? Plan{1, P.n_tiles} : make_plan(P.pairs, P.n_tiles);
+  Plan plan = kivi ? Plan{1, P.n_tiles} : make_plan(P.pairs, P.n_tiles);
+  if (E == kEltBf16) plan = fit_plan(plan, P.pairs, P.n_tiles, P.G, P.ws, ws_bytes);
   P.n_splits = plan.splits;
   P.tiles_per_split = plan.tps;
   if (plan.splits > 1) {
@@ -2182,7 +2209,7 @@ int launch_attn(AttnCommon P, const Src& S, bool kivi, size_t ws_bytes, hipStrea
   int rc = launch_status();
   if (rc != KVDEC_OK || plan.splits == 1) return rc;
   const int64_t outs = P.pairs * P.G * kHeadDim;
-  hipLaunchKernelGGL(merge_kernel, dim3((unsigned)((outs + 255) / 256)), dim3(256), 0, stream, P);
+  hipLaunchKernelGGL(merge_kernel<E>, dim3((unsigned)((outs + 255) / 256)), dim3(256), 0, stream, P);
   return launch_status();
 }
 
@@ -2208,21 +2235,41 @@ bool f16_lean_fits(const AttnCommon& P, int64_t rows) {
   return make_plan(P.pairs, P.n_tiles).splits == 1 && tiles && P.pairs <= 0x7fffffffLL;
 }
 
-int launch_f16_lean(const AttnCommon& P, const _Float16* k, const _Float16* v, int rows,
-                    hipStream_t stream) {
+// q, k, v, o of E rows: the lean kernel or the split-K kernel.
+template <int E>
+int launch_rows(const AttnCommon& P, const void* k, const void* v, int64_t rows, size_t ws_bytes,
+                hipStream_t stream) {
+  const _Float16* kr = static_cast<const _Float16*>(k);
+  const _Float16* vr = static_cast<const _Float16*>(v);
+  if (!f16_lean_fits(P, rows)) {
+    const RowsSrc<E> S{kr, vr, (int)rows};
+    return launch_attn(P, S, false, ws_bytes, stream);
+  }
   F16LeanArgs A;
   A.c = lean_common(P);
-  A.k = k;
-  A.v = v;
-  A.rows = rows;
+  A.k = kr;
+  A.v = vr;
+  A.rows = (int)rows;
   SET_CLOCK(A.c);
   if (P.n_tiles > 2 * kWaves)
-    hipLaunchKernelGGL(f16_lean_kernel<true>, dim3((unsigned)P.pairs), dim3(kThreads), kLdsBytes + kQLdsBytes,
-                       stream, A);
+    hipLaunchKernelGGL((f16_lean_kernel<true, E>), dim3((unsigned)P.pairs), dim3(kThreads),
+                       kLdsBytes + kQLdsBytes, stream, A);
   else
-    hipLaunchKernelGGL(f16_lean_kernel<false>, dim3((unsigned)P.pairs), dim3(kThreads), kLdsBytes + kQLdsBytes,
-                       stream, A);
+    hipLaunchKernelGGL((f16_lean_kernel<false, E>), dim3((unsigned)P.pairs), dim3(kThreads),
+                       kLdsBytes + kQLdsBytes, stream, A);
   return launch_status();
+}
+
+// bf16 rows take the MFMA kernels (bound, like fp16's, by the reads of K and
+// V: B=4, L=16411 in 46.7 us with its merge, 5.8 TB/s, against 221.9 us on the
+// generic kernel, whose fp32 dot products keep the matrix cores idle) when
+// every tensor allows their 16-byte accesses; a tensor that starts at another
+// 2-byte boundary takes the generic kernel.
+bool aligned16(const void* a, const void* b, const void* c, const void* d) {
+  return (((uintptr_t)a | (uintptr_t)b | (uintptr_t)c | (uintptr_t)d) & 15u) == 0;
+}
+bool mfma_rows(int dtype, const void* q, const void* k, const void* v, const void* o) {
+  return dtype == KVDEC_F16 || (dtype == KVDEC_BF16 && aligned16(q, k, v, o));
 }
 
 // The fused KIVI decode at one length (lens null) or at per-sequence
@@ -2708,7 +2755,7 @@ int kvdec_dense_decode(const void* q, const void* k, const void* v, void* o, int
                        size_t ws_bytes, void* stream) {
   int rc = check_dense(q, k, v, o, dtype, B, H, KVH, L, D);
   if (rc) return rc;
-  if (dtype != KVDEC_F16)
+  if (!mfma_rows(dtype, q, k, v, o))
     return generic_rows_decode(q, k, v, o, dtype, B, H, KVH, L, SlotRanges{(int)L, 0, 0}, nullptr, false,
                                0, 0, KVDEC_LAYOUT_LINEAR, sm_scale, ws, ws_bytes,
                                static_cast<hipStream_t>(stream));
@@ -2723,11 +2770,9 @@ int kvdec_dense_decode(const void* q, const void* k, const void* v, void* o, int
   P.n_tiles = (int)tiles_for(KVDEC_KIND_DENSE, L);
   P.scale_log2 = (float)((double)sm_scale * 1.4426950408889634);
   P.R = SlotRanges{(int)L, 0, 0};
-  if (f16_lean_fits(P, L))
-    return launch_f16_lean(P, static_cast<const _Float16*>(k), static_cast<const _Float16*>(v), (int)L,
-                           static_cast<hipStream_t>(stream));
-  F16Src S{static_cast<const _Float16*>(k), static_cast<const _Float16*>(v), (int)L};
-  return launch_attn(P, S, false, ws_bytes, static_cast<hipStream_t>(stream));
+  const hipStream_t st = static_cast<hipStream_t>(stream);
+  return dtype == KVDEC_BF16 ? launch_rows<kEltBf16>(P, k, v, L, ws_bytes, st)
+                             : launch_rows<kEltF16>(P, k, v, L, ws_bytes, st);
 }
 
 int kvdec_read_probe(const void* src, int64_t bytes, void* sink, int32_t blocks, void* stream) {
@@ -2790,7 +2835,7 @@ int kvdec_sparse_decode(const void* q, const void* k_cache, const void* v_cache,
   if (layout == KVDEC_LAYOUT_RING && window < 1) return KVDEC_E_WINDOW;
   const int64_t n = (int64_t)window + sink;
   if (n * kRowBytes >= ((int64_t)1 << 31)) return KVDEC_E_SHAPE;
-  if (dtype != KVDEC_F16)
+  if (!mfma_rows(dtype, q, k_cache, v_cache, o))
     return generic_rows_decode(q, k_cache, v_cache, o, dtype, B, H, KVH, n,
                                sparse_ranges(seq_len, window, sink, layout), nullptr, true, window, sink,
                                layout, sm_scale, ws, ws_bytes, static_cast<hipStream_t>(stream));
@@ -2805,11 +2850,9 @@ int kvdec_sparse_decode(const void* q, const void* k_cache, const void* v_cache,
   P.n_tiles = (int)tiles_for(KVDEC_KIND_SPARSE, n);
   P.scale_log2 = (float)((double)sm_scale * 1.4426950408889634);
   P.R = sparse_ranges(seq_len, window, sink, layout);
-  if (f16_lean_fits(P, n))
-    return launch_f16_lean(P, static_cast<const _Float16*>(k_cache), static_cast<const _Float16*>(v_cache),
-                           (int)n, static_cast<hipStream_t>(stream));
-  F16Src S{static_cast<const _Float16*>(k_cache), static_cast<const _Float16*>(v_cache), (int)n};
-  return launch_attn(P, S, false, ws_bytes, static_cast<hipStream_t>(stream));
+  const hipStream_t st = static_cast<hipStream_t>(stream);
+  return dtype == KVDEC_BF16 ? launch_rows<kEltBf16>(P, k_cache, v_cache, n, ws_bytes, st)
+                             : launch_rows<kEltF16>(P, k_cache, v_cache, n, ws_bytes, st);
 }
 
 int kvdec_paged_decode(const void* q, const void* k_pages, const void* v_pages,
@@ -2843,7 +2886,7 @@ int kvdec_paged_decode(const void* q, const void* k_pages, const void* v_pages,
   P.G = H / KVH;
   P.n_tiles = (int)tiles_for(KVDEC_KIND_DENSE, max_seq_len);
   P.scale_log2 = (float)((double)sm_scale * 1.4426950408889634);
-  PagedSrc S{};
+  PagedSrc<kEltF16> S{};
   S.k = static_cast<const char*>(k_pages);
   S.v = static_cast<const char*>(v_pages);
   S.bt = block_table;
@@ -2873,7 +2916,7 @@ int kvdec_sparse_decode_varlen(const void* q, const void* k_cache, const void* v
   if (layout == KVDEC_LAYOUT_RING && window < 1) return KVDEC_E_WINDOW;
   const int64_t n = (int64_t)window + sink;
   if (n >= ((int64_t)1 << 30)) return KVDEC_E_SHAPE;
-  if (dtype != KVDEC_F16)
+  if (!mfma_rows(dtype, q, k_cache, v_cache, o))
     return generic_rows_decode(q, k_cache, v_cache, o, dtype, B, H, KVH, n, SlotRanges{0, 0, 0}, seq_lens,
                                true, window, sink, layout, sm_scale, ws, ws_bytes,
                                static_cast<hipStream_t>(stream));
@@ -2887,20 +2930,22 @@ int kvdec_sparse_decode_varlen(const void* q, const void* k_cache, const void* v
   P.G = H / KVH;
   P.n_tiles = (int)tiles_for(KVDEC_KIND_SPARSE, n);
   P.scale_log2 = (float)((double)sm_scale * 1.4426950408889634);
-  PagedSrc S{};
-  S.k = static_cast<const char*>(k_cache);
-  S.v = static_cast<const char*>(v_cache);
-  S.lens = seq_lens;
-  S.page_bytes = (int64_t)KVH * n * kRowBytes;
-  S.head_bytes = n * kRowBytes;
-  S.row_bytes = kRowBytes;
-  S.max_len = 0x3fffffff;
-  S.rows = (int)n;
-  S.window = window;
-  S.sink = sink;
-  S.layout = layout;
-  S.sparse = true;
-  return launch_attn(P, S, false, ws_bytes, static_cast<hipStream_t>(stream));
+  auto launch = [&](auto S) {
+    S.k = static_cast<const char*>(k_cache);
+    S.v = static_cast<const char*>(v_cache);
+    S.lens = seq_lens;
+    S.page_bytes = (int64_t)KVH * n * kRowBytes;
+    S.head_bytes = n * kRowBytes;
+    S.row_bytes = kRowBytes;
+    S.max_len = 0x3fffffff;
+    S.rows = (int)n;
+    S.window = window;
+    S.sink = sink;
+    S.layout = layout;
+    S.sparse = true;
+    return launch_attn(P, S, false, ws_bytes, static_cast<hipStream_t>(stream));
+  };
+  return dtype == KVDEC_BF16 ? launch(PagedSrc<kEltBf16>{}) : launch(PagedSrc<kEltF16>{});
 }
 
 int kvdec_sparse_decode_kivi(const void* q, const void* k_res, const void* v_res,

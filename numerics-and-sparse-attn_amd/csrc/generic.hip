@@ -1,8 +1,8 @@
 // Reference-semantics decode attention for gfx950, for what the MFMA kernels
 // of attn.hip do not take:
-//   - bf16 and fp32 queries and caches (dense_kernel.py:21-67 and
-//     sparse_kernel.py:67-102 load q, k, v in whatever dtype they are given,
-//     compute in fp32 and store o in q's dtype);
+//   - fp32 queries and caches, and bf16 ones off a 16-byte boundary
+//     (dense_kernel.py:21-67 and sparse_kernel.py:67-102 load q, k, v in
+//     whatever dtype they are given, compute in fp32 and store o in q's dtype);
 //   - KIVI caches of any code width and group size (quant_kernel.py:436-548,
 //     whose BITS and GROUP_SIZE are kernel parameters: QMAX = 2^BITS - 1,
 //     8 / BITS codes per byte).

@@ -103,8 +103,32 @@ __device__ __forceinline__ float group_max(float x) {
   return fmaxf(__builtin_bit_cast(float, (uint32_t)s32[0]), __builtin_bit_cast(float, (uint32_t)s32[1]));
 }
 
+// The 16-bit element types of a row cache.  Rows, Q and the tile operands are
+// moved as bits (half8 registers for both); the type decides the matrix
+// instruction, the split of the probabilities and the output's rounding.
+enum { kEltF16 = 0, kEltBf16 = 1 };
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+
+template <int E = kEltF16>
 __device__ __forceinline__ float4v mfma16x16x32(u32x4 a, half8 b, float4v c) {
-  return __builtin_amdgcn_mfma_f32_16x16x32_f16(as_h8(a), b, c, 0, 0, 0);
+  if constexpr (E == kEltBf16)
+    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c,
+                                                   0, 0, 0);
+  else
+    return __builtin_amdgcn_mfma_f32_16x16x32_f16(as_h8(a), b, c, 0, 0, 0);
+}
+
+// Four floats rounded to the element type, as bits.
+template <int E = kEltF16>
+__device__ __forceinline__ u32x2 round_elt4(float4v v) {
+  if constexpr (E == kEltBf16) {
+    typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
+    const bf16x4 h = {(__bf16)v[0], (__bf16)v[1], (__bf16)v[2], (__bf16)v[3]};
+    return __builtin_bit_cast(u32x2, h);
+  } else {
+    const half4v h = {(_Float16)v[0], (_Float16)v[1], (_Float16)v[2], (_Float16)v[3]};
+    return __builtin_bit_cast(u32x2, h);
+  }
 }
 
 // Packed KIVI layout, for query groups of at most kPackGroup heads: the MFMA
@@ -254,20 +278,28 @@ __device__ __forceinline__ uint32_t tile_valid_bits(const SlotRanges& R, int slo
 // remainder is exact in fp32), so the PV product carries p to ~2^-22
 // instead of fp16's 2^-11 (one dominant token would otherwise put that
 // whole rounding error into the output).
+// bf16 rows take three bf16 parts, p = pB + pM + pL with 8 bits each (both
+// remainders are exact in fp32): p to ~2^-25, as a third MFMA per product of a
+// path whose time is its memory traffic.
+template <int E = kEltF16>
 struct TileProbs {
   half8 pB, pL;
+};
+template <>
+struct TileProbs<kEltBf16> {
+  half8 pB, pM, pL;
 };
 
 // QK, masking and the online-softmax update of one tile (the first half of
 // tile_body): returns the tile's probabilities against the updated st.m.
-template <bool FULL, class KOp, class Resc>
-__device__ __forceinline__ TileProbs tile_probs(KOp&& kop, uint32_t valid, const half8 (&qB)[4],
+template <bool FULL, int E = kEltF16, class KOp, class Resc>
+__device__ __forceinline__ TileProbs<E> tile_probs(KOp&& kop, uint32_t valid, const half8 (&qB)[4],
                                                 float scale_log2, WaveState& st, Resc&& resc) {
   float4v s0 = {0.f, 0.f, 0.f, 0.f}, s1 = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
   for (int c = 0; c < 4; ++c) {
-    s0 = mfma16x16x32(kop(0, c), qB[c], s0);
-    s1 = mfma16x16x32(kop(1, c), qB[c], s1);
+    s0 = mfma16x16x32<E>(kop(0, c), qB[c], s0);
+    s1 = mfma16x16x32<E>(kop(1, c), qB[c], s1);
   }
 
   float x[8];
@@ -297,22 +329,38 @@ __device__ __forceinline__ TileProbs tile_probs(KOp&& kop, uint32_t valid, const
     st.m = mnew;
   }
 
-  TileProbs P;
+  TileProbs<E> P;
   float ls = 0.f;
+  if constexpr (E == kEltBf16) {
+    bf16x8 hi, mid, lo;
 #pragma unroll
-  for (int j = 0; j < 8; ++j) {
-    const float p = __builtin_amdgcn_exp2f(x[j] - st.m);
-    ls += p;
-    P.pB[j] = (_Float16)p;
-    P.pL[j] = (_Float16)__builtin_fmaf(-1.0f, (float)P.pB[j], p);
+    for (int j = 0; j < 8; ++j) {
+      const float p = __builtin_amdgcn_exp2f(x[j] - st.m);
+      ls += p;
+      hi[j] = (__bf16)p;
+      const float r = p - (float)hi[j];
+      mid[j] = (__bf16)r;
+      lo[j] = (__bf16)(r - (float)mid[j]);
+    }
+    P.pB = __builtin_bit_cast(half8, hi);
+    P.pM = __builtin_bit_cast(half8, mid);
+    P.pL = __builtin_bit_cast(half8, lo);
+  } else {
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      const float p = __builtin_amdgcn_exp2f(x[j] - st.m);
+      ls += p;
+      P.pB[j] = (_Float16)p;
+      P.pL[j] = (_Float16)__builtin_fmaf(-1.0f, (float)P.pB[j], p);
+    }
   }
   st.l += ls;
   return P;
 }
 
 // PV of one tile (the second half of tile_body).
-template <class VOp>
-__device__ __forceinline__ void tile_pv(VOp&& vop, const TileProbs& P, WaveState& st) {
+template <int E = kEltF16, class VOp>
+__device__ __forceinline__ void tile_pv(VOp&& vop, const TileProbs<E>& P, WaveState& st) {
 #pragma unroll
   for (int w = 0; w < 4; ++w) {
     uint32_t d[8];
@@ -326,18 +374,19 @@ __device__ __forceinline__ void tile_pv(VOp&& vop, const TileProbs& P, WaveState
       a[1] = __builtin_amdgcn_perm(d[3], d[2], sel);
       a[2] = __builtin_amdgcn_perm(d[5], d[4], sel);
       a[3] = __builtin_amdgcn_perm(d[7], d[6], sel);
-      st.O[2 * w + e] = mfma16x16x32(a, P.pB, st.O[2 * w + e]);
-      st.O[2 * w + e] = mfma16x16x32(a, P.pL, st.O[2 * w + e]);
+      st.O[2 * w + e] = mfma16x16x32<E>(a, P.pB, st.O[2 * w + e]);
+      if constexpr (E == kEltBf16) st.O[2 * w + e] = mfma16x16x32<E>(a, P.pM, st.O[2 * w + e]);
+      st.O[2 * w + e] = mfma16x16x32<E>(a, P.pL, st.O[2 * w + e]);
     }
   }
 }
 
-template <bool FULL, class KOp, class VOp, class Resc>
+template <bool FULL, int E = kEltF16, class KOp, class VOp, class Resc>
 __device__ __forceinline__ void tile_body(KOp&& kop, VOp&& vop, uint32_t valid,
                                           const half8 (&qB)[4], float scale_log2, WaveState& st,
                                           Resc&& resc) {
-  const TileProbs P = tile_probs<FULL>(kop, valid, qB, scale_log2, st, resc);
-  tile_pv(vop, P, st);
+  const TileProbs<E> P = tile_probs<FULL, E>(kop, valid, qB, scale_log2, st, resc);
+  tile_pv<E>(vop, P, st);
 }
 
 // ---------------------------------------------------------------------------
@@ -413,9 +462,9 @@ struct NoRescale {
   __device__ __forceinline__ void operator()(float) const {}
 };
 
-// Consume an fp16 tile.  V rows of masked tokens are replaced by zeros at use
+// Consume a 16-bit tile.  V rows of masked tokens are replaced by zeros at use
 // time: unwritten cache slots may hold anything, including non-finite values.
-template <class Resc = NoRescale>
+template <int E = kEltF16, class Resc = NoRescale>
 __device__ __forceinline__ void f16_tile_step(const F16Raw& X, char* slot, const half8 (&qB)[4],
                                               const TileRows& T, const SlotRanges& R, float scale_log2,
                                               WaveState& st, int lane, Resc&& resc = Resc()) {
@@ -427,11 +476,11 @@ __device__ __forceinline__ void f16_tile_step(const F16Raw& X, char* slot, const
     return *reinterpret_cast<const u32x4*>(slot + kslot_off(16u * blk + t, 4u * c + g));
   };
   if (tile_fully_valid(R, T)) {
-    tile_body<true>(kop, [&](int w, int j) { return X.v[j][w]; }, 0u, qB, scale_log2, st, resc);
+    tile_body<true, E>(kop, [&](int w, int j) { return X.v[j][w]; }, 0u, qB, scale_log2, st, resc);
   } else {
     const uint32_t valid = tile_valid_bits(R, T, kTile, lane);
-    tile_body<false>(kop, [&](int w, int j) { return ((valid >> j) & 1u) ? X.v[j][w] : 0u; },
-                     valid, qB, scale_log2, st, resc);
+    tile_body<false, E>(kop, [&](int w, int j) { return ((valid >> j) & 1u) ? X.v[j][w] : 0u; },
+                        valid, qB, scale_log2, st, resc);
   }
 }
 
@@ -441,7 +490,8 @@ __device__ __forceinline__ void f16_tile_step(const F16Raw& X, char* slot, const
 //   f16_tile_probs: stage K (X.k), QK, softmax; returns the probabilities
 //   and the tile's validity bits (all ones for a fully valid tile)
 //   f16_tile_pv:    PV from X.v (V rows of masked tokens read as zeros)
-__device__ __forceinline__ TileProbs f16_tile_probs(const F16Raw& X, char* slot, const half8 (&qB)[4],
+template <int E = kEltF16>
+__device__ __forceinline__ TileProbs<E> f16_tile_probs(const F16Raw& X, char* slot, const half8 (&qB)[4],
                                                     const TileRows& T, const SlotRanges& R, float scale_log2,
                                                     WaveState& st, int lane, uint32_t& valid) {
   const uint32_t t = lane & 15, g = lane >> 4;
@@ -453,18 +503,20 @@ __device__ __forceinline__ TileProbs f16_tile_probs(const F16Raw& X, char* slot,
   };
   if (tile_fully_valid(R, T)) {
     valid = 0xffu;
-    return tile_probs<true>(kop, 0u, qB, scale_log2, st, NoRescale());
+    return tile_probs<true, E>(kop, 0u, qB, scale_log2, st, NoRescale());
   }
   valid = tile_valid_bits(R, T, kTile, lane);
-  return tile_probs<false>(kop, valid, qB, scale_log2, st, NoRescale());
+  return tile_probs<false, E>(kop, valid, qB, scale_log2, st, NoRescale());
 }
-__device__ __forceinline__ void f16_tile_pv(const F16Raw& X, const TileProbs& P, uint32_t valid, WaveState& st) {
-  tile_pv([&](int w, int j) { return ((valid >> j) & 1u) ? X.v[j][w] : 0u; }, P, st);
+template <int E = kEltF16>
+__device__ __forceinline__ void f16_tile_pv(const F16Raw& X, const TileProbs<E>& P, uint32_t valid, WaveState& st) {
+  tile_pv<E>([&](int w, int j) { return ((valid >> j) & 1u) ? X.v[j][w] : 0u; }, P, st);
 }
 
 // A value the compiler must treat as depending on the tile's probabilities,
 // so that loads addressed with it are issued only after them.
-__device__ __forceinline__ bool after_probs(bool live, const TileProbs& P) {
+template <int E = kEltF16>
+__device__ __forceinline__ bool after_probs(bool live, const TileProbs<E>& P) {
   uint32_t x = live ? 1u : 0u;
   asm volatile("" : "+v"(x) : "v"(as_u4(P.pB)), "v"(as_u4(P.pL)));
   return x != 0u;
@@ -490,11 +542,11 @@ __device__ __forceinline__ void load_f16_v(rsrc_t rv, const TileRows& T, bool li
 }
 
 // The contiguous tile of slots slot0 .. slot0 + 31.
-template <class Resc = NoRescale>
+template <int E = kEltF16, class Resc = NoRescale>
 __device__ __forceinline__ void f16_tile_step(const F16Raw& X, char* slot, const half8 (&qB)[4],
                                               int slot0, const SlotRanges& R, float scale_log2,
                                               WaveState& st, int lane, Resc&& resc = Resc()) {
-  f16_tile_step(X, slot, qB, TileRows{slot0, 4}, R, scale_log2, st, lane, resc);
+  f16_tile_step<E>(X, slot, qB, TileRows{slot0, 4}, R, scale_log2, st, lane, resc);
 }
 
 // ---------------------------------------------------------------------------

@@ -21,8 +21,8 @@ def dense_decode_attention(q, k, v, seq_len, sm_scale=None):
     Mirrors dense_kernel.py:70-82.  Shapes are read from the tensors and
     checked (the reference takes them from constants.py); D_HEAD must be 128
     and N_HEADS / N_KV_HEADS <= 16.  Asynchronous on torch's current stream.
-    q, k, v share one dtype: fp16 runs the MFMA kernels; bf16 and fp32, which
-    the reference's kernel also loads (dense_kernel.py:37,48-49), run the
+    q, k, v share one dtype: fp16 and bf16 run the MFMA kernels; fp32, which
+    the reference's kernel also loads (dense_kernel.py:37,48-49), runs the
     generic fp32 kernel (output in q's dtype).
 
     Beyond the reference: ``seq_len`` may be a [BATCH] int32 tensor on the

@@ -24,7 +24,7 @@ def sparse_decode_attention(q, k_cache, v_cache, seq_len, window, sink=SINK_SIZE
 
     Mirrors sparse_kernel.py:105-118 (same arguments and defaults; ``layout``
     is an added keyword).  Contiguous, D_HEAD == 128; q and the caches share
-    one dtype: fp16 runs the MFMA kernels, bf16 and fp32 the generic fp32
+    one dtype: fp16 and bf16 run the MFMA kernels, fp32 the generic fp32
     kernel.  ``seq_len`` may also be a [BATCH] int32 tensor on the GPU: each
     sequence is masked at its own length (each >= 1).
     """
