@@ -58,6 +58,8 @@ extern "C" {
 #define KVDEC_KIND_DENSE 0       /* n_slots = seq_len                          */
 #define KVDEC_KIND_SPARSE 1      /* n_slots = sink + window                    */
 #define KVDEC_KIND_KIVI 2        /* n_slots = window                           */
+#define KVDEC_KIND_KIVI_SPLIT 3  /* n_slots = window - residual: the workspace
+                                    that lets few KV heads use the whole GPU   */
 
 /* Human-readable text for any return code (never NULL). */
 const char* kvdec_strerror(int code);
@@ -205,9 +207,10 @@ int kvdec_quantize_v(const void* x, int in_dtype, void* packed_u8,
  *   undefined by the reference, quant_kernel.py:589-590) means the whole
  *   window stays fp16: k_res / v_res hold the `window` window tokens and
  *   there are no window-old tokens.
- *   Runs in one pass (one workgroup per KV head): ws / ws_bytes are
- *   accepted for interface stability and ignored (kvdec_workspace_bytes
- *   returns 0 for KVDEC_KIND_KIVI).
+ *   Needs no workspace (kvdec_workspace_bytes returns 0 for KVDEC_KIND_KIVI):
+ *   one pass, one workgroup per KV head.  With one of
+ *   kvdec_workspace_bytes(KVDEC_KIND_KIVI_SPLIT, ...) bytes, long windows of
+ *   few KV heads are split over the GPU (a smaller one: over less of it).
  *   bits / group other than 2 / 32 (the tensors of kvdec_quantize_k / _v at
  *   that width, /4 above reading /pf) run a generic kernel in fp32
  *   arithmetic: 1 <= bits <= 8, D % group == 0, group % pf == 0,

@@ -31,7 +31,7 @@ LIB_PATH = os.path.join(_HERE, _LIBRARIES[_which])
 # element types / layouts / workspace kinds (include/kvdec.h)
 F16, F32, BF16 = 0, 1, 2
 LAYOUT_LINEAR, LAYOUT_RING = 0, 1
-KIND_DENSE, KIND_SPARSE, KIND_KIVI = 0, 1, 2
+KIND_DENSE, KIND_SPARSE, KIND_KIVI, KIND_KIVI_SPLIT = 0, 1, 2, 3
 
 _vp = ctypes.c_void_p
 _i32 = ctypes.c_int32

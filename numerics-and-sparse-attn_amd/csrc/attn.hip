@@ -25,6 +25,7 @@
 #include "kvdec_stream.h"
 #include "kvdec.h"
 
+#include <algorithm>
 #include <mutex>
 
 using namespace kvdec;
@@ -1868,30 +1869,61 @@ __device__ __forceinline__ void wide_publish_ml(int G, WaveState& st, char* lds,
   }
 }
 
-template <bool PACK>
-__global__ __launch_bounds__(kWideThreads, 1) void kivi_wide_kernel(KiviLeanArgs A) {
+// Few KV heads leave CUs idle (one workgroup each), and the time grows with
+// the groups of one workgroup (~0.2 us each).  SPLIT: workgroup blockIdx.x =
+// head * n_splits + s takes window-old groups first + s * per_split .. of its
+// head, the last one the residual and the sink group too, and leaves fp32
+// partials for merge_kernel (kivi_splits has the rule and what it measured).
+// VAR: each sequence's own length (lens) decides its valid slots; groups
+// before the first valid slot are neither read nor stepped.
+struct KiviWideArgs : KiviLeanArgs {
+  float* ws;               // SPLIT: partials, as AttnCommon::ws
+  const int32_t* lens;     // VAR: [B]
+  int64_t pairs;
+  int32_t n_splits, per_split;
+  int32_t first;           // first window-old group with a valid slot (0 with VAR)
+  int32_t KVH, window;
+};
+
+template <bool SPLIT, bool VAR>
+__global__ __launch_bounds__(kWideThreads, 1) void kivi_wide_kernel(KiviWideArgs A) {
   extern __shared__ __align__(16) char lds[];
   CLOCK_STAMP(A.c, 0);
+  constexpr bool PACK = true;
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const uint32_t head = blockIdx.x;
+  const uint32_t head = SPLIT ? blockIdx.x / (uint32_t)A.n_splits : blockIdx.x;
+  const uint32_t split = SPLIT ? blockIdx.x - head * (uint32_t)A.n_splits : 0u;
   half8 qB[4];
-  lean_prologue<KiviLeanArgs, PACK>(A.c, head, lane, qB);
+  lean_prologue<KiviWideArgs, PACK>(A.c, head, lane, qB);
   char* slot = lds + kWideLdsSlots + wave * kSlotBytes;
   int* ctr = reinterpret_cast<int*>(lds + kWideLdsCtr);
-  const int nwt = A.nwt, n_q = nwt + 1;
+  const int nwt = A.nwt;
+  SlotRanges R = A.c.R;
+  int first = A.first;
+  if constexpr (VAR) {
+    const int len = max((int)((cint32*)A.lens)[head / (uint32_t)A.KVH], 0);
+    R = sparse_ranges(len, A.window, A.sink, KVDEC_LAYOUT_LINEAR);
+    first = min((R.vb - A.sink) / kTile, nwt);
+  }
+  // this workgroup's items: window-old groups g0 .. g1 - 1, then (`tail`:
+  // the head's last split) the sink group as item g1
+  const int g1 = SPLIT ? min((int)(split + 1) * A.per_split + A.first, nwt) : nwt;
+  const int g0 = SPLIT ? min(max((int)split * A.per_split + A.first, first), g1) : first;
+  const bool tail = !SPLIT || (int)split == A.n_splits - 1;
+  const int n_q = tail ? g1 + 1 : g1;
   const QTensors Tw = q_tensors(A.winq, A.win_code_bytes, A.win_meta_bytes);
   const QTensors Ts = q_sink_tensors(A.sinkq, head, A.sink);
-  // item i < nwt: window-old group i; item nwt: the sink group
+  // item i < g1: window-old group i; item g1: the sink group
   auto load = [&](int i, QTileRaw& X) {
-    const bool sk = i == nwt;
+    const bool sk = i == g1;
     load_q_group(sk ? Ts : Tw, sk ? 0u : head * (uint32_t)nwt + (uint32_t)i, i < n_q, lane, X);
   };
-  if (threadIdx.x == 0) *ctr = kWideQWaves;
+  if (threadIdx.x == 0) *ctr = g0 + kWideQWaves;
   QTileRaw X;
   int i = n_q;
   if (wave < kWideQWaves) {
-    i = wave;
+    i = g0 + wave;
     load(i, X);
   }
   __syncthreads();
@@ -1902,14 +1934,14 @@ __global__ __launch_bounds__(kWideThreads, 1) void kivi_wide_kernel(KiviLeanArgs
     const int slot0 = A.sink + kTile * nwt + kTile * r;
     const rsrc_t rk = make_rsrc(A.kres, A.res_bytes), rv = make_rsrc(A.vres, A.res_bytes);
     const uint32_t soff = head * (uint32_t)(A.res_rows * kRowBytes);
-    const bool has = r * kTile < A.res_rows;
-    const uint32_t base = has && tile_any_valid(A.c.R, slot0) ? (uint32_t)r * kSlotBytes : kOOB;
+    const bool has = tail && r * kTile < A.res_rows;
+    const uint32_t base = has && tile_any_valid(R, slot0) ? (uint32_t)r * kSlotBytes : kOOB;
     WaveState sf;
     wave_state_init(sf);
     if (has) {
       F16Raw F;
       load_f16(rk, rv, base, soff, lane, F);
-      f16_tile_step(F, slot, qB, slot0, A.c.R, A.c.scale_log2, sf, lane);
+      f16_tile_step(F, slot, qB, slot0, R, A.c.scale_log2, sf, lane);
     }
     wide_publish_ml(A.c.G, sf, lds, lane, kWideWaves + r);
     lean_publish_f(A.c.G, sf, lds + kWideLdsF16 + r * kWideF16Bytes, lane);
@@ -1926,17 +1958,16 @@ __global__ __launch_bounds__(kWideThreads, 1) void kivi_wide_kernel(KiviLeanArgs
   // window-old groups; the sink group (claimed last, at most 16 tokens: the
   // host's condition) is stepped after the loop, so that the loop holds one
   // tile body (with two, the registers of 4 waves per SIMD do not suffice)
-  while (i < nwt) {
+  while (i < g1) {
     const float slack = q_tile_stage(X, slot, lane);
     const int nx = grab(ctr, lane);
     load(nx, X);
-    q_tile_body<false, false, PACK>(slot, qB, A.sink + kTile * i, kTile, A.c.R, sl2, slack, st, qs,
-                                    lane);
+    q_tile_body<false, false, PACK>(slot, qB, A.sink + kTile * i, kTile, R, sl2, slack, st, qs, lane);
     i = nx;
   }
-  if (i == nwt) {
+  if (i == g1 && tail) {
     const float slack = q_tile_stage(X, slot, lane);
-    q_tile_body<false, true, PACK>(slot, qB, 0, A.sink, A.c.R, sl2, slack, st, qs, lane);
+    q_tile_body<false, true, PACK>(slot, qB, 0, A.sink, R, sl2, slack, st, qs, lane);
   }
   wide_publish_ml(A.c.G, st, lds, lane, wave);
   publish_q<false, PACK>(qs, slot, lane);
@@ -1978,8 +2009,17 @@ __global__ __launch_bounds__(kWideThreads, 1) void kivi_wide_kernel(KiviLeanArgs
       acc += ow[j] * f;
     }
   }
-  const float inv = L > 0.f ? 1.0f / L : 0.f;
-  store_out4(A.c.o + ((size_t)head * A.c.G + hn) * kHeadDim + 4 * ch, acc * inv);
+  if constexpr (SPLIT) {
+    const size_t units = (size_t)A.pairs * A.n_splits * A.c.G, u = (size_t)blockIdx.x * A.c.G + hn;
+    *reinterpret_cast<float4v*>(A.ws + u * kHeadDim + 4 * ch) = acc;
+    if (ch == 0) {
+      A.ws[units * kHeadDim + u] = M;
+      A.ws[units * kHeadDim + units + u] = L;
+    }
+  } else {
+    const float inv = L > 0.f ? 1.0f / L : 0.f;
+    store_out4(A.c.o + ((size_t)head * A.c.G + hn) * kHeadDim + 4 * ch, acc * inv);
+  }
   CLOCK_STAMP(A.c, 1);
 }
 
@@ -2078,34 +2118,68 @@ void launch_probe2_kind(int kind, bool upfront, unsigned blocks, size_t lds, hip
   }
 }
 
-// Log-sum-exp merge of the split partials: one thread per output element.
+// Log-sum-exp merge of the split partials: one workgroup per output row
+// (query head of a sequence), whose four waves share its splits, each lane two
+// channels.  The partials were written moments before, so the kernel is bound
+// by its round trips: every wave finds the row's maximum itself (lane s reads
+// split s's) while its first four partials are on their way (bf16 dense, B=4,
+// L=16411, 8 splits of 256 rows: 46.7 -> 45.4 us for the call against one
+// thread per output walking the splits in turn).
+constexpr int kMergeWaves = 4;
 template <int E>
-__global__ __launch_bounds__(256) void merge_kernel(AttnCommon P) {
-  const int64_t e = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  if (e >= P.pairs * P.G * kHeadDim) return;
-  const int d = (int)(e % kHeadDim);
-  const int hn = (int)((e / kHeadDim) % P.G);
-  const int64_t pair = e / ((int64_t)kHeadDim * P.G);
-  const int64_t b = pair / P.KVH;
-  const int kvh = (int)(pair % P.KVH);
-  const size_t total = (size_t)P.pairs * P.n_splits * P.G;
-  const float* wo = P.ws;
+__global__ __launch_bounds__(64 * kMergeWaves) void merge_kernel(AttnCommon P) {
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const uint32_t row = blockIdx.x, pair = row / (uint32_t)P.G;   // row = pair * G + head of the group
+  const int hn = (int)(row - pair * (uint32_t)P.G), S = P.n_splits;
+  const size_t total = (size_t)P.pairs * S * P.G;
+  const size_t base = (size_t)pair * S * P.G + hn;               // split s: base + s * G
+  const float* wo = P.ws + 2 * lane;
   const float* wm = P.ws + total * kHeadDim;
   const float* wl = wm + total;
-  const size_t base = (size_t)pair * P.n_splits * P.G + hn;
+  constexpr int kIn = 4;   // partials in flight per wave
+  float2v a[kIn];
+  float ms[kIn], ls[kIn];
+  auto fetch = [&](int s0) {
+#pragma unroll
+    for (int j = 0; j < kIn; ++j) {
+      const int s = s0 + kMergeWaves * j;
+      const size_t u = base + (size_t)(s < S ? s : 0) * P.G;
+      a[j] = *reinterpret_cast<const float2v*>(wo + u * kHeadDim);
+      ms[j] = s < S ? wm[u] : -INFINITY;
+      ls[j] = wl[u];
+    }
+  };
+  fetch(wave);
   float M = kMaxSentinel;
-  for (int s = 0; s < P.n_splits; ++s) M = fmaxf(M, wm[base + (size_t)s * P.G]);
-  float L = 0.f, acc = 0.f;
-#pragma unroll 4
-  for (int s = 0; s < P.n_splits; ++s) {
-    const size_t idx = base + (size_t)s * P.G;
-    const float f = __builtin_amdgcn_exp2f(wm[idx] - M);
-    L += wl[idx] * f;
-    acc += wo[idx * kHeadDim + d] * f;
+  for (int s = lane; s < S; s += 64) M = fmaxf(M, wm[base + (size_t)s * P.G]);
+#pragma unroll
+  for (int off = 32; off >= 1; off >>= 1) M = fmaxf(M, __shfl_xor(M, off));
+  float L = 0.f;
+  float2v acc = {0.f, 0.f};
+  for (int s0 = wave; s0 < S; s0 += kMergeWaves * kIn) {
+    if (s0 != wave) fetch(s0);
+#pragma unroll
+    for (int j = 0; j < kIn; ++j) {
+      const float f = __builtin_amdgcn_exp2f(ms[j] - M);   // 0 past the last split
+      L += ls[j] * f;
+      acc += a[j] * f;
+    }
   }
-  const uint32_t bits = round_elt4<E>(float4v{L > 0.f ? acc / L : 0.f, 0.f, 0.f, 0.f})[0];
-  __builtin_nontemporal_store((uint16_t)bits, reinterpret_cast<uint16_t*>(P.o) +
-                                                  ((size_t)b * P.H + (size_t)kvh * P.G + hn) * kHeadDim + d);
+  __shared__ float2v part[kMergeWaves][64];
+  __shared__ float part_l[kMergeWaves];
+  part[wave][lane] = acc;
+  if (lane == 0) part_l[wave] = L;
+  __syncthreads();
+  if (wave != 0) return;
+#pragma unroll
+  for (int w = 1; w < kMergeWaves; ++w) {
+    acc += part[w][lane];
+    L += part_l[w];
+  }
+  const float inv = L > 0.f ? 1.0f / L : 0.f;
+  const uint32_t bits = round_elt4<E>(float4v{acc[0] * inv, acc[1] * inv, 0.f, 0.f})[0];
+  __builtin_nontemporal_store(bits, reinterpret_cast<uint32_t*>(P.o) + (size_t)row * (kHeadDim / 2) + lane);
 }
 
 // ---------------------------------------------------------------------------
@@ -2133,6 +2207,23 @@ Plan make_plan(int64_t pairs, int64_t n_tiles) {
   p.splits = (int)s;
   p.tps = (int)t;
   return p;
+}
+
+// Splits of the wide KIVI kernel's window-old groups: one workgroup per CU,
+// at least kMinGroupsPerSplit groups in each, where the groups a workgroup no
+// longer steps (0.16 us each while few CUs run) outweigh the second launch
+// (3 us).  Measured per step in a graph, one pass -> split (B * 8 KV heads):
+// W = 16384: B=1 85.2 -> 12.7 us (32 splits), B=2 85.4 -> 14.4 (16), B=8
+// 86.4 -> 33.3 (4), B=16 86.8 -> 60.4 (2); W = 4096: B=1 26.2 -> 10.2, B=8
+// 26.6 -> 14.8, B=16 26.9 -> 22.0; W = 2048: B=16 16.4 -> 15.4.  W = 1024
+// (28 groups) loses by it: B=8 10.8 -> 11.2.  So do KV heads enough for every
+// CU: B=33, W = 4096 51.9 -> 54.7, B=48 55.5 -> 59.1 at 2 splits.
+constexpr int64_t kMinGroupsPerSplit = 8;
+int kivi_splits(int64_t pairs, int64_t groups) {
+  const int64_t s = std::min<int64_t>(groups / kMinGroupsPerSplit, kTargetUnits / pairs);
+  if (s < 2) return 1;
+  const int64_t saved = groups - (groups + s - 1) / s;
+  return 0.16f * (float)saved > 3.0f ? (int)s : 1;
 }
 
 int64_t tiles_for(int kind, int64_t n_slots) {
@@ -2188,6 +2279,12 @@ Plan fit_plan(Plan plan, int64_t pairs, int64_t n_tiles, int G, const void* ws, 
   return Plan{(int)((n_tiles + t - 1) / t), (int)t};
 }
 
+template <int E>
+int launch_merge(const AttnCommon& P, hipStream_t stream) {
+  hipLaunchKernelGGL(merge_kernel<E>, dim3((unsigned)(P.pairs * P.G)), dim3(64 * kMergeWaves), 0, stream, P);
+  return launch_status();
+}
+
 template <class Src>
 int launch_attn(AttnCommon P, const Src& S, bool kivi, size_t ws_bytes, hipStream_t stream) {
   constexpr int E = src_elt<Src>::value;
@@ -2208,9 +2305,7 @@ int launch_attn(AttnCommon P, const Src& S, bool kivi, size_t ws_bytes, hipStrea
                      P, S);
   int rc = launch_status();
   if (rc != KVDEC_OK || plan.splits == 1) return rc;
-  const int64_t outs = P.pairs * P.G * kHeadDim;
-  hipLaunchKernelGGL(merge_kernel<E>, dim3((unsigned)((outs + 255) / 256)), dim3(256), 0, stream, P);
-  return launch_status();
+  return launch_merge<E>(P, stream);
 }
 
 // The lean kernels' launches (one workgroup per KV head).
@@ -2308,11 +2403,32 @@ int check_dense(const void* q, const void* k, const void* v, void* o, int dtype,
   return KVDEC_OK;
 }
 
+int launch_wide(AttnCommon P, KiviWideArgs A, void* ws, size_t ws_bytes, hipStream_t st) {
+  const int64_t groups = A.nwt - A.first;
+  const size_t per_split = ws_bytes_for(P.pairs, 2, P.G) / 2;
+  int64_t s = kivi_splits(P.pairs, groups);
+  if (ws == nullptr) s = 1;
+  s = std::max<int64_t>(1, std::min<int64_t>(s, (int64_t)(ws_bytes / per_split)));
+  const int64_t per = (groups + s - 1) / s;
+  s = s > 1 ? (groups + per - 1) / per : 1;
+  P.ws = static_cast<float*>(ws);
+  P.n_splits = (int)s;
+  A.ws = P.ws;
+  A.pairs = P.pairs;
+  A.n_splits = P.n_splits;
+  A.per_split = (int)per;
+  void (*kern)(KiviWideArgs) = s > 1 ? (A.lens ? kivi_wide_kernel<true, true> : kivi_wide_kernel<true, false>)
+                                     : (A.lens ? kivi_wide_kernel<false, true> : kivi_wide_kernel<false, false>);
+  hipLaunchKernelGGL(kern, dim3((unsigned)(P.pairs * s)), dim3(kWideThreads), kWideLdsBytes, st, A);
+  const int rc = launch_status();
+  return rc != KVDEC_OK || s == 1 ? rc : launch_merge<kEltF16>(P, st);
+}
+
 template <bool PACK>
 int kivi_decode_t(const void* q, const void* k_res, const void* v_res, const void* const* kivi,
                 void* o, const int32_t* lens, int64_t B, int32_t H, int32_t KVH, int64_t seq_len,
                 int32_t window, int32_t sink, int32_t residual, int32_t group, int32_t bits,
-                float sm_scale, void* stream) {
+                float sm_scale, void* ws, size_t ws_bytes, void* stream) {
   if (!q || !k_res || !v_res || !kivi || !o) return KVDEC_E_NULL;
   if (bits != 2) return KVDEC_E_BITS;
   if (group != 32) return KVDEC_E_UNSUPPORTED;
@@ -2364,7 +2480,6 @@ int kivi_decode_t(const void* q, const void* k_res, const void* v_res, const voi
   S.lens = lens;
   S.window = window;
   const hipStream_t st = static_cast<hipStream_t>(stream);
-  if (lens) return launch_attn(P, S, true, 0, st);
   // the lean kernel: at most 4 residual tiles, at most 7 window-old groups,
   // and every tensor small enough for 31-bit offsets
   const int64_t lean_bytes = P.pairs * (int64_t)res_rows * kRowBytes;
@@ -2374,8 +2489,8 @@ int kivi_decode_t(const void* q, const void* k_res, const void* v_res, const voi
   // tensors small enough for 31-bit offsets too
   const bool wide = PACK && S.nwt >= kWideMinGroups && P.G <= kPackGroup && sink <= kTile / 2 &&
                     P.pairs * (int64_t)S.nwt * 1024 < ((int64_t)1 << 31);
-  if (res_rows <= 4 * kTile && (lean || wide) && lean_bytes < ((int64_t)1 << 31)) {
-    KiviLeanArgs A;
+  if (res_rows <= 4 * kTile && (wide || (lean && !lens)) && lean_bytes < ((int64_t)1 << 31)) {
+    KiviWideArgs A{};
     A.c = lean_common(P);
     A.kres = S.kres;
     A.vres = S.vres;
@@ -2388,15 +2503,23 @@ int kivi_decode_t(const void* q, const void* k_res, const void* v_res, const voi
     A.nwt = S.nwt;
     A.sink = sink;
     SET_CLOCK(A.c);
-    if (lean && S.nwt == 4)
+    const KiviLeanArgs& L = A;
+    if (lean && S.nwt == 4) {
       hipLaunchKernelGGL(kivi_lean9_kernel<PACK>, dim3((unsigned)P.pairs), dim3(64 * kLean9Waves),
-                         Lean9Lds::kBytes + kQLdsBytes, st, A);
-    else if (lean)
-      hipLaunchKernelGGL(kivi_lean_kernel<PACK>, dim3((unsigned)P.pairs), dim3(kThreads), kLdsBytes + kQLdsBytes, st, A);
-    else if constexpr (PACK)
-      hipLaunchKernelGGL(kivi_wide_kernel<true>, dim3((unsigned)P.pairs), dim3(kWideThreads), kWideLdsBytes, st, A);
-    return launch_status();
+                         Lean9Lds::kBytes + kQLdsBytes, st, L);
+      return launch_status();
+    }
+    if (lean) {
+      hipLaunchKernelGGL(kivi_lean_kernel<PACK>, dim3((unsigned)P.pairs), dim3(kThreads), kLdsBytes + kQLdsBytes, st, L);
+      return launch_status();
+    }
+    A.lens = lens;
+    A.KVH = KVH;
+    A.window = window;
+    A.first = lens ? 0 : std::min<int32_t>((P.R.vb - sink) / kTile, A.nwt);
+    return launch_wide(P, A, ws, ws_bytes, st);
   }
+  if (lens) return launch_attn(P, S, true, 0, st);
   KiviSrc<PACK> S1{};
   S1.kres = S.kres;
   S1.vres = S.vres;
@@ -2455,7 +2578,7 @@ int kivi_decode_generic(const void* q, const void* k_res, const void* v_res, con
 int kivi_decode(const void* q, const void* k_res, const void* v_res, const void* const* kivi,
                 void* o, const int32_t* lens, int64_t B, int32_t H, int32_t KVH, int64_t seq_len,
                 int32_t window, int32_t sink, int32_t residual, int32_t group, int32_t bits,
-                float sm_scale, void* stream) {
+                float sm_scale, void* ws, size_t ws_bytes, void* stream) {
   if (bits != 2 || group != kQGroup)
     return kivi_decode_generic(q, k_res, v_res, kivi, o, lens, B, H, KVH, seq_len, window, sink, residual,
                                group, bits, sm_scale, stream);
@@ -2463,10 +2586,10 @@ int kivi_decode(const void* q, const void* k_res, const void* v_res, const void*
   if (packed_group(H, KVH, group > 0 ? (window - res_rows) / group : 0))
     return kivi_decode_t<true>(
       q, k_res, v_res, kivi, o, lens, B, H, KVH, seq_len, window, sink, residual, group, bits,
-      sm_scale, stream);
+      sm_scale, ws, ws_bytes, stream);
   return kivi_decode_t<false>(
       q, k_res, v_res, kivi, o, lens, B, H, KVH, seq_len, window, sink, residual, group, bits,
-      sm_scale, stream);
+      sm_scale, ws, ws_bytes, stream);
 }
 
 // The fused decode over a decode-time KIVI cache: one ring state for every
@@ -2739,6 +2862,7 @@ int kvdec_clock_arm(void* log, int32_t slots) {
 int kvdec_num_splits(int kind, int64_t B, int32_t KVH, int64_t n_slots) {
   if (B < 1 || KVH < 1 || n_slots < 1) return 1;
   if (kind == KVDEC_KIND_KIVI) return 1;
+  if (kind == KVDEC_KIND_KIVI_SPLIT) return kivi_splits(B * KVH, n_slots / kTile);
   return make_plan(B * KVH, tiles_for(kind, n_slots)).splits;
 }
 
@@ -2746,6 +2870,8 @@ size_t kvdec_workspace_bytes(int kind, int64_t B, int32_t H, int32_t KVH, int64_
                              int32_t D) {
   if (check_heads(B, H, KVH, D) != KVDEC_OK || n_slots < 1) return 0;
   if (kind == KVDEC_KIND_KIVI) return 0;
+  if (kind == KVDEC_KIND_KIVI_SPLIT)
+    return ws_bytes_for(B * KVH, kivi_splits(B * KVH, n_slots / kTile), H / KVH);
   const Plan p = make_plan(B * KVH, tiles_for(kind, n_slots));
   return ws_bytes_for(B * KVH, p.splits, H / KVH);
 }
@@ -2953,10 +3079,8 @@ int kvdec_sparse_decode_kivi(const void* q, const void* k_res, const void* v_res
                              int64_t seq_len, int32_t window, int32_t sink, int32_t residual,
                              int32_t group, int32_t bits, float sm_scale, void* ws,
                              size_t ws_bytes, void* stream) {
-  (void)ws;         // one pass: no workspace
-  (void)ws_bytes;
   return kivi_decode(q, k_res, v_res, kivi, o, nullptr, B, H, KVH, seq_len, window, sink, residual,
-                     group, bits, sm_scale, stream);
+                     group, bits, sm_scale, ws, ws_bytes, stream);
 }
 
 int kvdec_sparse_decode_kivi_varlen(const void* q, const void* k_res, const void* v_res,
@@ -2966,7 +3090,7 @@ int kvdec_sparse_decode_kivi_varlen(const void* q, const void* k_res, const void
                                     float sm_scale, void* stream) {
   if (!seq_lens) return KVDEC_E_NULL;
   return kivi_decode(q, k_res, v_res, kivi, o, seq_lens, B, H, KVH, 1, window, sink, residual,
-                     group, bits, sm_scale, stream);
+                     group, bits, sm_scale, nullptr, 0, stream);
 }
 
 int kvdec_sparse_decode_kivi_typed(const void* q, const void* k_res, const void* v_res,
@@ -2977,7 +3101,7 @@ int kvdec_sparse_decode_kivi_typed(const void* q, const void* k_res, const void*
   const int64_t L = seq_lens ? 1 : seq_len;
   if (q_dtype == KVDEC_F16 && res_dtype == KVDEC_F16)
     return kivi_decode(q, k_res, v_res, kivi, o, seq_lens, B, H, KVH, L, window, sink, residual, group,
-                       bits, sm_scale, stream);
+                       bits, sm_scale, nullptr, 0, stream);
   return kivi_decode_generic(q, k_res, v_res, kivi, o, seq_lens, B, H, KVH, L, window, sink, residual,
                              group, bits, sm_scale, stream, q_dtype, res_dtype);
 }

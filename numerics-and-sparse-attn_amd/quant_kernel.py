@@ -238,7 +238,7 @@ def sparse_decode_attention_quantized(
                                                    float(sm_scale), K.stream_of(q))
         K.check(rc, "sparse_decode_attention_quantized")
         return o
-    ws, nbytes = K.workspace(K.KIND_KIVI, B, H, KVH, window, D, q.device)
+    ws, nbytes = K.workspace(K.KIND_KIVI_SPLIT, B, H, KVH, win_tok, D, q.device)
     rc = K.lib.kvdec_sparse_decode_kivi(K.ptr(q), K.ptr(k_cache), K.ptr(v_cache), arr, K.ptr(o), B,
                                         H, KVH, seq_len, window, sink, R, G, bits, float(sm_scale),
                                         K.ptr(ws), nbytes, K.stream_of(q))
