@@ -282,7 +282,7 @@ __device__ __forceinline__ void publish_f(const AttnCommon& P, const WaveState& 
 // read heads only).  ADD as in publish_q.  The elements are copied to
 // scalars before their bit casts: ROCm 7.2 clang compiles
 // `__builtin_bit_cast` of a vector element (`v[i]`) as a read of element 0.
-template <bool ADD>
+template <bool ADD, int BITS = 2>
 __device__ __forceinline__ void publish_q_folded(const QState& qs, char* slot, int lane) {
   const int t = lane & 15, g = lane >> 4;
   const int hb = g < 2 ? 4 * g : 4 * (g - 2) + 1;
@@ -290,7 +290,7 @@ __device__ __forceinline__ void publish_q_folded(const QState& qs, char* slot, i
   uint32_t off[4][2];
 #pragma unroll
   for (int grp = 0; grp < 4; ++grp) {
-    const int ch = q_state_channel(grp, 0, t);
+    const int ch = q_state_channel<BITS>(grp, 0, t);
 #pragma unroll
     for (int p = 0; p < 2; ++p) {
       off[grp][p] = row_off(hb + 2 * p, ch >> 2) + 4 * (ch & 3);
@@ -327,10 +327,11 @@ __device__ __forceinline__ void publish_q_folded(const QState& qs, char* slot, i
 // no write is predicated.  ADD: the slot already holds this wave's fp16-tile
 // rows (all reads are issued before any write, so the adds wait on LDS
 // once).  PACK: publish_q_folded.
-template <bool ADD, bool PACK = false>
+template <bool ADD, bool PACK = false, int BITS = 2>
 __device__ __forceinline__ void publish_q(const QState& qs, char* slot, int lane) {
+  static_assert(PACK || BITS == 2, "other widths take the packed layout");
   if (PACK) {
-    publish_q_folded<ADD>(qs, slot, lane);
+    publish_q_folded<ADD, BITS>(qs, slot, lane);
     return;
   }
   const int t = lane & 15, g = lane >> 4;
@@ -1847,25 +1848,31 @@ __global__ __launch_bounds__(64 * kStepWaves, 1) void kivi_ring_kernel(StepLeanA
 // and the 8-wave kernel is faster (measured per step, W = 384 / 480 / 512:
 // 8.11 / 8.96 / 9.89 us there, 8.45 / 9.42 / 9.22 us here).
 constexpr int kWideMinGroups = 12;
-constexpr int kWideWaves = 16;
-constexpr int kWideThreads = 64 * kWideWaves;
-constexpr int kWideQWaves = 12;                  // waves that start on quantized items
-constexpr int kWideParts = kWideWaves + 4;       // + the residual waves' fp16 partials
-constexpr int kWideLdsCtr = 0;
-constexpr int kWideLdsM = 16;
-constexpr int kWideLdsL = kWideLdsM + kWideParts * kMaxGroup * 4;
-constexpr int kWideLdsSlots = (kWideLdsL + kWideParts * kMaxGroup * 4 + 255) & ~255;
-constexpr int kWideF16Bytes = kPackGroup * kHeadDim * 4;   // an fp16 partial of <= 8 heads
-constexpr int kWideLdsF16 = kWideLdsSlots + kWideWaves * kSlotBytes;
-constexpr int kWideLdsBytes = kWideLdsF16 + 4 * kWideF16Bytes;
-static_assert(kWideLdsBytes <= 160 * 1024, "wide kernel LDS");
+// 4-bit tiles hold 8 more VGPRs of codes in flight, which 128 VGPRs spill
+// (15 of them), so their kernel has 12 waves of 168.
+template <int BITS>
+struct Wide {
+  static constexpr int kWaves = BITS == 4 ? 12 : 16;
+  static constexpr int kThreads = 64 * kWaves;
+  static constexpr int kQWaves = kWaves - 4;           // waves that start on quantized items
+  static constexpr int kParts = kWaves + 4;            // + the residual waves' fp16 partials
+  static constexpr int kCtr = 0;
+  static constexpr int kM = 16;
+  static constexpr int kL = kM + kParts * kMaxGroup * 4;
+  static constexpr int kSlots = (kL + kParts * kMaxGroup * 4 + 255) & ~255;
+  static constexpr int kF16Bytes = kPackGroup * kHeadDim * 4;   // an fp16 partial of <= 8 heads
+  static constexpr int kF16 = kSlots + kWaves * kSlotBytes;
+  static constexpr int kBytes = kF16 + 4 * kF16Bytes;
+  static_assert(kBytes <= 160 * 1024, "wide kernel LDS");
+};
 
+template <int BITS>
 __device__ __forceinline__ void wide_publish_ml(int G, WaveState& st, char* lds, int lane, int part) {
   st.l = group_sum(st.l);
   const int n = lane & 15, g = lane >> 4;
   if (n < G && g == 0) {
-    reinterpret_cast<float*>(lds + kWideLdsM)[part * kMaxGroup + n] = st.m;
-    reinterpret_cast<float*>(lds + kWideLdsL)[part * kMaxGroup + n] = st.l;
+    reinterpret_cast<float*>(lds + Wide<BITS>::kM)[part * kMaxGroup + n] = st.m;
+    reinterpret_cast<float*>(lds + Wide<BITS>::kL)[part * kMaxGroup + n] = st.l;
   }
 }
 
@@ -1885,19 +1892,24 @@ struct KiviWideArgs : KiviLeanArgs {
   int32_t KVH, window;
 };
 
-template <bool SPLIT, bool VAR>
-__global__ __launch_bounds__(kWideThreads, 1) void kivi_wide_kernel(KiviWideArgs A) {
+template <bool SPLIT, bool VAR, int BITS = 2, int E = kEltF16>
+__global__ __launch_bounds__(Wide<BITS>::kThreads, 1) void kivi_wide_kernel(KiviWideArgs A) {
   extern __shared__ __align__(16) char lds[];
   CLOCK_STAMP(A.c, 0);
   constexpr bool PACK = true;
+  typedef Wide<BITS> Wd;
+  // 2-bit codes under an fp16 query scale Q once; the other forms scale Q and
+  // each tile's K scales (q_tile_stage_n)
+  constexpr bool kNorm = BITS != 2 || E != kEltF16;
+  typedef typename std::conditional<kNorm, QTileRawN<BITS>, QTileRaw>::type Raw;
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const uint32_t head = SPLIT ? blockIdx.x / (uint32_t)A.n_splits : blockIdx.x;
   const uint32_t split = SPLIT ? blockIdx.x - head * (uint32_t)A.n_splits : 0u;
   half8 qB[4];
   lean_prologue<KiviWideArgs, PACK>(A.c, head, lane, qB);
-  char* slot = lds + kWideLdsSlots + wave * kSlotBytes;
-  int* ctr = reinterpret_cast<int*>(lds + kWideLdsCtr);
+  char* slot = lds + Wd::kSlots + wave * kSlotBytes;
+  int* ctr = reinterpret_cast<int*>(lds + Wd::kCtr);
   const int nwt = A.nwt;
   SlotRanges R = A.c.R;
   int first = A.first;
@@ -1913,24 +1925,24 @@ __global__ __launch_bounds__(kWideThreads, 1) void kivi_wide_kernel(KiviWideArgs
   const bool tail = !SPLIT || (int)split == A.n_splits - 1;
   const int n_q = tail ? g1 + 1 : g1;
   const QTensors Tw = q_tensors(A.winq, A.win_code_bytes, A.win_meta_bytes);
-  const QTensors Ts = q_sink_tensors(A.sinkq, head, A.sink);
+  const QTensors Ts = q_sink_tensors<BITS>(A.sinkq, head, A.sink);
   // item i < g1: window-old group i; item g1: the sink group
-  auto load = [&](int i, QTileRaw& X) {
+  auto load = [&](int i, Raw& X) {
     const bool sk = i == g1;
     load_q_group(sk ? Ts : Tw, sk ? 0u : head * (uint32_t)nwt + (uint32_t)i, i < n_q, lane, X);
   };
-  if (threadIdx.x == 0) *ctr = g0 + kWideQWaves;
-  QTileRaw X;
+  if (threadIdx.x == 0) *ctr = g0 + Wd::kQWaves;
+  Raw X;
   int i = n_q;
-  if (wave < kWideQWaves) {
+  if (wave < Wd::kQWaves) {
     i = g0 + wave;
     load(i, X);
   }
   __syncthreads();
-  if (wave >= kWideQWaves) {
+  if (wave >= Wd::kQWaves) {
     // residual tile r: rows 32 r .. + 31; rows past res_rows are slots past
     // the window (masked, V read as zeros)
-    const int r = wave - kWideQWaves;
+    const int r = wave - Wd::kQWaves;
     const int slot0 = A.sink + kTile * nwt + kTile * r;
     const rsrc_t rk = make_rsrc(A.kres, A.res_bytes), rv = make_rsrc(A.vres, A.res_bytes);
     const uint32_t soff = head * (uint32_t)(A.res_rows * kRowBytes);
@@ -1941,64 +1953,84 @@ __global__ __launch_bounds__(kWideThreads, 1) void kivi_wide_kernel(KiviWideArgs
     if (has) {
       F16Raw F;
       load_f16(rk, rv, base, soff, lane, F);
-      f16_tile_step(F, slot, qB, slot0, R, A.c.scale_log2, sf, lane);
+      f16_tile_step<E>(F, slot, qB, slot0, R, A.c.scale_log2, sf, lane);
     }
-    wide_publish_ml(A.c.G, sf, lds, lane, kWideWaves + r);
-    lean_publish_f(A.c.G, sf, lds + kWideLdsF16 + r * kWideF16Bytes, lane);
+    wide_publish_ml<BITS>(A.c.G, sf, lds, lane, Wd::kWaves + r);
+    lean_publish_f(A.c.G, sf, lds + Wd::kF16 + r * Wd::kF16Bytes, lane);
     i = grab(ctr, lane);
     load(i, X);
   }
   // the quantized items' Q operand, prescaled once the wave's first group
   // load is in flight (before it, the wait for Q would hold the load back)
-  const float sl2 = q_prescale(qB, A.c.scale_log2);
+  float sl2;
+  if constexpr (kNorm)
+    sl2 = scale_pow2(A.c.scale_log2, q_normalize<E>(qB));
+  else
+    sl2 = q_prescale(qB, A.c.scale_log2);
   WaveState st;   // the quantized items' max and sum (st.O stays zero)
   wave_state_init(st);
   QState qs;
   q_state_init(qs);
+  int v_field = 0;
+  // stages X and returns its slack; `f` is the staged tile's logit factor
+  auto stage = [&](int slot0, int xlim, float& f) {
+    if constexpr (kNorm) {
+      int k;
+      q_tile_stage_n<BITS>(X, slot, lane, slot0, xlim, R, k, v_field, qs);
+      f = scale_pow2(sl2, -k);
+      return kRescaleSlack;
+    } else {
+      f = sl2;
+      return q_tile_stage(X, slot, lane);
+    }
+  };
   // window-old groups; the sink group (claimed last, at most 16 tokens: the
   // host's condition) is stepped after the loop, so that the loop holds one
   // tile body (with two, the registers of 4 waves per SIMD do not suffice)
   while (i < g1) {
-    const float slack = q_tile_stage(X, slot, lane);
+    float f;
+    const float slack = stage(A.sink + kTile * i, kTile, f);
     const int nx = grab(ctr, lane);
     load(nx, X);
-    q_tile_body<false, false, PACK>(slot, qB, A.sink + kTile * i, kTile, R, sl2, slack, st, qs, lane);
+    q_tile_body<false, false, PACK, BITS>(slot, qB, A.sink + kTile * i, kTile, R, f, slack, st, qs, lane);
     i = nx;
   }
   if (i == g1 && tail) {
-    const float slack = q_tile_stage(X, slot, lane);
-    q_tile_body<false, true, PACK>(slot, qB, 0, A.sink, R, sl2, slack, st, qs, lane);
+    float f;
+    const float slack = stage(0, A.sink, f);
+    q_tile_body<false, true, PACK, BITS>(slot, qB, 0, A.sink, R, f, slack, st, qs, lane);
   }
-  wide_publish_ml(A.c.G, st, lds, lane, wave);
-  publish_q<false, PACK>(qs, slot, lane);
+  wide_publish_ml<BITS>(A.c.G, st, lds, lane, wave);
+  if constexpr (kNorm) q_state_unshift(qs, v_field);
+  publish_q<false, PACK, BITS>(qs, slot, lane);
 
   // merge: one thread per (head, 4 channels) over the 16 quantized partials
   // (remainders already folded in) and the 4 fp16 partials
   __syncthreads();
   const int e = threadIdx.x;
   if (e >= A.c.G * 32) return;
-  const float* sh_m = reinterpret_cast<const float*>(lds + kWideLdsM);
-  const float* sh_l = reinterpret_cast<const float*>(lds + kWideLdsL);
+  const float* sh_m = reinterpret_cast<const float*>(lds + Wd::kM);
+  const float* sh_l = reinterpret_cast<const float*>(lds + Wd::kL);
   const int hn = e >> 5, ch = e & 31;
-  float mw[kWideParts];
+  float mw[Wd::kParts];
 #pragma unroll
-  for (int p = 0; p < kWideParts; ++p) mw[p] = sh_m[p * kMaxGroup + hn];
+  for (int p = 0; p < Wd::kParts; ++p) mw[p] = sh_m[p * kMaxGroup + hn];
   float M = mw[0];
 #pragma unroll
-  for (int p = 1; p < kWideParts; ++p) M = fmaxf(M, mw[p]);
+  for (int p = 1; p < Wd::kParts; ++p) M = fmaxf(M, mw[p]);
   float L = 0.f;
   float4v acc = {0.f, 0.f, 0.f, 0.f};
   // four partials at a time (their reads issued together)
 #pragma unroll
-  for (int p0 = 0; p0 < kWideParts; p0 += 4) {
+  for (int p0 = 0; p0 < Wd::kParts; p0 += 4) {
     float lw[4];
     float4v ow[4];
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
       const int p = p0 + j;
       lw[j] = sh_l[p * kMaxGroup + hn];
-      const char* part = p < kWideWaves ? lds + kWideLdsSlots + p * kSlotBytes
-                                        : lds + kWideLdsF16 + (p - kWideWaves) * kWideF16Bytes;
+      const char* part = p < Wd::kWaves ? lds + Wd::kSlots + p * kSlotBytes
+                                        : lds + Wd::kF16 + (p - Wd::kWaves) * Wd::kF16Bytes;
       ow[j] = *reinterpret_cast<const float4v*>(part + row_off(hn, ch));
     }
 #pragma unroll
@@ -2018,7 +2050,7 @@ __global__ __launch_bounds__(kWideThreads, 1) void kivi_wide_kernel(KiviWideArgs
     }
   } else {
     const float inv = L > 0.f ? 1.0f / L : 0.f;
-    store_out4(A.c.o + ((size_t)head * A.c.G + hn) * kHeadDim + 4 * ch, acc * inv);
+    store_out4<E>(A.c.o + ((size_t)head * A.c.G + hn) * kHeadDim + 4 * ch, acc * inv);
   }
   CLOCK_STAMP(A.c, 1);
 }
@@ -2403,6 +2435,7 @@ int check_dense(const void* q, const void* k, const void* v, void* o, int dtype,
   return KVDEC_OK;
 }
 
+template <int BITS, int E>
 int launch_wide(AttnCommon P, KiviWideArgs A, void* ws, size_t ws_bytes, hipStream_t st) {
   const int64_t groups = A.nwt - A.first;
   const size_t per_split = ws_bytes_for(P.pairs, 2, P.G) / 2;
@@ -2417,11 +2450,12 @@ int launch_wide(AttnCommon P, KiviWideArgs A, void* ws, size_t ws_bytes, hipStre
   A.pairs = P.pairs;
   A.n_splits = P.n_splits;
   A.per_split = (int)per;
-  void (*kern)(KiviWideArgs) = s > 1 ? (A.lens ? kivi_wide_kernel<true, true> : kivi_wide_kernel<true, false>)
-                                     : (A.lens ? kivi_wide_kernel<false, true> : kivi_wide_kernel<false, false>);
-  hipLaunchKernelGGL(kern, dim3((unsigned)(P.pairs * s)), dim3(kWideThreads), kWideLdsBytes, st, A);
+  void (*kern)(KiviWideArgs) =
+      s > 1 ? (A.lens ? kivi_wide_kernel<true, true, BITS, E> : kivi_wide_kernel<true, false, BITS, E>)
+            : (A.lens ? kivi_wide_kernel<false, true, BITS, E> : kivi_wide_kernel<false, false, BITS, E>);
+  hipLaunchKernelGGL(kern, dim3((unsigned)(P.pairs * s)), dim3(Wide<BITS>::kThreads), Wide<BITS>::kBytes, st, A);
   const int rc = launch_status();
-  return rc != KVDEC_OK || s == 1 ? rc : launch_merge<kEltF16>(P, st);
+  return rc != KVDEC_OK || s == 1 ? rc : launch_merge<E>(P, st);
 }
 
 template <bool PACK>
@@ -2517,7 +2551,7 @@ int kivi_decode_t(const void* q, const void* k_res, const void* v_res, const voi
     A.KVH = KVH;
     A.window = window;
     A.first = lens ? 0 : std::min<int32_t>((P.R.vb - sink) / kTile, A.nwt);
-    return launch_wide(P, A, ws, ws_bytes, st);
+    return launch_wide<2, kEltF16>(P, A, ws, ws_bytes, st);
   }
   if (lens) return launch_attn(P, S, true, 0, st);
   KiviSrc<PACK> S1{};
@@ -2546,15 +2580,77 @@ bool packed_group(int32_t H, int32_t KVH, int64_t window_old_groups) {
 // The element types the attention entry points take (q, o and row caches).
 bool valid_attn_dtype(int dtype) { return dtype == KVDEC_F16 || dtype == KVDEC_F32 || dtype == KVDEC_BF16; }
 
+// 2- and 4-bit codes in groups of 32 under fp16 or bf16 queries and residual
+// rows (one type for both) take the wide kernel, whatever the window, for query
+// groups of at most kPackGroup heads, a residual of at most 128 rows and a sink
+// of at most 16 tokens, when every tensor allows its 16-byte accesses and
+// 31-bit offsets.  Measured per step in a graph against the generic kernel
+// (bound by its scalar dequantization and fp32 dot products, 11 us for every 64
+// slots): B=8, W=1024, 4-bit bf16 205 -> 13.3 us, 2-bit bf16 12.3; W=128
+// 31 -> 7.6; B=32, W=2944 31.9 (2-bit fp16: 29.1).  At 8 bits an inf zero
+// point, which those caches can hold, would turn an infinite key into NaN, so
+// they stay there.
+template <int BITS, int E>
+int kivi_decode_wide(const void* q, const void* k_res, const void* v_res, const void* const* kivi, void* o,
+                     const int32_t* lens, int64_t B, int32_t H, int32_t KVH, int64_t seq_len, int32_t window,
+                     int32_t sink, int32_t res_rows, int32_t win_tok, float sm_scale, void* ws, size_t ws_bytes,
+                     hipStream_t stream) {
+  AttnCommon P{};
+  P.q = static_cast<const _Float16*>(q);
+  P.o = static_cast<_Float16*>(o);
+  P.pairs = B * KVH;
+  P.H = H;
+  P.KVH = KVH;
+  P.G = H / KVH;
+  P.scale_log2 = (float)((double)sm_scale * 1.4426950408889634);
+  P.R = sparse_ranges(seq_len, window, sink, KVDEC_LAYOUT_LINEAR);
+  auto region = [&](int i) {
+    return QRegion{static_cast<const uint8_t*>(kivi[i]),      static_cast<const _Float16*>(kivi[i + 1]),
+                   static_cast<const _Float16*>(kivi[i + 2]), static_cast<const uint8_t*>(kivi[i + 3]),
+                   static_cast<const _Float16*>(kivi[i + 4]), static_cast<const _Float16*>(kivi[i + 5])};
+  };
+  KiviWideArgs A{};
+  A.c = lean_common(P);
+  A.kres = static_cast<const _Float16*>(k_res);
+  A.vres = static_cast<const _Float16*>(v_res);
+  A.sinkq = region(0);
+  A.winq = win_tok > 0 ? region(6) : A.sinkq;   // (no window-old groups: never read)
+  A.nwt = win_tok / kTile;
+  A.sink = sink;
+  A.res_rows = res_rows;
+  A.res_bytes = (uint32_t)(P.pairs * res_rows * kRowBytes);
+  A.win_code_bytes = (uint32_t)(P.pairs * A.nwt * 512 * BITS);
+  A.win_meta_bytes = (uint32_t)(P.pairs * A.nwt * 256);
+  A.lens = lens;
+  A.KVH = KVH;
+  A.window = window;
+  A.first = lens ? 0 : std::min<int32_t>((P.R.vb - sink) / kTile, A.nwt);
+  SET_CLOCK(A.c);
+  return launch_wide<BITS, E>(P, A, ws, ws_bytes, stream);
+}
+
+bool wide_form(const void* q, const void* k_res, const void* v_res, const void* const* kivi, const void* o,
+               int q_dtype, int res_dtype, int64_t pairs, int32_t G, int32_t sink, int32_t res_rows,
+               int32_t win_tok, int32_t group, int32_t bits) {
+  if ((bits != 2 && bits != 4) || group != kTile || G > kPackGroup) return false;
+  if (q_dtype != res_dtype || (q_dtype != KVDEC_F16 && q_dtype != KVDEC_BF16)) return false;
+  if (sink > kTile / 2 || res_rows > 4 * kTile) return false;
+  uintptr_t at = (uintptr_t)q | (uintptr_t)k_res | (uintptr_t)v_res | (uintptr_t)o;
+  for (int i = 0; i < (win_tok > 0 ? 12 : 6); ++i) at |= (uintptr_t)kivi[i];
+  const int64_t most = (int64_t)1 << 31;
+  return (at & 15u) == 0 && pairs * res_rows * kRowBytes < most && pairs * (win_tok / kTile) * 512 * bits < most;
+}
+
 // Code widths and group sizes other than 2 / 32, and queries or residual
-// rows other than fp16: the generic kernel, with the reference's layout
+// rows other than fp16: the wide kernel where it takes them (wide_form), else
+// the generic kernel, with the reference's layout
 // assumptions (whole bytes per group, channel groups that divide the head
 // dim).
 int kivi_decode_generic(const void* q, const void* k_res, const void* v_res, const void* const* kivi,
                         void* o, const int32_t* lens, int64_t B, int32_t H, int32_t KVH,
                         int64_t seq_len, int32_t window, int32_t sink, int32_t residual, int32_t group,
-                        int32_t bits, float sm_scale, void* stream, int q_dtype = KVDEC_F16,
-                        int res_dtype = KVDEC_F16) {
+                        int32_t bits, float sm_scale, void* ws, size_t ws_bytes, void* stream,
+                        int q_dtype = KVDEC_F16, int res_dtype = KVDEC_F16) {
   if (!q || !k_res || !v_res || !kivi || !o) return KVDEC_E_NULL;
   if (!valid_attn_dtype(q_dtype) || !valid_attn_dtype(res_dtype)) return KVDEC_E_DTYPE;
   if (bits < 1 || bits > 8) return KVDEC_E_BITS;
@@ -2571,8 +2667,17 @@ int kivi_decode_generic(const void* q, const void* k_res, const void* v_res, con
   if (win_tok > 0)
     for (int i = 6; i < 12; ++i)
       if (!kivi[i]) return KVDEC_E_NULL;
+  const hipStream_t st = static_cast<hipStream_t>(stream);
+  if (wide_form(q, k_res, v_res, kivi, o, q_dtype, res_dtype, B * KVH, H / KVH, sink, res_rows, win_tok, group, bits)) {
+    auto run = [&](auto decode) {
+      return decode(q, k_res, v_res, kivi, o, lens, B, H, KVH, seq_len, window, sink, res_rows, win_tok, sm_scale,
+                    ws, ws_bytes, st);
+    };
+    if (q_dtype == KVDEC_BF16) return bits == 2 ? run(kivi_decode_wide<2, kEltBf16>) : run(kivi_decode_wide<4, kEltBf16>);
+    if (bits == 4) return run(kivi_decode_wide<4, kEltF16>);
+  }
   return generic_kivi_decode(q, k_res, v_res, kivi, o, q_dtype, res_dtype, lens, B, H, KVH, seq_len, window,
-                             sink, res_rows, win_tok, group, bits, sm_scale, static_cast<hipStream_t>(stream));
+                             sink, res_rows, win_tok, group, bits, sm_scale, ws, ws_bytes, st);
 }
 
 int kivi_decode(const void* q, const void* k_res, const void* v_res, const void* const* kivi,
@@ -2581,7 +2686,7 @@ int kivi_decode(const void* q, const void* k_res, const void* v_res, const void*
                 float sm_scale, void* ws, size_t ws_bytes, void* stream) {
   if (bits != 2 || group != kQGroup)
     return kivi_decode_generic(q, k_res, v_res, kivi, o, lens, B, H, KVH, seq_len, window, sink, residual,
-                               group, bits, sm_scale, stream);
+                               group, bits, sm_scale, ws, ws_bytes, stream);
   const int64_t res_rows = window < residual ? window : residual;
   if (packed_group(H, KVH, group > 0 ? (window - res_rows) / group : 0))
     return kivi_decode_t<true>(
@@ -3103,7 +3208,7 @@ int kvdec_sparse_decode_kivi_typed(const void* q, const void* k_res, const void*
     return kivi_decode(q, k_res, v_res, kivi, o, seq_lens, B, H, KVH, L, window, sink, residual, group,
                        bits, sm_scale, nullptr, 0, stream);
   return kivi_decode_generic(q, k_res, v_res, kivi, o, seq_lens, B, H, KVH, L, window, sink, residual,
-                             group, bits, sm_scale, stream, q_dtype, res_dtype);
+                             group, bits, sm_scale, nullptr, 0, stream, q_dtype, res_dtype);
 }
 
 int kvdec_kivi_stream_decode(const void* q, const void* k_ring, const void* v_ring,

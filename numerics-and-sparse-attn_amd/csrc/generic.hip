@@ -373,11 +373,11 @@ template <int QT, int RT>
 int kivi_decode_t2(const void* q, const void* k_res, const void* v_res, const void* const* kivi, void* o,
                    const int32_t* lens, int64_t B, int32_t H, int32_t KVH, int64_t seq_len, int32_t window,
                    int32_t sink, int32_t res_rows, int32_t win_tok, int32_t group, int32_t bits,
-                   float sm_scale, hipStream_t stream) {
+                   float sm_scale, void* ws, size_t ws_bytes, hipStream_t stream) {
   GArgs<QT> A{};
   A.q = static_cast<const typename GElt<QT>::T*>(q);
   A.o = static_cast<typename GElt<QT>::T*>(o);
-  A.ws = nullptr;
+  A.ws = static_cast<float*>(ws);
   A.pairs = B * KVH;
   A.H = H;
   A.KVH = KVH;
@@ -386,8 +386,7 @@ int kivi_decode_t2(const void* q, const void* k_res, const void* v_res, const vo
   A.scale_log2 = (float)((double)sm_scale * 1.4426950408889634);
   A.range = GRange{sparse_ranges(seq_len, window, sink, KVDEC_LAYOUT_LINEAR), lens, true, window, sink,
                    KVDEC_LAYOUT_LINEAR, A.n_slots};
-  A.n_splits = 1;
-  A.per_split = ((A.n_slots + kGC - 1) / kGC) * kGC;
+  plan_splits(A.pairs, A.G, A.n_slots, ws, ws_bytes, A.n_splits, A.per_split);
   GKiviSrc<RT> S{};
   S.kres = static_cast<const typename GElt<RT>::T*>(k_res);
   S.vres = static_cast<const typename GElt<RT>::T*>(v_res);
@@ -414,33 +413,33 @@ template <int QT>
 int kivi_decode_q(int res_dtype, const void* q, const void* k_res, const void* v_res,
                   const void* const* kivi, void* o, const int32_t* lens, int64_t B, int32_t H, int32_t KVH,
                   int64_t seq_len, int32_t window, int32_t sink, int32_t res_rows, int32_t win_tok,
-                  int32_t group, int32_t bits, float sm_scale, hipStream_t stream) {
+                  int32_t group, int32_t bits, float sm_scale, void* ws, size_t ws_bytes, hipStream_t stream) {
   if (res_dtype == KVDEC_F16)
     return kivi_decode_t2<QT, KVDEC_F16>(q, k_res, v_res, kivi, o, lens, B, H, KVH, seq_len, window, sink,
-                                         res_rows, win_tok, group, bits, sm_scale, stream);
+                                         res_rows, win_tok, group, bits, sm_scale, ws, ws_bytes, stream);
   if (res_dtype == KVDEC_BF16)
     return kivi_decode_t2<QT, KVDEC_BF16>(q, k_res, v_res, kivi, o, lens, B, H, KVH, seq_len, window, sink,
-                                          res_rows, win_tok, group, bits, sm_scale, stream);
+                                          res_rows, win_tok, group, bits, sm_scale, ws, ws_bytes, stream);
   if (res_dtype == KVDEC_F32)
     return kivi_decode_t2<QT, KVDEC_F32>(q, k_res, v_res, kivi, o, lens, B, H, KVH, seq_len, window, sink,
-                                         res_rows, win_tok, group, bits, sm_scale, stream);
+                                         res_rows, win_tok, group, bits, sm_scale, ws, ws_bytes, stream);
   return KVDEC_E_DTYPE;
 }
 
 int generic_kivi_decode(const void* q, const void* k_res, const void* v_res, const void* const* kivi,
                         void* o, int q_dtype, int res_dtype, const int32_t* lens, int64_t B, int32_t H,
                         int32_t KVH, int64_t seq_len, int32_t window, int32_t sink, int32_t res_rows,
-                        int32_t win_tok, int32_t group, int32_t bits, float sm_scale,
-                        hipStream_t stream) {
+                        int32_t win_tok, int32_t group, int32_t bits, float sm_scale, void* ws,
+                        size_t ws_bytes, hipStream_t stream) {
   if (q_dtype == KVDEC_F16)
     return kivi_decode_q<KVDEC_F16>(res_dtype, q, k_res, v_res, kivi, o, lens, B, H, KVH, seq_len, window,
-                                    sink, res_rows, win_tok, group, bits, sm_scale, stream);
+                                    sink, res_rows, win_tok, group, bits, sm_scale, ws, ws_bytes, stream);
   if (q_dtype == KVDEC_BF16)
     return kivi_decode_q<KVDEC_BF16>(res_dtype, q, k_res, v_res, kivi, o, lens, B, H, KVH, seq_len, window,
-                                     sink, res_rows, win_tok, group, bits, sm_scale, stream);
+                                     sink, res_rows, win_tok, group, bits, sm_scale, ws, ws_bytes, stream);
   if (q_dtype == KVDEC_F32)
     return kivi_decode_q<KVDEC_F32>(res_dtype, q, k_res, v_res, kivi, o, lens, B, H, KVH, seq_len, window,
-                                    sink, res_rows, win_tok, group, bits, sm_scale, stream);
+                                    sink, res_rows, win_tok, group, bits, sm_scale, ws, ws_bytes, stream);
   return KVDEC_E_DTYPE;
 }
 

@@ -575,6 +575,18 @@ struct QTileRaw {
   uint32_t vs, vz;     // V scale / zero of token L/2, groups 2(L%2), 2(L%2)+1
 };
 
+// Codes of 2 or 4 bits, 8 / BITS in a byte, LSB first.  A 32-token group is
+// kQPieces<BITS> pieces of 1 KB for K (byte rows of 8 / BITS tokens x 128
+// channels) and as many for V (token rows of 16 BITS bytes), with the same
+// scales and zeros.  QTileRaw is the 2-bit tile.
+template <int BITS>
+constexpr int kQPieces = BITS / 2;
+template <int BITS>
+struct QTileRawN {
+  u32x4 kc[kQPieces<BITS>], vc[kQPieces<BITS>];   // bytes [1024 i + 16L, + 16)
+  uint32_t ks, kz, vs, vz;                        // as QTileRaw
+};
+
 // Resources over the six whole tensors of a KIVI region (all KV heads):
 // every 32-token group is 1024 bytes of K codes and of V codes and 256 bytes
 // of each scale / zero piece, so group n starts at n * 1024 and n * 256.
@@ -600,6 +612,22 @@ __device__ __forceinline__ void load_q_group(const QTensors& T, uint32_t n, bool
   X.vz = bload4(T.vz, l4, om);
 }
 
+template <int BITS>
+__device__ __forceinline__ void load_q_group(const QTensors& T, uint32_t n, bool valid, int lane,
+                                             QTileRawN<BITS>& X) {
+  constexpr uint32_t kCode = 1024u * kQPieces<BITS>;
+  const uint32_t oc = n * kCode, om = n * 256u;
+  const uint32_t l16 = valid ? 16u * lane : kOOB, l4 = valid ? 4u * lane : kOOB;
+#pragma unroll
+  for (int i = 0; i < kQPieces<BITS>; ++i) X.kc[i] = bload16(T.kc, l16 + 1024u * i, oc);
+#pragma unroll
+  for (int i = 0; i < kQPieces<BITS>; ++i) X.vc[i] = bload16(T.vc, l16 + 1024u * i, oc);
+  X.ks = bload4(T.ks, l4, om);
+  X.kz = bload4(T.kz, l4, om);
+  X.vs = bload4(T.vs, l4, om);
+  X.vz = bload4(T.vz, l4, om);
+}
+
 // Bytes of a group's pieces that hold its first `rows` tokens: K code byte
 // rows of 4 tokens x 128 channels, V code rows of 32 bytes, V scale / zero
 // rows of 4 fp16 (the K scales and zeros are per channel: all 256 bytes).
@@ -612,9 +640,11 @@ __device__ __forceinline__ uint32_t q_vmeta_bytes(int rows) { return 8u * (uint3
 
 // Resources over the sink group of KV head `head` alone (group `head` of
 // the sink tensors), sized to its `sink` real tokens; load it as group 0.
+template <int BITS = 2>
 __device__ __forceinline__ QTensors q_sink_tensors(const QRegion& Q, uint32_t head, int sink) {
-  return QTensors{make_rsrc(Q.kp + (size_t)head * 1024, q_kcode_bytes(sink)),
-                  make_rsrc(Q.vp + (size_t)head * 1024, q_vcode_bytes(sink)),
+  constexpr int kPf = 8 / BITS, kCode = 1024 * kQPieces<BITS>;
+  return QTensors{make_rsrc(Q.kp + (size_t)head * kCode, 128u * (uint32_t)((sink + kPf - 1) / kPf)),
+                  make_rsrc(Q.vp + (size_t)head * kCode, q_vcode_bytes(sink) * kQPieces<BITS>),
                   make_rsrc(Q.ks + (size_t)head * kHeadDim, 256u),
                   make_rsrc(Q.kz + (size_t)head * kHeadDim, 256u),
                   make_rsrc(Q.vs + (size_t)head * 128, q_vmeta_bytes(sink)),
@@ -657,7 +687,9 @@ __device__ __forceinline__ void q_state_init(QState& qs) {
 
 // Output channel of accumulator column t of QState::O[2 grp + m]: the two
 // accumulators of a group hold adjacent channels.
+template <int BITS = 2>
 __device__ __forceinline__ int q_state_channel(int grp, int m, int t) {
+  if constexpr (BITS == 4) return 32 * grp + 2 * t + m;
   return 32 * grp + 4 * (t & 7) + 2 * (t >> 3) + m;
 }
 
@@ -690,6 +722,23 @@ constexpr int kQsBytes = 4608;
 static_assert(kQsBytes <= kSlotBytes, "a staged KIVI tile fits a wave slot");
 constexpr uint32_t kNegPk = 0x80008000u;   // sign bits of an fp16 pair
 constexpr uint32_t kOnePk = 0x3C003C00u;   // fp16 pair (1, 1)
+
+// Where the pieces of a staged tile sit in a wave slot.  4 bits: 16 K byte
+// rows 160 bytes apart (QK reads 8 of them at once), 32 V token rows 80 bytes
+// apart (the transposed read takes 16 bytes of each: no two rows of 16 share
+// a bank), the scale and zero rows as for 2 bits.
+template <int BITS>
+struct QSlot {
+  static constexpr int kK = kQsK, kKS = kQsKS, kKZ = kQsKZ, kV = kQsV, kVS = kQsVS, kVZ = kQsVZ;
+  static constexpr int kVRow = 32, kBytes = kQsBytes;
+};
+template <>
+struct QSlot<4> {
+  static constexpr int kVRow = 80;
+  static constexpr int kK = 0, kKS = 16 * kQsKRow, kKZ = kKS + 256, kV = kKZ + 256, kVS = kV + 32 * kVRow,
+                       kVZ = kVS + 256, kBytes = kVZ + 256;
+};
+static_assert(QSlot<4>::kBytes <= kSlotBytes, "a staged 4-bit tile fits a wave slot");
 
 __device__ __forceinline__ void stage_q_raw(const QTileRaw& X, char* slot, int lane) {
   *reinterpret_cast<u32x4*>(slot + kQsK + kQsKRow * (lane >> 3) + 16 * (lane & 7)) = X.kc;
@@ -742,7 +791,7 @@ constexpr float kCodeScale = 512.0f;   // code * 2^-9 * 2^9 = code
 // e4m3 byte, as code * 2^-7 (code 1 the subnormal 2^-7, codes 2 and 3 the
 // least normal binade's 2^-6 and 1.5 * 2^-6): such fields need no shift.
 constexpr float kCodeScale2 = 128.0f;
-constexpr uint32_t kField0 = 0x03030303u, kField1 = 0x0C0C0C0Cu;
+constexpr uint32_t kField0 = 0x03030303u, kField1 = 0x0C0C0C0Cu, kNibble = 0x0F0F0F0Fu;
 
 // |x| <= 2^(E - 15) (1 + m / 1024) for the fp16 bits x of exponent E and
 // mantissa m: the least el with |x| <= 2^el (for normal x).
@@ -847,11 +896,12 @@ constexpr float kSlackVScale = 128.0f;
 // negated as bits with the mask (one v_bitop3 per dword), not as fp16: the
 // compiler turns some fp16 negations of packed operands into three-step
 // integer sequences.
-template <bool MIXED, bool HALF, bool PACK>
+template <bool MIXED, bool HALF, bool PACK, int BITS = 2>
 __device__ __forceinline__ void q_tile_body(const char* slot, const half8 (&qB)[4], int slot0,
                                             int xlim, const SlotRanges& R, float scale_log2,
                                             float slack, WaveState& st, QState& qs, int lane,
                                             uint32_t kmul = kOnePk) {
+  typedef QSlot<BITS> Lay;
   const int t = lane & 15, g = lane >> 4;
   const uint32_t pm = PACK ? pack_lanes(lane) : 0u;
   // scale and negated zero of the lane's K channels 32c + 8g .. +7; kmul
@@ -859,9 +909,9 @@ __device__ __forceinline__ void q_tile_body(const char* slot, const half8 (&qB)[
   half8 ks[4], nz[4];
 #pragma unroll
   for (int c = 0; c < 4; ++c) {
-    ks[c] = *reinterpret_cast<const half8*>(slot + kQsKS + 2 * (32 * c + 8 * g));
+    ks[c] = *reinterpret_cast<const half8*>(slot + Lay::kKS + 2 * (32 * c + 8 * g));
     if (kmul != kOnePk) ks[c] = ks[c] * as_h8(u32x4{kmul, kmul, kmul, kmul});
-    nz[c] = *reinterpret_cast<const half8*>(slot + kQsKZ + 2 * (32 * c + 8 * g));
+    nz[c] = *reinterpret_cast<const half8*>(slot + Lay::kKZ + 2 * (32 * c + 8 * g));
   }
 
   // S[token][head] on MFMA: lane (t, g) feeds token 16 blk + t, channels
@@ -869,9 +919,15 @@ __device__ __forceinline__ void q_tile_body(const char* slot, const half8 (&qB)[
   // Fields 2 and 3 come from the rows shifted by 4 bits, so the lane's
   // field sits at bits 0..1 (t even) or 2..3 (t odd) of each byte and is
   // masked in place.
-  const uint32_t kmask = (t & 1) ? kField1 : kField0;
-  const float kcs = (t & 1) ? kCodeScale2 : kCodeScale;
-  const char* krow = slot + ((t & 2) ? kQsK4 : kQsK) + (t >> 2) * kQsKRow + 8 * g;
+  // 4 bits: byte row (16 blk + t) / 2, the nibble t % 2 shifted down (a byte
+  // 0..15 read as e4m3 is the subnormal or least binade's code * 2^-9, like a
+  // 2-bit code).
+  const uint32_t kmask = BITS == 4 ? kNibble : (t & 1) ? kField1 : kField0;
+  const float kcs = BITS == 2 && (t & 1) ? kCodeScale2 : kCodeScale;
+  const uint32_t ksh = 4u * (uint32_t)(t & 1);
+  constexpr int kBlkRows = 2 * BITS;   // K byte rows of 16 tokens
+  const char* krow = BITS == 4 ? slot + Lay::kK + (t >> 1) * kQsKRow + 8 * g
+                               : slot + ((t & 2) ? kQsK4 : kQsK) + (t >> 2) * kQsKRow + 8 * g;
   float4v s0 = {0.f, 0.f, 0.f, 0.f}, s1 = {0.f, 0.f, 0.f, 0.f};
   float4v sz = {0.f, 0.f, 0.f, 0.f};   // the zero term of every token row
 #pragma unroll
@@ -885,7 +941,8 @@ __device__ __forceinline__ void q_tile_body(const char* slot, const half8 (&qB)[
     if (!PACK) sz = mfma16x16x32(as_u4(nz[c]), ql, sz);
 #pragma unroll
     for (int blk = 0; blk < (HALF ? 1 : 2); ++blk) {
-      const u32x2 w = *reinterpret_cast<const u32x2*>(krow + 4 * blk * kQsKRow + 32 * c);
+      u32x2 w = *reinterpret_cast<const u32x2*>(krow + kBlkRows * blk * kQsKRow + 32 * c);
+      if constexpr (BITS == 4) w = u32x2{w[0] >> ksh, w[1] >> ksh};
       const u32x2 d0 = codes_f16(w[0] & kmask, kcs), d1 = codes_f16(w[1] & kmask, kcs);
       const u32x4 d = {d0[0], d0[1], d1[0], d1[1]};
       float4v& sb = blk == 0 ? s0 : s1;
@@ -933,10 +990,20 @@ __device__ __forceinline__ void q_tile_body(const char* slot, const half8 (&qB)[
   u32x4 nBm = {0u, 0u, 0u, 0u}, prm = {0u, 0u, 0u, 0u};
   if (PACK) {
     const u32x4 pBu = as_u4(pB);
-    const u32x4 pr = {fma_mix_pk_f16(pf[0], pf[1], kOnePk, pBu[0]), fma_mix_pk_f16(pf[2], pf[3], kOnePk, pBu[1]),
-                      fma_mix_pk_f16(pf[4], pf[5], kOnePk, pBu[2]), fma_mix_pk_f16(pf[6], pf[7], kOnePk, pBu[3])};
-    nBm = (pBu ^ kNegPk) & pm;
-    prm = pr & pm;
+    // (4 bits: the compiler's own conversions, which it schedules around the
+    // matrix instructions)
+    if constexpr (BITS != 2) {
+      half8 d;
+#pragma unroll
+      for (int j = 0; j < 8; ++j) d[j] = (_Float16)(pf[j] - (float)pB[j]);
+      nBm = (pBu ^ kNegPk) & pm;
+      prm = as_u4(d) & pm;
+    } else {
+      const u32x4 pr = {fma_mix_pk_f16(pf[0], pf[1], kOnePk, pBu[0]), fma_mix_pk_f16(pf[2], pf[3], kOnePk, pBu[1]),
+                        fma_mix_pk_f16(pf[4], pf[5], kOnePk, pBu[2]), fma_mix_pk_f16(pf[6], pf[7], kOnePk, pBu[3])};
+      nBm = (pBu ^ kNegPk) & pm;
+      prm = pr & pm;
+    }
   }
 
   // PV, one V group (32 channels, code byte columns 8 grp .. 8 grp + 7) at
@@ -948,15 +1015,17 @@ __device__ __forceinline__ void q_tile_body(const char* slot, const half8 (&qB)[
   // head pq and the fp16 remainder pl (as for fp16 tiles);
   // tau(g, 0..3) = 4g..4g+3 and tau(g, 4..7) = 16 + 4g .. +3 sit
   // contiguously in the transposed scale and zero rows.
-  const char* vrow = slot + kQsV + 32 * tau(g, t >> 1);
-  const uint32_t vsh = 4u * (uint32_t)(t >> 3);
+  // 4 bits: byte column 16 grp + t (lane t supplies half t & 1 of the row's 16
+  // bytes), whose nibble m is channel 32 grp + 2 t + m.
+  const char* vrow = slot + Lay::kV + Lay::kVRow * tau(g, t >> 1) + (BITS == 4 ? 8 * (t & 1) : 0);
+  const uint32_t vsh = BITS == 4 ? 0u : 4u * (uint32_t)(t >> 3);
 #pragma unroll
   for (int grp = 0; grp < 4; ++grp) {
-    const u32x2 s_lo = *reinterpret_cast<const u32x2*>(slot + kQsVS + grp * 64 + 8 * g);
-    const u32x2 s_hi = *reinterpret_cast<const u32x2*>(slot + kQsVS + grp * 64 + 32 + 8 * g);
-    const u32x2 z_lo = *reinterpret_cast<const u32x2*>(slot + kQsVZ + grp * 64 + 8 * g);
-    const u32x2 z_hi = *reinterpret_cast<const u32x2*>(slot + kQsVZ + grp * 64 + 32 + 8 * g);
-    const u32x2 vb = lds_read_tr8(vrow + 8 * grp);
+    const u32x2 s_lo = *reinterpret_cast<const u32x2*>(slot + Lay::kVS + grp * 64 + 8 * g);
+    const u32x2 s_hi = *reinterpret_cast<const u32x2*>(slot + Lay::kVS + grp * 64 + 32 + 8 * g);
+    const u32x2 z_lo = *reinterpret_cast<const u32x2*>(slot + Lay::kVZ + grp * 64 + 8 * g);
+    const u32x2 z_hi = *reinterpret_cast<const u32x2*>(slot + Lay::kVZ + grp * 64 + 32 + 8 * g);
+    const u32x2 vb = lds_read_tr8(vrow + 4 * BITS * grp);
     const u32x4 vsc = {s_lo[0], s_lo[1], s_hi[0], s_hi[1]};
     u32x4 pq, pl;
     if (PACK) {
@@ -977,9 +1046,10 @@ __device__ __forceinline__ void q_tile_body(const char* slot, const half8 (&qB)[
     const uint64_t vx = ((uint64_t)vb[1] << 32 | vb[0]) >> vsh;
 #pragma unroll
     for (int m = 0; m < 2; ++m) {
-      const uint32_t msk = m ? kField1 : kField0;
-      const float csc = m ? kCodeScale2 : kCodeScale;
-      const u32x2 c = {(uint32_t)vx & msk, HALF ? 0u : (uint32_t)(vx >> 32) & msk};
+      const uint32_t msk = BITS == 4 ? kNibble : m ? kField1 : kField0;
+      const float csc = BITS == 2 && m ? kCodeScale2 : kCodeScale;
+      const uint32_t sh = BITS == 4 ? 4u * m : 0u;
+      const u32x2 c = {((uint32_t)vx >> sh) & msk, HALF ? 0u : ((uint32_t)(vx >> 32) >> sh) & msk};
       const u32x2 b0 = codes_f16(c[0], csc);
       const u32x2 b1 = HALF ? u32x2{0u, 0u} : codes_f16(c[1], csc);
       const half8 b = as_h8(u32x4{b0[0], b0[1], b1[0], b1[1]});
@@ -999,6 +1069,113 @@ __device__ __forceinline__ float q_tile_stage(const QTileRaw& raw, char* slot, i
   // every lane holds two of the tile's 128 V scales
   const half2v vs = __builtin_bit_cast(half2v, raw.vs);
   return __ballot(!(fmaxf((float)vs[0], (float)vs[1]) <= kSlackVScale)) ? 0.0f : kRescaleSlack;
+}
+
+// The staging of a tile whose Q operand is scaled to less than 1 in magnitude
+// (q_normalize), with powers of two taken out of its scales: K scales come to
+// [2^13, 2^14) at their largest (k_exp: the tile's logits are 2^k_exp too
+// large), V scales to at most 2^7 over all of the wave's tiles so far (v_field:
+// the largest exponent field seen; a tile with a larger one rescales the
+// accumulators), so that neither product's exact remainder falls into fp16's
+// subnormal range, for wide codes and small scales alike, and P' < 2^15 with
+// the softmax's slack.  (The 2-bit fp16 path scales Q alone: its remainders
+// below 2^-24 cost less than its codes' 0..3 carry into a result of order 1.)
+// Tokens of a tile that is not fully valid lose their V scale and zero: a slot
+// never written may hold any bits.
+// The largest exponent field (0..31) of fp16 magnitudes over the wave.
+__device__ __forceinline__ int max_field(uint32_t h2) {
+  const int el = (int)(max(h2 & 0x7FFFu, (h2 >> 16) & 0x7FFFu) >> 10);
+  int e = 0;
+#pragma unroll
+  for (int b = 16; b >= 1; b >>= 1)
+    if (__ballot(el >= e + b)) e += b;
+  return e;
+}
+// The power of two that V scales are multiplied by under v_field.
+__device__ __forceinline__ int v_shift(int v_field) { return 21 - v_field; }
+__device__ __forceinline__ uint32_t scale_pk(uint32_t h2, int k) {
+  const half2v h = __builtin_bit_cast(half2v, h2);
+  const half2v r = {(_Float16)__builtin_ldexpf((float)h[0], k), (_Float16)__builtin_ldexpf((float)h[1], k)};
+  return __builtin_bit_cast(uint32_t, r);
+}
+template <int BITS>
+__device__ __forceinline__ void q_tile_stage_n(const QTileRawN<BITS>& X, char* slot, int lane, int slot0, int xlim,
+                                               const SlotRanges& R, int& k_exp, int& v_field, QState& qs) {
+  typedef QSlot<BITS> Lay;
+  k_exp = 28 - max_field(X.ks);
+#pragma unroll
+  for (int i = 0; i < kQPieces<BITS>; ++i) {
+    const int krow = 8 * i + (lane >> 3);
+    *reinterpret_cast<u32x4*>(slot + Lay::kK + kQsKRow * krow + 16 * (lane & 7)) = X.kc[i];
+    if constexpr (BITS == 2)
+      *reinterpret_cast<u32x4*>(slot + kQsK4 + kQsKRow * krow + 16 * (lane & 7)) =
+          u32x4{X.kc[i][0] >> 4, X.kc[i][1] >> 4, X.kc[i][2] >> 4, X.kc[i][3] >> 4};
+    // V piece i: tokens of 16 BITS bytes, BITS lanes each
+    const int tok = (64 / BITS) * i + lane / BITS;
+    *reinterpret_cast<u32x4*>(slot + Lay::kV + Lay::kVRow * tok + 16 * (lane % BITS)) = X.vc[i];
+  }
+  *reinterpret_cast<uint32_t*>(slot + Lay::kKS + 4 * lane) = scale_pk(X.ks, k_exp);
+  *reinterpret_cast<uint32_t*>(slot + Lay::kKZ + 4 * lane) = X.kz ^ kNegPk;
+  const int tok = lane >> 1, g0 = 2 * (lane & 1);
+  uint32_t vs = X.vs, nvz = X.vz ^ kNegPk;
+  if (!(xlim == kTile && tile_fully_valid(R, slot0)) && !(tok < xlim && slot_valid(R, slot0 + tok))) vs = nvz = 0u;
+  const int vf = max_field(vs);
+  if (vf > v_field) {   // (wave-uniform)
+    const float down = __builtin_ldexpf(1.0f, v_field - vf);
+#pragma unroll
+    for (int b = 0; b < 8; ++b) qs.O[b] = qs.O[b] * down;
+    v_field = vf;
+  }
+  vs = scale_pk(vs, v_shift(v_field));
+  *reinterpret_cast<uint16_t*>(slot + Lay::kVS + g0 * 64 + 2 * tok) = (uint16_t)vs;
+  *reinterpret_cast<uint16_t*>(slot + Lay::kVS + (g0 + 1) * 64 + 2 * tok) = (uint16_t)(vs >> 16);
+  *reinterpret_cast<uint16_t*>(slot + Lay::kVZ + g0 * 64 + 2 * tok) = (uint16_t)nvz;
+  *reinterpret_cast<uint16_t*>(slot + Lay::kVZ + (g0 + 1) * 64 + 2 * tok) = (uint16_t)(nvz >> 16);
+}
+// The accumulators without the V scales' power of two.
+__device__ __forceinline__ void q_state_unshift(QState& qs, int v_field) {
+  const float down = __builtin_ldexpf(1.0f, -v_shift(v_field));
+#pragma unroll
+  for (int b = 0; b < 8; ++b) qs.O[b] = qs.O[b] * down;
+}
+
+// The Q operand of element type E as fp16, scaled by the power of two 2^-e
+// that brings the KV head's largest |q| below 1; returns e.  bf16's 8 bits
+// fit fp16's 11: exact for every channel within 2^-14 of the largest, the
+// rest off by at most 2^-25 of it.
+template <int E>
+__device__ __forceinline__ int q_normalize(half8 (&qB)[4]) {
+  constexpr int kMant = E == kEltBf16 ? 7 : 10, kBias = E == kEltBf16 ? 126 : 14;
+  uint32_t top = 0;
+#pragma unroll
+  for (int c = 0; c < 4; ++c)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const uint32_t u = as_u4(qB[c])[i];
+      top = max(top, max(u & 0x7FFFu, (u >> 16) & 0x7FFFu));
+    }
+#pragma unroll
+  for (int off = 32; off >= 1; off >>= 1) top = max(top, (uint32_t)__shfl_xor((int)top, off));
+  const int e = __builtin_amdgcn_readfirstlane((int)(top >> kMant)) - kBias;
+#pragma unroll
+  for (int c = 0; c < 4; ++c) {
+    const u32x4 u = as_u4(qB[c]);
+    half8 h;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      const uint32_t w = u[j >> 1];
+      float f;
+      if constexpr (E == kEltBf16) {
+        f = __builtin_bit_cast(float, (j & 1) ? w & 0xFFFF0000u : w << 16);
+      } else {
+        const uint16_t hb = (uint16_t)(w >> (16 * (j & 1)));
+        f = (float)__builtin_bit_cast(_Float16, hb);
+      }
+      h[j] = (_Float16)__builtin_ldexpf(f, -e);
+    }
+    qB[c] = h;
+  }
+  return e;
 }
 
 // Consume the staged tile (xlim real tokens: the sink group has at most 16).

@@ -167,13 +167,14 @@ def sparse_decode_attention_quantized(
     build_quantized_kv_cache returns then) and there is no window-old part.
     ``seq_len`` may also be a [BATCH] int32 tensor on the GPU: each sequence
     is masked at its own length (ramp-up per sequence).
-    ``bits`` / ``group_size`` other than 2 / 32 (caches from
+    ``bits`` / ``group_size`` other than 2 / 32 are those of caches from
     quantize_k_cache / quantize_v_cache with the same arguments, the sink
-    padded to one group) take the generic fp32 kernel: 1..8-bit codes,
+    padded to one group: 1..8-bit codes,
     8 // bits per byte, groups that divide D_HEAD and hold whole bytes.
     q and the residual may each be fp16, bf16 or fp32 (quant_kernel.py:
-    436-548 loads them in their own dtype); o has q's dtype.  Anything but
-    fp16 / fp16 takes the generic fp32 kernel.
+    436-548 loads them in their own dtype); o has q's dtype.  2- and 4-bit
+    codes in groups of 32 with fp16 or bf16 for both run on the matrix
+    cores, the rest takes the generic fp32 kernel.
     """
     tensors = dict(zip(_KIVI_ORDER, (k_sink_packed, k_sink_scale, k_sink_zero,
                                      v_sink_packed, v_sink_scale, v_sink_zero,
@@ -223,7 +224,7 @@ def sparse_decode_attention_quantized(
     arr = (K._vp * 12)(*[K.ptr(tensors[n]) if tensors[n].numel() else None for n in _KIVI_ORDER])
     if q.dtype != torch.float16 or k_cache.dtype != torch.float16:
         # quant_kernel.py:436-548 loads q and the residual in their own dtype
-        # and stores o in q's: the generic kernel (fp32 arithmetic)
+        # and stores o in q's
         lens = K.ptr(seq_len) if varlen else None
         rc = K.lib.kvdec_sparse_decode_kivi_typed(K.ptr(q), K.ptr(k_cache), K.ptr(v_cache), arr, K.ptr(o),
                                                   _checks.ATTN_DTYPES[q.dtype],

@@ -1,0 +1,124 @@
+"""The KIVI decode on the matrix cores at 4-bit codes and under bf16 queries,
+against the fp64 oracle: window-old group counts from none to several per wave,
+partial residuals, sinks up to the form's limit and past it, ramp-up with
+never-written slots, per-sequence lengths, scales far from 1, and the calls
+that stay with the generic kernel (other widths, types, groups, alignments)."""
+
+import numpy as np
+import pytest
+import torch
+
+from helpers import SCALE, assert_nearly_rounded, dev, randn, say
+from oracle import kvdec_oracle as O
+
+pytestmark = pytest.mark.gpu
+
+DT = {"fp16": torch.float16, "bf16": torch.bfloat16}
+
+
+def _check(o, ref, dt):
+    """fp16: half an ulp plus the repository's 5e-5; bf16: half an ulp plus
+    1e-5, a few fp32 ulps of logits up to ~20 (the x10 channel) and of the
+    two-part products."""
+    ref = np.asarray(ref, dtype=np.float64)
+    if dt == "fp16":
+        return assert_nearly_rounded(o.cpu().numpy(), ref)
+    e = np.floor(np.log2(np.maximum(np.abs(ref), 2.0**-126)))
+    assert (np.abs(o.float().cpu().numpy() - ref) - 2.0 ** (e - 8)).max() <= 1e-5
+
+
+def _cache(B, KVH, S, W, R, bits, dt, seed, k_mul=1.0, v_mul=1.0):
+    kc = randn((B, KVH, S + W, 128), seed) * k_mul
+    kc[..., 3] *= 10
+    vc = randn((B, KVH, S + W, 128), seed + 1) * v_mul
+    kc, vc = (torch.from_numpy(x).to(DT[dt]) for x in (kc, vc))
+    hc = O.build_quantized_kv_cache(kc.float().numpy(), vc.float().numpy(), residual_size=R, sink=S, bits=bits)
+    res = min(R, W)
+    hc["k_residual"], hc["v_residual"] = (x[:, :, -res:].float().numpy() for x in (kc, vc))
+    return hc
+
+
+def _upload(hc, dt, device):
+    return {k: dev(v, device).to(DT[dt]) if k.endswith("residual") else dev(v, device) for k, v in hc.items()}
+
+
+def _attend(q, c, L, W, S, R, bits):
+    from quant_kernel import sparse_decode_attention_quantized
+    return sparse_decode_attention_quantized(q, *[c[k] for k in O.CACHE_KEYS], seq_len=L, window=W, sink=S,
+                                             residual_size=R, bits=bits)
+
+
+@pytest.mark.parametrize("bits,dt", [(4, "fp16"), (4, "bf16"), (2, "bf16")])
+@pytest.mark.parametrize("W,S,R", [(40, 4, 128), (128, 16, 128), (160, 4, 128), (128 + 32 * 9, 1, 128),
+                                   (100 + 32 * 3, 4, 100), (128 + 32 * 61, 3, 128), (256, 17, 128), (352, 4, 160)])
+def test_forms(bits, dt, W, S, R, device):
+    B, H, KVH = 2, 64, 8
+    hc = _cache(B, KVH, S, W, R, bits, dt, 10 * bits + W)
+    c = _upload(hc, dt, device)
+    q = torch.from_numpy(randn((B, H, 128), 3)).to(DT[dt])
+    qh = q.float().numpy()
+    for L in (163840, S + W - 5, S + W // 3, 2):
+        say(f"kivi bits={bits} {dt} W={W} S={S} R={R} L={L}")
+        o = _attend(q.to(device), c, L, W, S, R, bits)
+        _check(o, O.quantized_attention_masked(qh, hc, L, W, SCALE, sink=S, residual_size=R, bits=bits), dt)
+    lens = np.array([S + W // 2, 90000], dtype=np.int32)
+    o = _attend(q.to(device), c, dev(lens, device), W, S, R, bits)
+    _check(o, O.quantized_attention_varlen(qh, hc, lens, W, SCALE, sink=S, residual_size=R, bits=bits), dt)
+
+
+@pytest.mark.parametrize("bits,dt", [(4, "fp16"), (4, "bf16"), (2, "bf16")])
+@pytest.mark.parametrize("q_mul,k_mul,v_mul", [(1e-3, 1e3, 1.0), (300.0, 1e-3, 1.0), (1.0, 1.0, 300.0),
+                                               (1.0, 1.0, 1e-3)])
+def test_scales_far_from_one(bits, dt, q_mul, k_mul, v_mul, device):
+    """Logits of the usual size from large and small factors, and outputs of
+    any size: relative to the largest output the bounds above hold."""
+    B, H, KVH, S, W, R = 1, 16, 2, 4, 448, 128
+    hc = _cache(B, KVH, S, W, R, bits, dt, 77, k_mul, v_mul)
+    q = (torch.from_numpy(randn((B, H, 128), 5)) * q_mul).to(DT[dt])
+    say(f"kivi bits={bits} {dt} q x {q_mul} k x {k_mul} v x {v_mul}")
+    o = _attend(q.to(device), _upload(hc, dt, device), 163840, W, S, R, bits)
+    ref = O.quantized_attention_masked(q.float().numpy(), hc, 163840, W, SCALE, sink=S, residual_size=R, bits=bits)
+    got, top = o.double().cpu().numpy(), np.abs(ref).max()
+    ulp = 2.0 ** (np.floor(np.log2(np.maximum(np.abs(ref), 1e-30))) - (11 if dt == "fp16" else 8))
+    # below fp16's normal range the output's own spacing is 2^-24
+    assert (np.abs(got - ref) - ulp).max() <= 1e-5 * top + (2.0**-25 if dt == "fp16" else 0.0)
+
+
+@pytest.mark.parametrize("bits,dt", [(4, "fp16"), (2, "bf16")])
+def test_slots_never_written(bits, dt, device):
+    """NaN patterns in every quantized byte and residual row of slots past the
+    sequence's length must not reach the output."""
+    B, H, KVH, S, W, R, L = 1, 64, 8, 4, 512, 128, 300
+    hc = _cache(B, KVH, S, W, R, bits, dt, 21)
+    c = _upload(hc, dt, device)
+    valid = O.slot_validity(L, W, S, 0)
+    dead = (~valid[S:S + W - R]).reshape(-1, 32)
+    whole = torch.from_numpy(dead.all(1))
+    tok = torch.from_numpy(~valid[S:S + W - R])
+    for n in ("k_win_scale", "k_win_zero"):
+        c[n][:, :, whole] = float("nan")
+    for n in ("v_win_scale", "v_win_zero"):
+        c[n][:, :, tok] = float("nan")
+    q = torch.from_numpy(randn((B, H, 128), 6)).to(DT[dt])
+    say(f"kivi bits={bits} {dt} with never-written slots")
+    o = _attend(q.to(device), c, L, W, S, R, bits)
+    _check(o, O.quantized_attention_masked(q.float().numpy(), hc, L, W, SCALE, sink=S, residual_size=R, bits=bits), dt)
+
+
+def test_stays_generic(device):
+    """Groups of more than 8 query heads and tensors off a 16-byte boundary."""
+    B, H, KVH, S, W, R, bits = 1, 32, 2, 4, 320, 128, 4
+    hc = _cache(B, KVH, S, W, R, bits, "bf16", 31)
+    c = _upload(hc, "bf16", device)
+    q = torch.from_numpy(randn((B, H, 128), 8)).to(torch.bfloat16)
+    ref = O.quantized_attention_masked(q.float().numpy(), hc, 9999, W, SCALE, sink=S, residual_size=R, bits=bits)
+    say("kivi 4-bit, 16 heads per KV head")
+    _check(_attend(q.to(device), c, 9999, W, S, R, bits), ref, "bf16")
+    q = q[:, :16].contiguous()
+    ref = O.quantized_attention_masked(q.float().numpy(), hc, 9999, W, SCALE, sink=S, residual_size=R, bits=bits)
+    x = c["v_win_packed"]
+    buf = torch.zeros(x.numel() + 1, dtype=torch.uint8, device=device)
+    buf[1:] = x.flatten()
+    c["v_win_packed"] = buf[1:].view(x.shape)
+    say("kivi 4-bit, codes off a 16-byte boundary")
+    _check(_attend(q.to(device), c, 9999, W, S, R, bits), ref, "bf16")
