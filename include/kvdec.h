@@ -168,8 +168,9 @@ int kvdec_sparse_decode_varlen(const void* q, const void* k_cache, const void* v
  *            token pf*p+j in bits j*bits .. j*bits + bits - 1
  *   scale, zero : [B, KVH, N/group, D] fp16
  *   1 <= bits <= 8, N % group == 0, group % pf == 0 (whole bytes per group).
- *   bits == 2 with group == 32 (D even) is the fast path, anything else a
- *   generic kernel.  QMAX = 2^bits - 1; codes are bit-exact to the
+ *   bits of 1, 2, 4 or 8 with group == 32 (D even, tensors on 16-byte
+ *   boundaries) is the fast path, anything else a generic kernel.
+ *   QMAX = 2^bits - 1; codes are bit-exact to the
  *   IEEE-float32 closed form s = (mx - mn) / QMAX, ... (quant_kernel.py:77-99).
  */
 int kvdec_quantize_k(const void* x, int in_dtype, void* packed_u8,
@@ -182,8 +183,8 @@ int kvdec_quantize_k(const void* x, int in_dtype, void* packed_u8,
  * (quantize_v_cache) and quant_kernel.py:129-190.
  *   packed : [B, KVH, N, D/pf] u8, code of channel pf*c+j in bits j*bits ..
  *   scale, zero : [B, KVH, N, D/group] fp16
- *   1 <= bits <= 8, D % group == 0, group % pf == 0; bits == 2 with group
- *   == 32 is the fast path.
+ *   1 <= bits <= 8, D % group == 0, group % pf == 0; the fast path as
+ *   for kvdec_quantize_k.
  */
 int kvdec_quantize_v(const void* x, int in_dtype, void* packed_u8,
                      void* scale_f16, void* zero_f16, int64_t B, int32_t KVH,

@@ -18,10 +18,10 @@ namespace kvdec {
 constexpr int kQGroup = 32;
 
 // Scale and zero-point of one group (float32, the reference's formula,
-// quant_kernel.py:77-81 for K and :166-170 for V).
-__device__ __forceinline__ void group_params(float mn, float mx, float& s, float& z) {
+// quant_kernel.py:77-81 for K and :166-170 for V); qmax = 2^bits - 1.
+__device__ __forceinline__ void group_params(float mn, float mx, float& s, float& z, float qmax = 3.0f) {
 #pragma clang fp contract(off)
-  s = (mx - mn) / 3.0f;
+  s = (mx - mn) / qmax;
   s = (s == 0.0f) ? 1.0f : s;
   z = floorf(-mn / s + 0.5f);
 }
@@ -33,23 +33,23 @@ struct QParams {
   bool fast;
 };
 
-__device__ __forceinline__ QParams make_params(float mn, float mx) {
+__device__ __forceinline__ QParams make_params(float mn, float mx, float qmax = 3.0f) {
 #pragma clang fp contract(off)
   QParams q;
-  group_params(mn, mx, q.s, q.z);
+  group_params(mn, mx, q.s, q.z, qmax);
   q.fast = q.s >= 0x1p-40f && q.s <= 0x1p100f;
   q.y = 1.0f / q.s;
   q.rinv = 1.0 / (double)q.s;
   return q;
 }
 
-// clamp(floor(fl32(x / s) + 0.5) + z, 0, 3) as a float (see file header).
+// clamp(floor(fl32(x / s) + 0.5) + z, 0, qmax) as a float (see file header).
 // E is float or _Float16.  q0 is formed as fma(x, y, +0), equal to fl32(x * y)
 // up to the sign of a zero (which cannot change a code), so that a 16-bit x
 // enters both FMAs unconverted.  The slow path converts x to double
 // directly, which keeps the two paths from sharing a converted copy of x.
 template <bool FAST, typename E>
-__device__ __forceinline__ float quant_code(E x, const QParams& q) {
+__device__ __forceinline__ float quant_code(E x, const QParams& q, float qmax = 3.0f) {
 #pragma clang fp contract(off)
   float qv;
   if (FAST) {
@@ -60,10 +60,10 @@ __device__ __forceinline__ float quant_code(E x, const QParams& q) {
     qv = (float)((double)x * q.rinv);
   }
   const float c = floorf(qv + 0.5f) + q.z;
-  return fminf(fmaxf(c, 0.0f), 3.0f);
+  return fminf(fmaxf(c, 0.0f), qmax);
 }
 
-// Replace byte `b` of `w` by the code c (an integer-valued float in [0, 3]).
+// Replace byte `b` of `w` by the code c (an integer-valued float in [0, 255]).
 __device__ __forceinline__ uint32_t put_code(float c, uint32_t b, uint32_t w) {
   return __builtin_amdgcn_cvt_pk_u8_f32(c, b, w);
 }

@@ -1,4 +1,5 @@
-// KIVI 2-bit quantizers (K per-channel, V per-token, groups of 32) and the
+// KIVI quantizers (K per-channel, V per-token; 2 bits in groups of 32 and the
+// other widths; the closed form below is that of 2 bits, 3 = 2^bits - 1) and the
 // isolated tile dequantizers, for gfx950, with their C-ABI entry points.
 //
 // Codes must be bit-exact to the IEEE-float32 closed form
@@ -152,11 +153,13 @@ __device__ __forceinline__ auto k_elem(const KRaw<T>& r, int t, int c) {
   return Fmt<T>::elem(r.w[2 * t + c], 0);
 }
 
-template <typename T>
+template <typename T, int BITS>
 __device__ __forceinline__ void k_quantize(const KRaw<T>& r, KUnit u, int D, int lane,
                                            uint8_t* __restrict__ packed,
                                            _Float16* __restrict__ scale,
                                            _Float16* __restrict__ zero) {
+  constexpr int kPf = 8 / BITS, kRows = kGroup / kPf;   // codes per byte, byte rows of the group
+  constexpr float kQmax = (float)((1 << BITS) - 1);
   // lanes past D compute codes of zeros and store out of range (dropped)
   const int ch = u.chunk * 128 + 2 * lane;
   const uint32_t vo = ch < D ? (uint32_t)ch : kOOB;
@@ -173,20 +176,20 @@ __device__ __forceinline__ void k_quantize(const KRaw<T>& r, KUnit u, int D, int
     minmax<T, kGroup, kW>(r.w, 0, amn, amx);
     minmax<T, kGroup, kW>(r.w + (kW - 1), kW == 1 ? 1 : 0, bmn, bmx);
   }
-  const QParams qa = make_params(amn, amx), qb = make_params(bmn, bmx);
-  // byte p of each channel holds the codes of tokens 4p .. 4p + 3, LSB first
-  uint32_t rows[kGroup / 4];
+  const QParams qa = make_params(amn, amx, kQmax), qb = make_params(bmn, bmx, kQmax);
+  // byte p of each channel holds the codes of tokens kPf p .., LSB first
+  uint32_t rows[kRows];
   auto codes = [&](auto fast) {
     constexpr bool F = decltype(fast)::value;
 #pragma unroll
-    for (int p = 0; p < kGroup / 4; ++p) {
+    for (int p = 0; p < kRows; ++p) {
       uint32_t w = 0;
 #pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const int t = 4 * p + j;
-        const uint32_t c = put_code(quant_code<F>(k_elem(r, t, 1), qb), 1,
-                                    put_code(quant_code<F>(k_elem(r, t, 0), qa), 0, 0u));
-        w |= c << (2 * j);
+      for (int j = 0; j < kPf; ++j) {
+        const int t = kPf * p + j;
+        const uint32_t c = put_code(quant_code<F>(k_elem(r, t, 1), qb, kQmax), 1,
+                                    put_code(quant_code<F>(k_elem(r, t, 0), qa, kQmax), 0, 0u));
+        w |= c << (BITS * j);
       }
       rows[p] = w;
     }
@@ -196,10 +199,9 @@ __device__ __forceinline__ void k_quantize(const KRaw<T>& r, KUnit u, int D, int
     codes(std::true_type());
   else
     codes(std::false_type());
-  const rsrc_t rp = make_rsrc_uniform(packed + (size_t)u.pg * (kGroup / 4) * D,
-                                      (uint32_t)(kGroup / 4 * D));
+  const rsrc_t rp = make_rsrc_uniform(packed + (size_t)u.pg * kRows * D, (uint32_t)(kRows * D));
 #pragma unroll
-  for (int p = 0; p < kGroup / 4; ++p)
+  for (int p = 0; p < kRows; ++p)
     __builtin_amdgcn_raw_buffer_store_b16((uint16_t)rows[p], rp, vo, p * D, kStreamAux);
   const uint32_t mbytes = (uint32_t)D * 2, mo = vo == kOOB ? kOOB : 2 * vo;
   const half2v sv = {(_Float16)qa.s, (_Float16)qb.s};
@@ -214,7 +216,7 @@ __device__ __forceinline__ void k_quantize(const KRaw<T>& r, KUnit u, int D, int
 
 // Grid-stride loop over units, one wave per unit; the next unit's loads are
 // issued before the current unit is quantized.
-template <typename T>
+template <typename T, int BITS>
 __global__ __launch_bounds__(256) void quantize_k_kernel(const T* __restrict__ x,
                                                          uint8_t* __restrict__ packed,
                                                          _Float16* __restrict__ scale,
@@ -233,7 +235,7 @@ __global__ __launch_bounds__(256) void quantize_k_kernel(const T* __restrict__ x
     KRaw<T> nxt;
     const KUnit un = k_unit(unit + stride, chunks);
     k_load(x, un, unit + stride < n_units, D, lane, nxt);
-    k_quantize(cur, u, D, lane, packed, scale, zero);
+    k_quantize<T, BITS>(cur, u, D, lane, packed, scale, zero);
     cur = nxt;
     u = un;
   }
@@ -265,10 +267,12 @@ __device__ __forceinline__ auto v_elem(const VRaw<T>& r, int c) {
   return Fmt<T>::elem(r.w[c / k], c % k);
 }
 
-template <typename T>
+template <typename T, int BITS>
 __device__ __forceinline__ void v_quantize(const VRaw<T>& r, int64_t u, uint8_t* __restrict__ packed,
                                            _Float16* __restrict__ scale,
                                            _Float16* __restrict__ zero) {
+  constexpr int kPf = 8 / BITS;
+  constexpr float kQmax = (float)((1 << BITS) - 1);
   float mn, mx;
   if (std::is_same<T, _Float16>::value) {
     half2v hn, hx;
@@ -283,20 +287,21 @@ __device__ __forceinline__ void v_quantize(const VRaw<T>& r, int64_t u, uint8_t*
       mx = fmaxf(mx, (float)v_elem(r, c));
     }
   }
-  const QParams q = make_params(mn, mx);
-  // byte b of the 8 holds the codes of channels 4b .. 4b + 3, LSB first
-  u32x2 out;
+  const QParams q = make_params(mn, mx, kQmax);
+  // byte b holds the codes of channels kPf b .., LSB first
+  uint32_t out[BITS];
   auto codes = [&](auto fast) {
     constexpr bool F = decltype(fast)::value;
 #pragma unroll
-    for (int w = 0; w < 2; ++w) {
+    for (int w = 0; w < BITS; ++w) {
       uint32_t word = 0;
 #pragma unroll
-      for (int j = 0; j < 4; ++j) {
+      for (int j = 0; j < kPf; ++j) {
         uint32_t t = 0;
 #pragma unroll
-        for (int b = 0; b < 4; ++b) t = put_code(quant_code<F>(v_elem(r, 16 * w + 4 * b + j), q), b, t);
-        word |= t << (2 * j);
+        for (int b = 0; b < 4; ++b)
+          t = put_code(quant_code<F>(v_elem(r, kPf * (4 * w + b) + j), q, kQmax), b, t);
+        word |= t << (BITS * j);
       }
       out[w] = word;
     }
@@ -306,12 +311,22 @@ __device__ __forceinline__ void v_quantize(const VRaw<T>& r, int64_t u, uint8_t*
   else
     codes(std::false_type());
   // streaming (non-temporal) stores: outputs are not read again here
-  __builtin_nontemporal_store(out, reinterpret_cast<u32x2*>(packed) + u);
+  if constexpr (BITS % 4 == 0) {
+#pragma unroll
+    for (int i = 0; i < BITS / 4; ++i)
+      __builtin_nontemporal_store(u32x4{out[4 * i], out[4 * i + 1], out[4 * i + 2], out[4 * i + 3]},
+                                  reinterpret_cast<u32x4*>(packed) + (size_t)u * (BITS / 4) + i);
+  } else if constexpr (BITS == 2) {
+    __builtin_nontemporal_store(u32x2{out[0], out[1]}, reinterpret_cast<u32x2*>(packed) + u);
+  } else {
+    static_assert(BITS == 1, "one 32-bit word");
+    __builtin_nontemporal_store(out[0], reinterpret_cast<uint32_t*>(packed) + u);
+  }
   __builtin_nontemporal_store((_Float16)q.s, scale + u);
   __builtin_nontemporal_store((_Float16)q.z, zero + u);
 }
 
-template <typename T>
+template <typename T, int BITS>
 __global__ __launch_bounds__(256) void quantize_v_kernel(const T* __restrict__ x,
                                                          uint8_t* __restrict__ packed,
                                                          _Float16* __restrict__ scale,
@@ -325,7 +340,7 @@ __global__ __launch_bounds__(256) void quantize_v_kernel(const T* __restrict__ x
   for (; u < n_units; u += stride) {
     VRaw<T> nxt;
     v_load(x, u + stride, n_units, nxt);
-    v_quantize(cur, u, packed, scale, zero);
+    v_quantize<T, BITS>(cur, u, packed, scale, zero);
     cur = nxt;
   }
 }
@@ -334,7 +349,7 @@ __global__ __launch_bounds__(256) void quantize_v_kernel(const T* __restrict__ x
 // BITS and GROUP_SIZE as parameters): QMAX = 2^bits - 1, 8 / bits codes per
 // byte at bits j * bits, LSB first.  One thread per (group, channel) of K or
 // (token, channel group) of V, reading its inputs twice (min / max, then the
-// codes); the 2-bit, 32-group kernels above are the fast path.  The
+// codes); the streaming kernels above take what stream_form names.  The
 // quotient is the HIP default fp32 division, correctly rounded like the
 // reference's IEEE division.
 template <typename T>
@@ -645,6 +660,34 @@ int launch_quant_generic(bool k, const void* x, int in_dtype, void* packed_u8, v
   return launch_status();
 }
 
+// Groups of 32 with 1, 2, 4 or 8 bits take the streaming kernels above, which
+// read the input once and divide by Markstein's sequence (bound by the
+// read/write mix); the rest, and tensors that do not allow their accesses (the
+// 2-bit form has always assumed them), the generic ones: K and V of B=8, N=4096,
+// bf16 at 4 bits 236.6 -> 32.3 us (5.4 TB/s of input and output; there two reads
+// of the input, an IEEE division per element and byte stores).
+bool stream_form(const void* x, const void* p, const void* s, const void* z, int group, int bits) {
+  if (group != kGroup || (bits & (bits - 1)) != 0) return false;
+  if (bits == 2) return true;
+  return (((uintptr_t)x | (uintptr_t)p) & 15u) == 0 && (((uintptr_t)s | (uintptr_t)z) & 3u) == 0;
+}
+
+template <typename F>
+int with_elt(int in_dtype, F&& f) {
+  if (in_dtype == KVDEC_F32) return f(float{});
+  if (in_dtype == KVDEC_F16) return f(_Float16{});
+  return f(uint16_t{});
+}
+template <typename F>
+int with_bits(int bits, F&& f) {
+  switch (bits) {
+    case 1: return f(std::integral_constant<int, 1>());
+    case 4: return f(std::integral_constant<int, 4>());
+    case 8: return f(std::integral_constant<int, 8>());
+    default: return f(std::integral_constant<int, 2>());
+  }
+}
+
 }  // namespace
 
 extern "C" {
@@ -655,34 +698,26 @@ int kvdec_quantize_k(const void* x, int in_dtype, void* packed_u8, void* scale_f
   int rc = check_quant_args(x, in_dtype, packed_u8, scale_f16, zero_f16, B, KVH, N, D, group, bits);
   if (rc) return rc;
   if (N % group != 0) return KVDEC_E_GROUP;
-  if (bits != 2 || group != kGroup) {
-    // any width: whole bytes per group
-    if (group % (8 / bits) != 0) return KVDEC_E_GROUP;
-    const int64_t n_units = B * KVH * (N / group) * D;
-    return launch_quant_generic(true, x, in_dtype, packed_u8, scale_f16, zero_f16, n_units, D, group,
-                                bits, stream);
-  }
-  if (D % 2 != 0) return KVDEC_E_SHAPE;
-  if ((int64_t)D * kGroup * 4 >= ((int64_t)1 << 31)) return KVDEC_E_SHAPE;   // 32-bit buffer offsets
-  const int64_t pairs = B * KVH;
-  const int64_t groups = N / kGroup;
+  if (group % (8 / bits) != 0) return KVDEC_E_GROUP;   // whole bytes per group
+  const int64_t groups = N / group;
+  const bool narrow = D % 2 == 0 && (int64_t)D * kGroup * 4 < ((int64_t)1 << 31);   // 32-bit buffer offsets
+  if (bits == 2 && group == kGroup && !narrow) return KVDEC_E_SHAPE;
+  if (!narrow || !stream_form(x, packed_u8, scale_f16, zero_f16, group, bits))
+    return launch_quant_generic(true, x, in_dtype, packed_u8, scale_f16, zero_f16, B * KVH * groups * D, D,
+                                group, bits, stream);
   const int chunks = (D + 127) / 128;
-  const int64_t n_units = pairs * groups * chunks;
+  const int64_t n_units = B * KVH * groups * chunks;
   const unsigned grid = grid_for(n_units * 64, 256);
-  hipStream_t st = static_cast<hipStream_t>(stream);
-  auto* p = static_cast<uint8_t*>(packed_u8);
-  auto* s = static_cast<_Float16*>(scale_f16);
-  auto* z = static_cast<_Float16*>(zero_f16);
-  if (in_dtype == KVDEC_F32)
-    hipLaunchKernelGGL(quantize_k_kernel<float>, dim3(grid), dim3(256), 0, st,
-                       static_cast<const float*>(x), p, s, z, n_units, D, chunks);
-  else if (in_dtype == KVDEC_F16)
-    hipLaunchKernelGGL(quantize_k_kernel<_Float16>, dim3(grid), dim3(256), 0, st,
-                       static_cast<const _Float16*>(x), p, s, z, n_units, D, chunks);
-  else
-    hipLaunchKernelGGL(quantize_k_kernel<uint16_t>, dim3(grid), dim3(256), 0, st,
-                       static_cast<const uint16_t*>(x), p, s, z, n_units, D, chunks);
-  return launch_status();
+  return with_elt(in_dtype, [&](auto elt) {
+    typedef decltype(elt) T;
+    return with_bits(bits, [&](auto width) {
+      hipLaunchKernelGGL((quantize_k_kernel<T, decltype(width)::value>), dim3(grid), dim3(256), 0,
+                         static_cast<hipStream_t>(stream), static_cast<const T*>(x),
+                         static_cast<uint8_t*>(packed_u8), static_cast<_Float16*>(scale_f16),
+                         static_cast<_Float16*>(zero_f16), n_units, D, chunks);
+      return launch_status();
+    });
+  });
 }
 
 int kvdec_quantize_v(const void* x, int in_dtype, void* packed_u8, void* scale_f16, void* zero_f16,
@@ -691,28 +726,20 @@ int kvdec_quantize_v(const void* x, int in_dtype, void* packed_u8, void* scale_f
   int rc = check_quant_args(x, in_dtype, packed_u8, scale_f16, zero_f16, B, KVH, N, D, group, bits);
   if (rc) return rc;
   if (D % group != 0) return KVDEC_E_DGROUP;
-  if (bits != 2 || group != kGroup) {
-    if (group % (8 / bits) != 0) return KVDEC_E_DGROUP;
-    const int64_t n_units = B * KVH * N * (D / group);
-    return launch_quant_generic(false, x, in_dtype, packed_u8, scale_f16, zero_f16, n_units, D, group,
-                                bits, stream);
-  }
-  const int64_t n_units = B * KVH * N * (D / kGroup);
-  const unsigned grid = grid_for(n_units, 256);
-  hipStream_t st = static_cast<hipStream_t>(stream);
-  auto* p = static_cast<uint8_t*>(packed_u8);
-  auto* s = static_cast<_Float16*>(scale_f16);
-  auto* z = static_cast<_Float16*>(zero_f16);
-  if (in_dtype == KVDEC_F32)
-    hipLaunchKernelGGL(quantize_v_kernel<float>, dim3(grid), dim3(256), 0, st,
-                       static_cast<const float*>(x), p, s, z, n_units);
-  else if (in_dtype == KVDEC_F16)
-    hipLaunchKernelGGL(quantize_v_kernel<_Float16>, dim3(grid), dim3(256), 0, st,
-                       static_cast<const _Float16*>(x), p, s, z, n_units);
-  else
-    hipLaunchKernelGGL(quantize_v_kernel<uint16_t>, dim3(grid), dim3(256), 0, st,
-                       static_cast<const uint16_t*>(x), p, s, z, n_units);
-  return launch_status();
+  if (group % (8 / bits) != 0) return KVDEC_E_DGROUP;
+  const int64_t n_units = B * KVH * N * (D / group);
+  if (!stream_form(x, packed_u8, scale_f16, zero_f16, group, bits))
+    return launch_quant_generic(false, x, in_dtype, packed_u8, scale_f16, zero_f16, n_units, D, group, bits, stream);
+  return with_elt(in_dtype, [&](auto elt) {
+    typedef decltype(elt) T;
+    return with_bits(bits, [&](auto width) {
+      hipLaunchKernelGGL((quantize_v_kernel<T, decltype(width)::value>), dim3(grid_for(n_units, 256)), dim3(256), 0,
+                         static_cast<hipStream_t>(stream), static_cast<const T*>(x),
+                         static_cast<uint8_t*>(packed_u8), static_cast<_Float16*>(scale_f16),
+                         static_cast<_Float16*>(zero_f16), n_units);
+      return launch_status();
+    });
+  });
 }
 
 int kvdec_kivi_stream_append(const void* k_new, const void* v_new, void* k_ring, void* v_ring,

@@ -13,8 +13,9 @@ Codes, scales and zeros are bit-exact to the IEEE-float32 closed form of the
 reference's formulas (s = (mx - mn) / 3, s := 1 if 0, z = floor(-mn / s + 0.5),
 code = clamp(floor(x / s + 0.5) + z, 0, 3)).  The quantizers and the fused
 decode also take the reference's ``bits`` (1..8, QMAX = 2^bits - 1, 8 // bits
-codes per byte) and ``group_size`` parameters; widths and groups other than
-2 / 32 run generic kernels (the 2-bit, 32-group kernels are the fast path).
+codes per byte) and ``group_size`` parameters; groups of 32 at 1, 2, 4 or 8 bits
+(quantizers) and 2 or 4 bits (decode) are the fast path, the rest runs generic
+kernels.
 """
 
 import torch
