@@ -123,24 +123,25 @@ __device__ __forceinline__ KUnit k_unit(int64_t unit, int chunks) {
   return KUnit{unit / chunks, (int)(unit % chunks)};
 }
 
-template <typename T>
-__device__ __forceinline__ void k_load(const T* x, KUnit u, bool live, int D, int lane,
-                                       KRaw<T>& r) {
+// The 32 rows of the group at `grp`, its channels chunk * 128 + 2 lane, + 1.
+// SINK: the group's rows past the first `sink` repeat row 0 (the padding of
+// the sink group).
+template <typename T, bool SINK = false>
+__device__ __forceinline__ void k_load(const T* grp, int chunk, int D, int lane, KRaw<T>& r, int sink = kGroup) {
   constexpr int kW = KRaw<T>::kW;
-  if (!live) return;
   // the group's 32 rows as one buffer: per-lane offset in a VGPR, per-row
   // offset in an SGPR (no 64-bit address arithmetic per load).  Lanes past
   // D read out of range: zeros, no access, no divergent branch.
-  const int ch = u.chunk * 128 + 2 * lane;
-  const rsrc_t rs = make_rsrc_uniform(x + (size_t)u.pg * kGroup * D,
-                                      (uint32_t)(kGroup * D * sizeof(T)));
+  const int ch = chunk * 128 + 2 * lane;
+  const rsrc_t rs = make_rsrc_uniform(grp, (uint32_t)((SINK ? sink : kGroup) * D * sizeof(T)));
   const uint32_t vo = ch < D ? (uint32_t)ch * sizeof(T) : kOOB, row = (uint32_t)D * sizeof(T);
 #pragma unroll
   for (int t = 0; t < kGroup; ++t) {
+    const uint32_t so = SINK && t >= sink ? 0u : t * row;
     if (kW == 1) {
-      r.w[t] = __builtin_amdgcn_raw_buffer_load_b32(rs, vo, t * row, kStreamAux);
+      r.w[t] = __builtin_amdgcn_raw_buffer_load_b32(rs, vo, so, kStreamAux);
     } else {
-      const u32x2 v = __builtin_amdgcn_raw_buffer_load_b64(rs, vo, t * row, kStreamAux);
+      const u32x2 v = __builtin_amdgcn_raw_buffer_load_b64(rs, vo, so, kStreamAux);
       r.w[2 * t] = v[0];
       r.w[2 * t + 1] = v[1];
     }
@@ -230,11 +231,11 @@ __global__ __launch_bounds__(256) void quantize_k_kernel(const T* __restrict__ x
   if (unit >= n_units) return;
   KRaw<T> cur;
   KUnit u = k_unit(unit, chunks);
-  k_load(x, u, true, D, lane, cur);
+  k_load(x + (size_t)u.pg * kGroup * D, u.chunk, D, lane, cur);
   for (; unit < n_units; unit += stride) {
     KRaw<T> nxt;
     const KUnit un = k_unit(unit + stride, chunks);
-    k_load(x, un, unit + stride < n_units, D, lane, nxt);
+    if (unit + stride < n_units) k_load(x + (size_t)un.pg * kGroup * D, un.chunk, D, lane, nxt);
     k_quantize<T, BITS>(cur, u, D, lane, packed, scale, zero);
     cur = nxt;
     u = un;
@@ -250,9 +251,8 @@ struct VRaw {
 };
 
 template <typename T>
-__device__ __forceinline__ void v_load(const T* x, int64_t u, int64_t n_units, VRaw<T>& r) {
-  if (u >= n_units) return;
-  const u32x4* p = reinterpret_cast<const u32x4*>(x + (size_t)u * kGroup);
+__device__ __forceinline__ void v_load(const T* grp, VRaw<T>& r) {
+  const u32x4* p = reinterpret_cast<const u32x4*>(grp);
 #pragma unroll
   for (int i = 0; i < VRaw<T>::kW / 4; ++i) {
     const u32x4 v = p[i];
@@ -336,10 +336,10 @@ __global__ __launch_bounds__(256) void quantize_v_kernel(const T* __restrict__ x
   int64_t u = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (u >= n_units) return;
   VRaw<T> cur;
-  v_load(x, u, n_units, cur);
+  v_load(x + (size_t)u * kGroup, cur);
   for (; u < n_units; u += stride) {
     VRaw<T> nxt;
-    v_load(x, u + stride, n_units, nxt);
+    if (u + stride < n_units) v_load(x + (size_t)(u + stride) * kGroup, nxt);
     v_quantize<T, BITS>(cur, u, packed, scale, zero);
     cur = nxt;
   }
@@ -551,6 +551,7 @@ __device__ __forceinline__ float elem(const void* p, size_t i) {
     return (float)static_cast<const T*>(p)[i];
 }
 
+// Any alignment; caches that allow 16-byte accesses take build_stream_kernel.
 template <typename T, typename RT>
 __global__ __launch_bounds__(256) void build_kernel(BuildArgs a) {
   const int64_t pair = blockIdx.x;
@@ -605,6 +606,98 @@ __global__ __launch_bounds__(256) void build_kernel(BuildArgs a) {
     a.vs[r][tok * ng + cg] = (_Float16)q.s;
     a.vz[r][tok * ng + cg] = (_Float16)q.z;
   }
+}
+
+// The same from caches that allow 16-byte accesses, on the quantizers' own
+// loads (wave-wide rows for K, 16 bytes a lane for V and the residual): each
+// KV head is a run of `bpp` workgroups: one for the sink group, rb of residual
+// rows (16 bytes of output per thread and step, K then V), kb of K window-old
+// groups (a wave each) and vb of V window-old (token, group)s (a thread each).
+// The sink and residual workgroups, whose threads take several steps, come
+// first: placed last they end the launch (131.1 -> 111.8 us).  Bound by the
+// read/write mix: B=32, W=4096, bf16 157.0 -> 111.8 us (5.8 TB/s) against
+// build_kernel (2-byte loads for K, a 64-byte stride between lanes for V), W=256
+// fp16 20.1 -> 15.8; waves per SIMD forced up by launch bounds (6, 8) measured
+// no faster (bf16) or spilled (8: 1.6x slower).
+struct BuildPlan {
+  unsigned kb, vb, rb, bpp;
+  int chunks;
+};
+
+// 16 bytes of output from as many elements of input.
+template <typename T, typename RT>
+__device__ __forceinline__ u32x4 convert16(const T* src) {
+  if constexpr (std::is_same<T, RT>::value) {
+    return *reinterpret_cast<const u32x4*>(src);
+  } else {
+    constexpr int n = 16 / sizeof(RT), words = n * sizeof(T) / 16;
+    static_assert(sizeof(RT) == 2, "converted residuals are fp16");
+    u32x4 w[words];
+#pragma unroll
+    for (int i = 0; i < words; ++i) w[i] = reinterpret_cast<const u32x4*>(src)[i];
+    half8 h;
+#pragma unroll
+    for (int i = 0; i < n; ++i) {
+      constexpr int k = Fmt<T>::kPerWord;
+      h[i] = (_Float16)Fmt<T>::get(w[i / k / 4][i / k % 4], i % k);
+    }
+    return as_u4(h);
+  }
+}
+
+template <typename T, typename RT>
+__global__ __launch_bounds__(256) void build_stream_kernel(BuildArgs a, BuildPlan B) {
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const uint32_t pair = blockIdx.x / B.bpp;
+  uint32_t blk = blockIdx.x - pair * B.bpp;
+  const int D = a.D, ng = D / kGroup, nwg = a.win_tok / kGroup;
+  const T* kc = static_cast<const T*>(a.kc) + (size_t)pair * a.n * D;
+  const T* vc = static_cast<const T*>(a.vc) + (size_t)pair * a.n * D;
+  if (blk == 0) {
+    // the sink group: the sink tokens, then token 0 again
+    for (int chunk = wave; chunk < B.chunks; chunk += 4) {
+      KRaw<T> r;
+      k_load<T, true>(kc, chunk, D, lane, r, a.sink);
+      k_quantize<T, 2>(r, KUnit{(int64_t)pair, chunk}, D, lane, a.kp[0], a.ks[0], a.kz[0]);
+    }
+    for (int u = 255 - (int)threadIdx.x; u < kGroup * ng; u += 256) {   // (the last waves first)
+      const int t = u / ng, cg = u % ng;
+      VRaw<T> r;
+      v_load(vc + (size_t)(t < a.sink ? t : 0) * D + cg * kGroup, r);
+      v_quantize<T, 2>(r, (int64_t)pair * kGroup * ng + u, a.vp[0], a.vs[0], a.vz[0]);
+    }
+    return;
+  }
+  blk -= 1;
+  if (blk < B.rb) {
+    constexpr int n = 16 / sizeof(RT);
+    const int total = a.res_rows * D / n;
+    const size_t src = (size_t)(a.n - a.res_rows) * D, dst = (size_t)pair * a.res_rows * D;
+    for (int i = (int)(blk * 256 + threadIdx.x); i < 2 * total; i += (int)B.rb * 256) {
+      const bool v = i >= total;
+      const size_t e = (size_t)(v ? i - total : i) * n;
+      const u32x4 x = convert16<T, RT>((v ? vc : kc) + src + e);
+      __builtin_nontemporal_store(x, reinterpret_cast<u32x4*>(static_cast<RT*>(v ? a.vres : a.kres) + dst + e));
+    }
+    return;
+  }
+  blk -= B.rb;
+  if (blk < B.kb) {
+    const int unit = (int)blk * 4 + wave;
+    if (unit >= nwg * B.chunks) return;
+    const int g = B.chunks == 1 ? unit : unit / B.chunks, chunk = B.chunks == 1 ? 0 : unit % B.chunks;
+    KRaw<T> r;
+    k_load(kc + (size_t)(a.sink + kGroup * g) * D, chunk, D, lane, r);
+    k_quantize<T, 2>(r, KUnit{(int64_t)pair * nwg + g, chunk}, D, lane, a.kp[1], a.ks[1], a.kz[1]);
+    return;
+  }
+  blk -= B.kb;
+  const int u = (int)(blk * 256 + threadIdx.x);
+  if (u >= a.win_tok * ng) return;
+  VRaw<T> r;
+  v_load(vc + (size_t)a.sink * D + (size_t)u * kGroup, r);
+  v_quantize<T, 2>(r, (int64_t)pair * a.win_tok * ng + u, a.vp[1], a.vs[1], a.vz[1]);
 }
 
 int launch_status() {
@@ -877,12 +970,30 @@ int kvdec_build_kivi_cache(const void* k_compacted, const void* v_compacted, int
     a.vs[r] = static_cast<_Float16*>(out[6 + 6 * r]);
     a.vz[r] = static_cast<_Float16*>(out[7 + 6 * r]);
   }
-  hipStream_t st = static_cast<hipStream_t>(stream);
+  const hipStream_t st = static_cast<hipStream_t>(stream);
+  const bool same = residual_dtype == in_dtype;
+  uintptr_t at = (uintptr_t)k_compacted | (uintptr_t)v_compacted;
+  for (int i = 0; i < (win_tok > 0 ? 14 : 8); ++i) at |= (uintptr_t)out[i];
+  BuildPlan plan{};
+  plan.chunks = (D + 127) / 128;
+  plan.kb = (unsigned)((win_tok / kGroup * plan.chunks + 3) / 4);
+  plan.vb = (unsigned)((win_tok * (D / kGroup) + 255) / 256);
+  plan.rb = (unsigned)std::max(1, res_rows * D / 2048);   // two steps of a thread at 2 bytes
+  plan.bpp = plan.kb + plan.vb + plan.rb + 1;
+  const int64_t blocks = B * KVH * (int64_t)plan.bpp;
+  if ((at & 15u) == 0 && blocks <= 0x7fffffffLL && (int64_t)D * kGroup * 4 < ((int64_t)1 << 31)) {
+    void (*kern)(BuildArgs, BuildPlan) = build_stream_kernel<_Float16, _Float16>;
+    if (in_dtype == KVDEC_F32)
+      kern = same ? build_stream_kernel<float, float> : build_stream_kernel<float, _Float16>;
+    else if (in_dtype == KVDEC_BF16)
+      kern = same ? build_stream_kernel<uint16_t, uint16_t> : build_stream_kernel<uint16_t, _Float16>;
+    hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(256), 0, st, a, plan);
+    return launch_status();
+  }
   // about 1024 work items per workgroup, at most 64 workgroups per head
   const int64_t items = std::max<int64_t>((int64_t)res_rows * D, (int64_t)(kGroup + win_tok) * (D / kGroup));
   const unsigned split = (unsigned)std::min<int64_t>(64, std::max<int64_t>(1, (items + 1023) / 1024));
   const dim3 grid((unsigned)(B * KVH), split);
-  const bool same = residual_dtype == in_dtype;
   void (*kern)(BuildArgs) = build_kernel<_Float16, _Float16>;
   if (in_dtype == KVDEC_F32)
     kern = same ? build_kernel<float, float> : build_kernel<float, _Float16>;
