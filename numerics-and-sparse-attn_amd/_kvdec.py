@@ -110,6 +110,20 @@ def _load() -> ctypes.CDLL:
 lib = _load()
 
 
+def _load_host():
+    """The wrappers' native fast path (csrc/host.cpp), bound to the library
+    loaded above: each function makes a whole call, or returns None for a call
+    that the wrapper itself has to check (and refuse, or convert)."""
+    try:
+        import _kvdec_host
+    except ModuleNotFoundError as e:
+        raise ImportError(
+            f"_kvdec_host.so is missing: build it with `python {os.path.join(_HERE, 'build.py')}` "
+            "(or __graft_entry__.build())") from e
+    _kvdec_host.bind(LIB_PATH, check)
+    return _kvdec_host
+
+
 class KvdecLaunchError(RuntimeError):
     """A HIP launch inside libkvdec failed (positive return code)."""
 
@@ -147,3 +161,6 @@ def workspace(kind: int, B: int, H: int, KVH: int, n_slots: int, D: int, device)
     if nbytes == 0:
         return None, 0
     return torch.empty(nbytes, dtype=torch.uint8, device=device), nbytes
+
+
+host = _load_host()

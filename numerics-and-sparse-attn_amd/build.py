@@ -7,6 +7,9 @@ selection disabled; quant.hip additionally forbids FP contraction so its codes
 match the IEEE closed form bit for bit.  The shared library lands next to this
 file, where the ctypes loader (_kvdec.py) looks for it.
 
+host.cpp, the wrappers' native fast path, becomes the CPython module
+_kvdec_host.so (g++, torch's C++ interface).
+
 The same sources also make libkvdec_clock.so, the timing build: attn.hip
 compiled with -DKVDEC_CLOCK, whose attention kernels record the GPU realtime
 counter at their start and end into a log armed by kvdec_clock_arm (the
@@ -15,10 +18,12 @@ loader takes it when KVDEC_LIBRARY=clock; bench.py --kernel-clock).
 
 from __future__ import annotations
 
+import importlib.util
 import os
 import shutil
 import subprocess
 import sys
+import sysconfig
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
@@ -40,6 +45,7 @@ OBJECTS = (
     ("quant", "quant.hip", ["-ffp-contract=off"]),
     ("generic", "generic.hip", []),
 )
+HOST_LIB_PATH = os.path.join(HERE, "_kvdec_host.so")
 LIBRARIES = (
     (LIB_PATH, ("attn", "quant", "generic")),
     (CLOCK_LIB_PATH, ("attn_clock", "quant", "generic")),
@@ -65,6 +71,22 @@ def _hipcc() -> str:
     raise RuntimeError("hipcc not found (ROCm toolchain required to build libkvdec.so)")
 
 
+def _host_command() -> list[str]:
+    """g++ line of the wrappers' native fast path, a CPython module on torch's
+    C++ interface (host code only)."""
+    cxx = shutil.which("g++")
+    if not cxx:
+        raise RuntimeError("g++ not found (required to build _kvdec_host.so)")
+    torch_dir = importlib.util.find_spec("torch").submodule_search_locations[0]
+    rocm = os.path.dirname(os.path.dirname(os.path.realpath(_hipcc())))
+    return [cxx, "-O2", "-fPIC", "-shared", "-std=c++17", "-Wall", "-DUSE_ROCM", "-D__HIP_PLATFORM_AMD__",
+            "-I", INCLUDE, "-isystem", os.path.join(torch_dir, "include"),
+            "-isystem", os.path.join(torch_dir, "include", "torch", "csrc", "api", "include"),
+            "-isystem", os.path.join(rocm, "include"), "-isystem", sysconfig.get_paths()["include"],
+            os.path.join(CSRC, "host.cpp"), "-o", HOST_LIB_PATH + ".tmp",
+            "-L", os.path.join(torch_dir, "lib"), "-lc10", "-lc10_hip", "-ltorch_cpu", "-ltorch_python", "-ldl"]
+
+
 def _filter_host_feature_warning(text: str) -> str:
     # The host pass does not know the GPU-only target feature; that warning
     # is expected and harmless.
@@ -73,8 +95,8 @@ def _filter_host_feature_warning(text: str) -> str:
 
 
 def build(verbose: bool = False) -> str:
-    """Compile every HIP source and link libkvdec.so and the timing build
-    libkvdec_clock.so; returns the product library's path."""
+    """Compile every source and link libkvdec.so, the timing build
+    libkvdec_clock.so and the fast path's _kvdec_host.so; returns the product library's path."""
     hipcc = _hipcc()
     os.makedirs(BUILD_DIR, exist_ok=True)
     procs = []
@@ -86,6 +108,10 @@ def build(verbose: bool = False) -> str:
             print(" ".join(cmd), flush=True)
         procs.append((name, subprocess.Popen(cmd, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)))
         objs[name] = obj
+    cmd = _host_command()
+    if verbose:
+        print(" ".join(cmd), flush=True)
+    procs.append(("host", subprocess.Popen(cmd, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)))
     failed = []
     for name, p in procs:
         out, _ = p.communicate()
@@ -95,7 +121,8 @@ def build(verbose: bool = False) -> str:
         if p.returncode:
             failed.append(name)
     if failed:
-        raise RuntimeError(f"hipcc failed on {', '.join(failed)}")
+        raise RuntimeError(f"compiling {', '.join(failed)} failed")
+    os.replace(HOST_LIB_PATH + ".tmp", HOST_LIB_PATH)
     for lib, names in LIBRARIES:
         tmp = lib + ".tmp"
         cmd = [hipcc, f"--offload-arch={ARCH}", "-shared", "-fPIC", "-o", tmp, *[objs[n] for n in names]]

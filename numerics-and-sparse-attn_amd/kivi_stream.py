@@ -287,6 +287,11 @@ class KiviStreamBatch:
         (b, kv) workgroup writes its token's row and quantizes its evicted
         block before it attends); returns o [B, H, D].  Leaves the cache as
         the two calls do."""
+        o = K.host.step_attend(self.t, q, k_new, v_new, active, self.appended, self.arrive, self.plan, self.ring,
+                               self.sink, self.residual, self.n_groups, self.cap, GROUP_SIZE, QUANT_BITS,
+                               D_HEAD**-0.5 if sm_scale is None else sm_scale)
+        if o is not None:
+            return o
         B, KVH, D = self.shape
         k_new = k_new.reshape(B, KVH, D).contiguous()
         v_new = v_new.reshape(B, KVH, D).contiguous()

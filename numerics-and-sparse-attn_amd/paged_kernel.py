@@ -36,6 +36,10 @@ def paged_decode_attention(q, k_pages, v_pages, block_table, seq_lens, max_seq_l
     """
     if kv_layout not in _LAYOUTS:
         raise ValueError(f"kv_layout must be one of {_LAYOUTS}, got {kv_layout!r}")
+    o = K.host.paged(q, k_pages, v_pages, block_table, seq_lens, max_seq_len,
+                     D_HEAD**-0.5 if sm_scale is None else sm_scale, kv_layout == "HND")
+    if o is not None:
+        return o
     _checks.require_gpu_tensor("q", q, ndim=3)
     _checks.require_gpu_tensor("k_pages", k_pages, ndim=4, contiguous=False)
     _checks.require_gpu_tensor("v_pages", v_pages, ndim=4, contiguous=False)

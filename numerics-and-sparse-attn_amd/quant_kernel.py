@@ -41,6 +41,9 @@ def quantize_k_cache(k, group_size=GROUP_SIZE, bits=QUANT_BITS):
     conversion to fp32 is exact, so the codes are the same).
     Shapes: packed [B, KVH, seq_len/4, D] u8; scale, zero [B, KVH, seq_len/group, D] fp16.
     """
+    out = K.host.quantize(k, group_size, bits, False)
+    if out is not None:
+        return out
     batch, n_kv_heads, seq_len, d_head = k.shape
     if seq_len % group_size != 0:
         raise AssertionError("this simple version assumes seq_len is a multiple of group_size")
@@ -70,6 +73,9 @@ def quantize_v_cache(v, group_size=GROUP_SIZE, bits=QUANT_BITS):
     Mirrors quant_kernel.py:193-214.  Shapes: packed [B, KVH, seq_len, D/4] u8;
     scale, zero [B, KVH, seq_len, D/group] fp16.
     """
+    out = K.host.quantize(v, group_size, bits, True)
+    if out is not None:
+        return out
     batch, n_kv_heads, seq_len, d_head = v.shape
     if d_head % group_size != 0:
         raise AssertionError("this simple version assumes D_HEAD is a multiple of group_size")
@@ -177,6 +183,12 @@ def sparse_decode_attention_quantized(
     codes in groups of 32 with fp16 or bf16 for both run on the matrix
     cores, the rest takes the generic fp32 kernel.
     """
+    o = K.host.kivi(q, k_cache, v_cache, k_sink_packed, k_sink_scale, k_sink_zero, v_sink_packed, v_sink_scale,
+                    v_sink_zero, k_win_packed, k_win_scale, k_win_zero, v_win_packed, v_win_scale, v_win_zero,
+                    seq_len, window, sink, residual_size, group_size, bits,
+                    D_HEAD**-0.5 if sm_scale is None else sm_scale)
+    if o is not None:
+        return o
     tensors = dict(zip(_KIVI_ORDER, (k_sink_packed, k_sink_scale, k_sink_zero,
                                      v_sink_packed, v_sink_scale, v_sink_zero,
                                      k_win_packed, k_win_scale, k_win_zero,
@@ -266,6 +278,11 @@ def build_quantized_kv_cache(k_compacted, v_compacted, residual_size=RESIDUAL_SI
     the residual) keeps the whole window as the residual and has no
     window-old part.
     """
+    if residual_dtype is None or residual_dtype is torch.float16:
+        out = K.host.build(k_compacted, v_compacted, residual_size, sink, GROUP_SIZE, QUANT_BITS,
+                           residual_dtype is torch.float16)
+        if out is not None:
+            return out
     _checks.require_gpu_tensor("k_compacted", k_compacted, dtypes=tuple(_IN_DTYPES), ndim=4,
                                contiguous=False)
     _checks.require_gpu_tensor("v_compacted", v_compacted, dtypes=tuple(_IN_DTYPES), ndim=4,

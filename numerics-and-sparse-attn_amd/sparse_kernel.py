@@ -28,6 +28,10 @@ def sparse_decode_attention(q, k_cache, v_cache, seq_len, window, sink=SINK_SIZE
     kernel.  ``seq_len`` may also be a [BATCH] int32 tensor on the GPU: each
     sequence is masked at its own length (each >= 1).
     """
+    o = K.host.sparse(q, k_cache, v_cache, seq_len, window, sink, _LAYOUTS.get(layout),
+                      D_HEAD**-0.5 if sm_scale is None else sm_scale)
+    if o is not None:
+        return o
     _checks.require_gpu_tensor("q", q, dtypes=tuple(_checks.ATTN_DTYPES), ndim=3)
     _checks.require_gpu_tensor("k_cache", k_cache, dtypes=(q.dtype,), ndim=4)
     _checks.require_gpu_tensor("v_cache", v_cache, dtypes=(q.dtype,), ndim=4)
