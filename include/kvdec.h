@@ -215,7 +215,7 @@ int kvdec_quantize_v(const void* x, int in_dtype, void* packed_u8,
  *   bits / group other than 2 / 32 (the tensors of kvdec_quantize_k / _v at
  *   that width, /4 above reading /pf): 4 / 32 with H / KVH <= 8, sink <= 16,
  *   residual <= 128 and tensors on 16-byte boundaries runs the MFMA kernel,
- *   anything else a generic kernel in fp32 arithmetic: 1 <= bits <= 8, D % group == 0, group % pf == 0,
+ *   anything else a generic kernel in fp32 arithmetic (fp32 MFMA): 1 <= bits <= 8, D % group == 0, group % pf == 0,
  *   (window - residual) % group == 0, 1 <= sink <= group, residual >= 1.
  */
 int kvdec_sparse_decode_kivi(const void* q, const void* k_res, const void* v_res,
@@ -253,7 +253,7 @@ int kvdec_sparse_decode_kivi_varlen(const void* q, const void* k_res, const void
  *   Other arguments and limits as kvdec_sparse_decode_kivi.  Both dtypes
  *   KVDEC_F16 run exactly kvdec_sparse_decode_kivi / _varlen; both
  *   KVDEC_BF16 with 2- or 4-bit codes in groups of 32 the MFMA kernel under
- *   its limits above; any other pair the generic kernel in fp32 arithmetic
+ *   its limits above; any other pair the generic kernel in fp32 arithmetic (fp32 MFMA)
  *   (one rounding of the output to q_dtype).  No workspace.
  */
 int kvdec_sparse_decode_kivi_typed(const void* q, const void* k_res, const void* v_res,

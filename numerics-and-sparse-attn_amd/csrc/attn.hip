@@ -2423,8 +2423,9 @@ int launch_rows(const AttnCommon& P, const void* k, const void* v, int64_t rows,
 }
 
 // bf16 rows take the MFMA kernels (bound, like fp16's, by the reads of K and
-// V: B=4, L=16411 in 46.7 us with its merge, 5.8 TB/s, against 221.9 us on the
-// generic kernel, whose fp32 dot products keep the matrix cores idle) when
+// V: B=4, L=16411 in 45.5 us with its merge, 5.9 TB/s, against 93.1 us on the
+// generic kernel, which
+// widens every value to fp32 for the sixteenth of the matrix rate) when
 // every tensor allows their 16-byte accesses; a tensor that starts at another
 // 2-byte boundary takes the generic kernel.
 bool aligned16(const void* a, const void* b, const void* c, const void* d) {
@@ -2619,10 +2620,10 @@ bool valid_attn_dtype(int dtype) { return dtype == KVDEC_F16 || dtype == KVDEC_F
 // rows (one type for both) take the wide kernel, whatever the window, for query
 // groups of at most kPackGroup heads, a residual of at most 128 rows and a sink
 // of at most 16 tokens, when every tensor allows its 16-byte accesses and
-// 31-bit offsets.  Measured per step in a graph against the generic kernel
-// (bound by its scalar dequantization and fp32 dot products, 11 us for every 64
-// slots): B=8, W=1024, 4-bit bf16 205 -> 13.3 us, 2-bit bf16 12.3; W=128
-// 31 -> 7.6; B=32, W=2944 31.9 (2-bit fp16: 29.1).  At 8 bits an inf zero
+// 31-bit offsets.  Measured per step in a graph: B=8, W=1024, 4-bit bf16
+// 13.3 us, 2-bit bf16 12.3; W=128 7.6; B=32, W=2944 31.9 (2-bit fp16: 29.1);
+// the generic kernel dequantizes value by value into fp32 products (4 bits, B=8,
+// W=1024: 51.2 us).  At 8 bits an inf zero
 // point, which those caches can hold, would turn an infinite key into NaN, so
 // they stay there.
 template <int BITS, int E>
