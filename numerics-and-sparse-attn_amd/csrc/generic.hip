@@ -180,9 +180,12 @@ __device__ __forceinline__ void generic_tile(K&& k, V&& v, uint32_t valid, const
       for (int e = 0; e < 4; ++e) st.O[h][e] *= alpha;
     st.m = mnew;
   }
+  // m = -inf: every logit so far is masked, whose exp2 is 0, or NaN, which has
+  // to reach the output also where a tile holds nothing else.
+  const float m = st.m == -INFINITY ? 0.f : st.m;
 #pragma unroll
   for (int r = 0; r < 4; ++r) {
-    const float p = st.m == -INFINITY ? 0.f : exp2f(x[r] - st.m);
+    const float p = exp2f(x[r] - m);
     st.l += p;
     const bool ok = (valid >> r) & 1u;
 #pragma unroll

@@ -75,6 +75,15 @@ def test_logits_of_any_size(size, device):
     _check(dense_decode_attention(q, k * size, v, 900), _ref(q, k * size, v), "fp32")
 
 
+@pytest.mark.parametrize("L,at", [(17, 16), (900, 0), (5000, 4999)])
+def test_nan_reaches_the_output(L, at, device):
+    """An attended token's NaN, also where its tile holds no other logit."""
+    from dense_kernel import dense_decode_attention
+    q, k, v = _rows((1, 8, 128), "fp32", 1), _rows((1, 1, L, 128), "fp32", 2), _rows((1, 1, L, 128), "fp32", 3)
+    k[:, :, at, 5] = float("nan")
+    assert dense_decode_attention(q, k, v, L).isnan().all()
+
+
 @pytest.mark.parametrize("bits,group", [(8, 1), (8, 2), (5, 4), (8, 32), (4, 2), (3, 4), (4, 64), (2, 4), (1, 8),
                                         (1, 128)])
 @pytest.mark.parametrize("q_dt,res_dt", [("fp16", "fp16"), ("fp32", "bf16")])
