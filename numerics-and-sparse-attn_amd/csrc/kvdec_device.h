@@ -165,7 +165,9 @@ struct WaveState {
   float fs;
 };
 
-constexpr float kMaxSentinel = -1e30f;
+// Near fp32's lowest value: bf16 rows reach logits far below -1e30, whose
+// probabilities against a higher start would all be 0.
+constexpr float kMaxSentinel = -3e38f;
 // The reference max is refreshed only when a tile's max exceeds it by more
 // than this (log2 units), so probabilities stay <= 2^8: exact range for the
 // fp16 P operand, and most tiles skip the cross-lane max and the O rescale.

@@ -97,3 +97,17 @@ def test_dominant_token(device):
     say("dense bf16 dominant token")
     o = dense_decode_attention(q.to(device), k.to(device), v.to(device), seq_len=L)
     _check(o, O.dense_attention(q.float().numpy(), k.float().numpy(), v.float().numpy(), SCALE))
+
+
+@pytest.mark.parametrize("L", [20, 600, 9000])
+def test_logits_far_below_zero(L, device):
+    """Every logit near -1e33: still weights that sum to 1."""
+    from dense_kernel import dense_decode_attention
+    q = torch.full((1, 16, 128), 1e16, dtype=torch.bfloat16)
+    k = torch.full((1, 2, L, 128), -1e15, dtype=torch.bfloat16)
+    v = _bf16((1, 2, L, 128), 16)
+    say(f"dense bf16 low logits L={L}")
+    o = dense_decode_attention(q.to(device), k.to(device), v.to(device), seq_len=L)
+    # equal logits: the mean of V
+    want = v.double().mean(2, keepdim=True).expand(1, 2, 8, 128).reshape(1, 16, 128).numpy()
+    _check(o, want)
