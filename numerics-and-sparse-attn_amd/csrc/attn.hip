@@ -83,6 +83,10 @@ struct AttnCommon {
   int64_t pairs;
   int32_t H, KVH, G;
   int32_t n_tiles, tiles_per_split, n_splits;
+  // Splits shared out by the sequences' own lengths (share_splits), or null.
+  const int32_t* lens;
+  int32_t max_len;
+  int32_t share_limit, share_max;   // splits per KV head in all, tiles of the largest share
   float scale_log2;
   SlotRanges R;
   KVDEC_CLOCK_FIELD
@@ -363,10 +367,56 @@ __device__ __forceinline__ void publish_q(const QState& qs, char* slot, int lane
     for (int r = 0; r < 4; ++r) *reinterpret_cast<float2v*>(slot + off[grp][r]) = v[grp][r];
 }
 
+// Sequences of different lengths.  One workgroup fits a CU, and with every
+// sequence cut into the same n_splits the time is that of the longest one's
+// share while the others' CUs idle: the paged decode of B=16, KVH=8, lengths
+// 1024..16384 took 118.4 us for 570 MB.  The splits per KV head (share_limit
+// in all) go to the sequences by length instead: every wave finds, from the
+// lengths alone, the least t (of 64 values up to share_max, one a lane) for
+// which shares of t tiles are no more than that: 107.3 us, and 80.5 instead of
+// 110.8 with all lengths at their mean (plan_shares has the rule).  (More and smaller splits, 4 to 16
+// workgroups a CU in turn, cost each its start: 127 to 148 us there.)
+// Lane b: the splits of sequence b and those before it; at most 64 sequences
+// and 2^20 tiles (quotients in fp32).
+struct Shares {
+  int splits, first;
+};
+constexpr int kShareSeqs = 64;
+constexpr int kShareTiles = 1 << 20;
+__device__ __forceinline__ int ceil_quot(int n, int t, float rt) {   // n + t < 2^21
+  return max((int)(((float)(n + t - 1) + 0.5f) * rt), 1);
+}
+__device__ __forceinline__ Shares share_splits(const AttnCommon& P, int lane) {
+  const int B = (int)(P.pairs / P.KVH), limit = P.share_limit;
+  int n = 0;
+  if (lane < B) n = (min(max(P.lens[lane], 0), P.max_len) + kTile - 1) / kTile;
+  int sum = n;
+#pragma unroll
+  for (int off = 32; off >= 1; off >>= 1) sum += __shfl_xor(sum, off);
+  const int hi = P.share_max, lo = min(max(sum / limit, 1), hi);
+  const int t = lo + (hi - lo) * lane / (kShareSeqs - 1);
+  const float rt = 1.0f / (float)t;
+  int need = 0;
+  for (int b = 0; b < B; ++b) need += ceil_quot(__builtin_amdgcn_readlane(n, b), t, rt);
+  // the last lane's t = hi always suffices (plan_shares)
+  const int best = min((int)__builtin_ctzll(__ballot(need <= limit) | (1ull << 63)), 63);
+  const int tb = __builtin_amdgcn_readlane(t, best);
+  Shares s;
+  s.splits = lane < B ? ceil_quot(n, tb, 1.0f / (float)tb) : 0;
+  int upto = s.splits;
+#pragma unroll
+  for (int off = 1; off < 64; off <<= 1) {
+    const int y = __shfl_up(upto, off);
+    if (lane >= off) upto += y;
+  }
+  s.first = upto - s.splits;
+  return s;
+}
+
 // Barrier, then combine the waves' published partials into the output (one
-// split) or the split's fp32 partial.
+// split) or the split's fp32 partial (`unit` of pairs * n_splits).
 template <int E>
-__device__ __forceinline__ void merge_out(const AttnCommon& P, char* lds, int64_t pair, int split) {
+__device__ __forceinline__ void merge_out(const AttnCommon& P, char* lds, int64_t pair, size_t unit) {
   __syncthreads();
   const float* sh_m = reinterpret_cast<const float*>(lds + kLdsM);
   const float* sh_l = reinterpret_cast<const float*>(lds + kLdsL);
@@ -401,7 +451,7 @@ __device__ __forceinline__ void merge_out(const AttnCommon& P, char* lds, int64_
     const float inv = L > 0.f ? 1.0f / L : 0.f;   // L == 0: a sequence of length 0
     store_out4<E>(P.o + ((size_t)b * P.H + (size_t)kvh * P.G + hn) * kHeadDim + 4 * ch, acc * inv);
   } else {
-    const size_t idx = ((size_t)pair * P.n_splits + split) * P.G + hn;
+    const size_t idx = unit * P.G + hn;
     *reinterpret_cast<float4v*>(P.ws + idx * kHeadDim + 4 * ch) = acc;
     if (ch == 0) {
       P.ws[total * kHeadDim + idx] = M;
@@ -904,6 +954,12 @@ struct src_elt<Src, decltype((void)Src::kElt)> {
   static constexpr int value = Src::kElt;
 };
 
+// Sources with per-sequence lengths of a whole context.
+template <class Src>
+struct has_lens : std::false_type {};
+template <int E>
+struct has_lens<PagedSrc<E>> : std::true_type {};
+
 template <class Src>
 __global__ __launch_bounds__(kThreads, 1) void attn_kernel(AttnCommon P, Src S) {
   extern __shared__ __align__(16) char lds[];
@@ -923,8 +979,23 @@ __global__ __launch_bounds__(kThreads, 1) void attn_kernel(AttnCommon P, Src S) 
   }
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int split = (int)(blockIdx.x % (unsigned)P.n_splits);
-  const int64_t pair = blockIdx.x / (unsigned)P.n_splits;
+  int split = (int)(blockIdx.x % (unsigned)P.n_splits);
+  int64_t pair = blockIdx.x / (unsigned)P.n_splits;
+  if constexpr (has_lens<Src>::value) {
+    if (P.lens) {
+      const Shares s = share_splits(P, lane);
+      const int B = (int)(P.pairs / P.KVH), u = (int)blockIdx.x;
+      // the last sequence whose units begin at or before u
+      const int bu = __builtin_popcountll(__ballot(lane < B && s.first * P.KVH <= u)) - 1;
+      const int n = __builtin_amdgcn_readlane(s.splits, bu);
+      const int r = u - __builtin_amdgcn_readlane(s.first, bu) * P.KVH;
+      if (r >= n * P.KVH) return;   // past the last sequence's
+      pair = (int64_t)bu * P.KVH + r / n;
+      split = r % n;
+      const int len = min(max(((cint32*)P.lens)[bu], 0), P.max_len);
+      P.tiles_per_split = ((len + kTile - 1) / kTile + n - 1) / n;
+    }
+  }
   const int64_t b = pair / P.KVH;
   const int kvh = (int)(pair % P.KVH);
 
@@ -974,7 +1045,7 @@ __global__ __launch_bounds__(kThreads, 1) void attn_kernel(AttnCommon P, Src S) 
   WaveState st;
   wave_state_init(st);
   S.process(pair, split, P, wave, lane, ctr, sync, st);
-  merge_out<src_elt<Src>::value>(P, lds, pair, split);
+  merge_out<src_elt<Src>::value>(P, lds, pair, blockIdx.x);
   if constexpr (has_arrive<Src>::value) S.arrive(pair, P);
 }
 
@@ -2198,9 +2269,17 @@ __global__ __launch_bounds__(64 * kMergeWaves) void merge_kernel(AttnCommon P) {
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const uint32_t row = blockIdx.x, pair = row / (uint32_t)P.G;   // row = pair * G + head of the group
-  const int hn = (int)(row - pair * (uint32_t)P.G), S = P.n_splits;
+  const int hn = (int)(row - pair * (uint32_t)P.G);
+  int S = P.n_splits;
   const size_t total = (size_t)P.pairs * S * P.G;
-  const size_t base = (size_t)pair * S * P.G + hn;               // split s: base + s * G
+  size_t unit = (size_t)pair * S;
+  if (P.lens) {
+    const Shares sh = share_splits(P, lane);
+    const int b = __builtin_amdgcn_readfirstlane((int)(pair / (uint32_t)P.KVH));
+    S = __builtin_amdgcn_readlane(sh.splits, b);
+    unit = (size_t)__builtin_amdgcn_readlane(sh.first, b) * P.KVH + (size_t)(pair - (uint32_t)(b * P.KVH)) * S;
+  }
+  const size_t base = unit * P.G + hn;                           // split s: base + s * G
   const float* wo = P.ws + 2 * lane;
   const float* wm = P.ws + total * kHeadDim;
   const float* wl = wm + total;
@@ -2352,6 +2431,23 @@ int launch_merge(const AttnCommon& P, hipStream_t stream) {
   return launch_status();
 }
 
+// Whether P's splits are shared out by length.  A wave's search and the
+// merge's take 2 to 3 us, which equal splits of 64 tiles (30 us) outweigh:
+// B=16, KVH=8, L=4000 (63 tiles) 35.1 -> 34.4 us, L=2000 (32) 21.7 -> 23.5.
+// One round of workgroups where it holds two splits a sequence (a few
+// workgroups more than the CUs cost a second round: B=5, L=30000, 280 of them,
+// 70.2 -> 81.8, and 67.6 in one round), else the plan's two rounds (B=30, L=20000: 283.4 -> 220.2).
+constexpr int kShareMinTiles = 64;
+void plan_shares(AttnCommon& P) {
+  const int64_t B = P.pairs / P.KVH, round = kTargetUnits / P.KVH;
+  if (B < 2 || B > kShareSeqs || P.n_splits == 1 || P.n_tiles > kShareTiles || P.tiles_per_split < kShareMinTiles)
+    P.lens = nullptr;
+  if (!P.lens) return;
+  P.share_limit = (int)(round >= 2 * B ? std::min(round, B * P.n_splits) : B * P.n_splits);
+  const int64_t each = P.share_limit / B;   // every sequence may take this many
+  P.share_max = (int)((P.n_tiles + each - 1) / each);
+}
+
 template <class Src>
 int launch_attn(AttnCommon P, const Src& S, bool kivi, size_t ws_bytes, hipStream_t stream) {
   constexpr int E = src_elt<Src>::value;
@@ -2361,6 +2457,7 @@ int launch_attn(AttnCommon P, const Src& S, bool kivi, size_t ws_bytes, hipStrea
   if (E == kEltBf16) plan = fit_plan(plan, P.pairs, P.n_tiles, P.G, P.ws, ws_bytes);
   P.n_splits = plan.splits;
   P.tiles_per_split = plan.tps;
+  plan_shares(P);
   if (plan.splits > 1) {
     if (P.ws == nullptr) return KVDEC_E_WORKSPACE;
     if (ws_bytes < ws_bytes_for(P.pairs, plan.splits, P.G)) return KVDEC_E_WORKSPACE;
@@ -3167,6 +3264,8 @@ int kvdec_paged_decode(const void* q, const void* k_pages, const void* v_pages,
   S.max_len = (int)max_seq_len;
   S.rows = (int)max_seq_len;
   S.sparse = false;
+  P.lens = seq_lens;
+  P.max_len = S.max_len;
   return launch_attn(P, S, false, ws_bytes, static_cast<hipStream_t>(stream));
 }
 
