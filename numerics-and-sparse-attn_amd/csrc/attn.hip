@@ -2068,9 +2068,9 @@ __global__ __launch_bounds__(Wide<BITS>::kThreads, 1) void kivi_wide_kernel(Kivi
   }
   // the quantized items' Q operand, prescaled once the wave's first group
   // load is in flight (before it, the wait for Q would hold the load back)
-  float sl2;
+  float sl2;   // (kNorm: the lane's head's)
   if constexpr (kNorm)
-    sl2 = scale_pow2(A.c.scale_log2, q_normalize<E>(qB));
+    sl2 = __builtin_ldexpf(A.c.scale_log2, q_normalize<E>(qB));
   else
     sl2 = q_prescale(qB, A.c.scale_log2);
   WaveState st;   // the quantized items' max and sum (st.O stays zero)
@@ -2083,7 +2083,7 @@ __global__ __launch_bounds__(Wide<BITS>::kThreads, 1) void kivi_wide_kernel(Kivi
     if constexpr (kNorm) {
       int k;
       q_tile_stage_n<BITS>(X, slot, lane, slot0, xlim, R, k, v_field, qs);
-      f = scale_pow2(sl2, -k);
+      f = __builtin_ldexpf(sl2, -k);
       return kRescaleSlack;
     } else {
       f = sl2;

@@ -1073,9 +1073,9 @@ __device__ __forceinline__ float q_tile_stage(const QTileRaw& raw, char* slot, i
   return __ballot(!(fmaxf((float)vs[0], (float)vs[1]) <= kSlackVScale)) ? 0.0f : kRescaleSlack;
 }
 
-// The staging of a tile whose Q operand is scaled to less than 1 in magnitude
-// (q_normalize), with powers of two taken out of its scales: K scales come to
-// [2^13, 2^14) at their largest (k_exp: the tile's logits are 2^k_exp too
+// The staging of a tile whose Q operand is scaled to less than 2^15 in
+// magnitude (q_normalize), with powers of two taken out of its scales: K scales
+// come to [2^-1, 1) at their largest (k_exp: the tile's logits are 2^k_exp too
 // large), V scales to at most 2^7 over all of the wave's tiles so far (v_field:
 // the largest exponent field seen; a tile with a larger one rescales the
 // accumulators), so that neither product's exact remainder falls into fp16's
@@ -1104,7 +1104,7 @@ template <int BITS>
 __device__ __forceinline__ void q_tile_stage_n(const QTileRawN<BITS>& X, char* slot, int lane, int slot0, int xlim,
                                                const SlotRanges& R, int& k_exp, int& v_field, QState& qs) {
   typedef QSlot<BITS> Lay;
-  k_exp = 28 - max_field(X.ks);
+  k_exp = 14 - max_field(X.ks);
 #pragma unroll
   for (int i = 0; i < kQPieces<BITS>; ++i) {
     const int krow = 8 * i + (lane >> 3);
@@ -1141,13 +1141,15 @@ __device__ __forceinline__ void q_state_unshift(QState& qs, int v_field) {
   for (int b = 0; b < 8; ++b) qs.O[b] = qs.O[b] * down;
 }
 
-// The Q operand of element type E as fp16, scaled by the power of two 2^-e
-// that brings the KV head's largest |q| below 1; returns e.  bf16's 8 bits
-// fit fp16's 11: exact for every channel within 2^-14 of the largest, the
-// rest off by at most 2^-25 of it.
+// The Q operand of element type E as fp16, each query head scaled by its own
+// power of two 2^-e, which brings that head's largest |q| to [2^14, 2^15);
+// returns the lane's head's e (heads share nothing: one that is far larger than
+// the others, or not finite, must not reach them).  Exact for every channel
+// within 2^-28 of the head's largest (bf16's 8 bits: 2^-31), the rest off by at
+// most 2^-39 of it.
 template <int E>
 __device__ __forceinline__ int q_normalize(half8 (&qB)[4]) {
-  constexpr int kMant = E == kEltBf16 ? 7 : 10, kBias = E == kEltBf16 ? 126 : 14;
+  constexpr int kMant = E == kEltBf16 ? 7 : 10, kBias = E == kEltBf16 ? 141 : 29;
   uint32_t top = 0;
 #pragma unroll
   for (int c = 0; c < 4; ++c)
@@ -1156,9 +1158,10 @@ __device__ __forceinline__ int q_normalize(half8 (&qB)[4]) {
       const uint32_t u = as_u4(qB[c])[i];
       top = max(top, max(u & 0x7FFFu, (u >> 16) & 0x7FFFu));
     }
-#pragma unroll
-  for (int off = 32; off >= 1; off >>= 1) top = max(top, (uint32_t)__shfl_xor((int)top, off));
-  const int e = __builtin_amdgcn_readfirstlane((int)(top >> kMant)) - kBias;
+  // the head's four lanes n, n + 16, n + 32, n + 48 (and n + 8 .. hold copies)
+  top = max(top, (uint32_t)__shfl_xor((int)top, 16));
+  top = max(top, (uint32_t)__shfl_xor((int)top, 32));
+  const int e = (int)(top >> kMant) - kBias;
 #pragma unroll
   for (int c = 0; c < 4; ++c) {
     const u32x4 u = as_u4(qB[c]);

@@ -84,6 +84,44 @@ def test_scales_far_from_one(bits, dt, q_mul, k_mul, v_mul, device):
     assert (np.abs(got - ref) - ulp).max() <= 1e-5 * top + (2.0**-25 if dt == "fp16" else 0.0)
 
 
+@pytest.mark.parametrize("bits,dt", [(4, "fp16"), (4, "bf16"), (2, "bf16")])
+@pytest.mark.parametrize("odd", ["x2^14", "x2^-14", "nan", "inf", "-inf"])
+def test_heads_stand_alone(bits, dt, odd, device):
+    """One query head far from the size of the others of its KV head, or with
+    one element that is not finite: the others' results do not change by it."""
+    B, H, KVH, S, W, R = 1, 16, 2, 4, 448, 128
+    hc = _cache(B, KVH, S, W, R, bits, dt, 55)
+    q = torch.from_numpy(randn((B, H, 128), 9))
+    q[:, 2] *= {"x2^14": 2.0**14, "x2^-14": 2.0**-14}.get(odd, 1.0)
+    q = q.to(DT[dt])
+    ref = O.quantized_attention_masked(q.float().numpy(), hc, 163840, W, SCALE, sink=S, residual_size=R, bits=bits)
+    if odd[0] != "x":
+        q[:, 2, 40] = float(odd)
+    say(f"kivi bits={bits} {dt} head 2 {odd}")
+    o = _attend(q.to(device), _upload(hc, dt, device), 163840, W, S, R, bits)
+    rest = [h for h in range(H) if h != 2]
+    _check(o[:, rest], ref[:, rest], dt)
+
+
+@pytest.mark.parametrize("bits", [2, 4])
+def test_channels_far_apart(bits, device):
+    """Query channels 2^-20 the size of the head's largest, against keys 2^10
+    times the others': the small ones keep all their bits."""
+    B, H, KVH, S, W, R = 1, 16, 2, 4, 448, 128
+    small = torch.arange(128) % 2 == 0
+    kc, vc = (torch.from_numpy(randn((B, KVH, S + W, 128), n)) for n in (61, 62))
+    kc = torch.where(small, kc * 2.0**10, kc).to(torch.bfloat16)
+    vc = vc.to(torch.bfloat16)
+    q = torch.from_numpy(randn((B, H, 128), 63)) * 8
+    q = torch.where(small, q * 2.0**-20, q).to(torch.bfloat16)
+    hc = O.build_quantized_kv_cache(kc.float().numpy(), vc.float().numpy(), residual_size=R, sink=S, bits=bits)
+    hc["k_residual"], hc["v_residual"] = (x[:, :, -R:].float().numpy() for x in (kc, vc))
+    ref = O.quantized_attention_masked(q.float().numpy(), hc, 163840, W, SCALE, sink=S, residual_size=R, bits=bits)
+    say(f"kivi bits={bits} channels far apart")
+    o = _attend(q.to(device), _upload(hc, "bf16", device), 163840, W, S, R, bits)
+    _check(o, ref, "bf16")
+
+
 @pytest.mark.parametrize("bits,dt", [(4, "fp16"), (2, "bf16")])
 def test_slots_never_written(bits, dt, device):
     """NaN patterns in every quantized byte and residual row of slots past the
