@@ -413,6 +413,74 @@ __device__ __forceinline__ Shares share_splits(const AttnCommon& P, int lane) {
   return s;
 }
 
+// ---------------------------------------------------------------------------
+// Results that are not a number.  An fp32 product taken as a sum of 16-bit
+// parts is NaN where a factor is infinite (inf * 0, or inf - inf between
+// parts), and so is scale * code - scale * zero; scale * (code - zero), the
+// probabilities and V in fp32 have a value: an infinite zero point (a nearly
+// constant channel far from 0, quantized from fp32 or bf16) gives a key of
+// -inf, weight 0 under a positive query.  The merge therefore computes a NaN
+// result once more, from the cache in fp32 as the generic kernel does, slot by
+// slot: the half wave that holds a query head's output (lane c of 32: channels
+// 4c .. 4c + 3) steps all of its workgroup's slots.  Finite calls pay one
+// comparison of the merged values.
+// ---------------------------------------------------------------------------
+struct PlainState {
+  float m = kMaxSentinel, l = 0.f;
+  float4v o = {0.f, 0.f, 0.f, 0.f};
+};
+__device__ __forceinline__ bool any_nan(float l, float4v o) {
+  return __any(!(l == l) || !(o[0] == o[0]) || !(o[1] == o[1]) || !(o[2] == o[2]) || !(o[3] == o[3]));
+}
+
+// Four adjacent values of element type E (8-byte aligned) as floats.
+template <int E>
+__device__ __forceinline__ float4v row4(const _Float16* p) {
+  const u32x2 u = *reinterpret_cast<const u32x2*>(p);
+  if constexpr (E == kEltBf16) {
+    return float4v{__builtin_bit_cast(float, u[0] << 16), __builtin_bit_cast(float, u[0] & 0xFFFF0000u),
+                   __builtin_bit_cast(float, u[1] << 16), __builtin_bit_cast(float, u[1] & 0xFFFF0000u)};
+  } else {
+    const half4v h = __builtin_bit_cast(half4v, u);
+    return float4v{(float)h[0], (float)h[1], (float)h[2], (float)h[3]};
+  }
+}
+
+// x of lane L ^ N, N < 32 (no lane address to keep in a register).
+template <int N>
+__device__ __forceinline__ float swap_lane(float x) {
+  return __builtin_bit_cast(float, __builtin_amdgcn_ds_swizzle(__builtin_bit_cast(int, x), N << 10 | 0x1f));
+}
+
+// Slots lo .. hi - 1, four in flight; fetch(slot, k, v) reads the lane's
+// channels of one slot in [lo, hi).
+template <class Fetch>
+__device__ __forceinline__ void plain_slots(Fetch&& fetch, int lo, int hi, const SlotRanges& R, float4v q,
+                                            float scale_log2, PlainState& st) {
+  constexpr int kIn = 4;
+  for (int s0 = lo; s0 < hi; s0 += kIn) {
+    float4v k[kIn], v[kIn];
+#pragma unroll
+    for (int j = 0; j < kIn; ++j) fetch(min(s0 + j, hi - 1), k[j], v[j]);
+#pragma unroll
+    for (int j = 0; j < kIn; ++j) {
+      const bool ok = s0 + j < hi && slot_valid(R, s0 + j);
+      float d = fmaf(q[3], k[j][3], fmaf(q[2], k[j][2], fmaf(q[1], k[j][1], q[0] * k[j][0])));
+      d += swap_lane<16>(d);
+      d += swap_lane<8>(d);
+      d += swap_lane<4>(d);
+      d += swap_lane<2>(d);
+      d += swap_lane<1>(d);
+      const float x = ok ? d * scale_log2 : -INFINITY, m = fmaxf(st.m, x);
+      const float alpha = exp2f(st.m - m), p = exp2f(x - m);
+      st.l = fmaf(st.l, alpha, p);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) st.o[e] = fmaf(p, ok ? v[j][e] : 0.f, st.o[e] * alpha);
+      st.m = m;
+    }
+  }
+}
+
 // Barrier, then combine the waves' published partials into the output (one
 // split) or the split's fp32 partial (`unit` of pairs * n_splits).
 template <int E>
@@ -1998,6 +2066,90 @@ struct KiviWideArgs : KiviLeanArgs {
   int32_t KVH, window;
 };
 
+// A workgroup's KV head, its items (window-old groups g0 .. g1 - 1, then
+// (`tail`: the head's last split) the sink group as item g1 and the residual)
+// and the head's valid slots.
+template <bool SPLIT>
+__device__ __forceinline__ uint32_t wide_head(const KiviWideArgs& A) {
+  return SPLIT ? blockIdx.x / (uint32_t)A.n_splits : blockIdx.x;
+}
+struct WideShare {
+  SlotRanges R;
+  int g0, g1;
+  bool tail;
+};
+template <bool SPLIT, bool VAR>
+__device__ __forceinline__ WideShare wide_share(const KiviWideArgs& A, uint32_t head) {
+  const int split = SPLIT ? (int)(blockIdx.x - head * (uint32_t)A.n_splits) : 0, nwt = A.nwt;
+  WideShare w;
+  w.R = A.c.R;
+  int first = A.first;
+  if constexpr (VAR) {
+    const int len = max((int)((cint32*)A.lens)[head / (uint32_t)A.KVH], 0);
+    w.R = sparse_ranges(len, A.window, A.sink, KVDEC_LAYOUT_LINEAR);
+    first = min((w.R.vb - A.sink) / kTile, nwt);
+  }
+  w.g1 = SPLIT ? min((split + 1) * A.per_split + A.first, nwt) : nwt;
+  w.g0 = SPLIT ? min(max(split * A.per_split + A.first, first), w.g1) : first;
+  w.tail = !SPLIT || split == A.n_splits - 1;
+  return w;
+}
+
+// K and V of slot s of KV head `head`, channels 4 ch .. 4 ch + 3, in fp32.
+template <int BITS, int E>
+__device__ __forceinline__ void kivi_slot4(const KiviWideArgs& A, uint32_t head, int s, int ch, float4v& k,
+                                           float4v& v) {
+  constexpr int kPf = 8 / BITS;
+  const int win = kTile * A.nwt;
+  if (s >= A.sink + win) {
+    const size_t at = ((size_t)head * A.res_rows + (s - A.sink - win)) * kHeadDim + 4 * ch;
+    k = row4<E>(A.kres + at);
+    v = row4<E>(A.vres + at);
+    return;
+  }
+  const bool sk = s < A.sink;
+  const QRegion Q = sk ? A.sinkq : A.winq;
+  const int t = sk ? s : s - A.sink;                             // token of the region
+  const size_t tok = (size_t)head * (sk ? kTile : win) + t;      // over all heads
+  const uint32_t kc = *reinterpret_cast<const uint32_t*>(Q.kp + tok / kPf * kHeadDim + 4 * ch) >> (t % kPf * BITS);
+  const uint8_t* vp = Q.vp + tok * (kHeadDim / kPf) + 4 * ch / kPf;
+  const uint32_t vc = BITS == 4 ? *reinterpret_cast<const uint16_t*>(vp) : *vp;
+  const size_t km = tok / kTile * kHeadDim + 4 * ch, vm = tok * (kHeadDim / kTile) + ch / 8;
+  const float4v ks = row4<kEltF16>(Q.ks + km), kz = row4<kEltF16>(Q.kz + km);
+  const float vs = (float)Q.vs[vm], vz = (float)Q.vz[vm];
+  constexpr uint32_t kMask = (1u << BITS) - 1u;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    k[e] = ks[e] * ((float)((kc >> (8 * e)) & kMask) - kz[e]);
+    v[e] = vs * ((float)((vc >> (BITS * e)) & kMask) - vz);
+  }
+}
+
+// The workgroup's slots for query head hn in plain fp32 (plain_slots).  The
+// kernel's arguments are read again, through a pointer the compiler cannot see
+// through: kept from the kernel's start, they would spill its registers.
+template <bool SPLIT, bool VAR, int BITS, int E>
+__device__ __forceinline__ PlainState wide_plain(int hn, int ch) {
+  typedef __attribute__((address_space(4))) const KiviWideArgs Args;
+  Args* ka = (Args*)__builtin_amdgcn_kernarg_segment_ptr();
+  asm volatile("" : "+s"(ka));
+  KiviWideArgs A;
+  __builtin_memcpy(&A, (const void*)ka, sizeof A);
+  const uint32_t head = wide_head<SPLIT>(A);
+  const WideShare w = wide_share<SPLIT, VAR>(A, head);
+  const float4v q = row4<E>(A.c.q + ((size_t)head * A.c.G + hn) * kHeadDim + 4 * ch);
+  PlainState st;
+  auto step = [&](int lo, int hi) {
+    plain_slots([&](int s, float4v& k, float4v& v) { kivi_slot4<BITS, E>(A, head, s, ch, k, v); }, lo, hi, w.R, q,
+                A.c.scale_log2, st);
+  };
+  const int res0 = A.sink + kTile * A.nwt;
+  step(A.sink + kTile * w.g0, A.sink + kTile * w.g1);
+  if (w.tail) step(res0, res0 + A.res_rows);
+  if (w.tail) step(0, A.sink);
+  return st;
+}
+
 template <bool SPLIT, bool VAR, int BITS = 2, int E = kEltF16>
 __global__ __launch_bounds__(Wide<BITS>::kThreads, 1) void kivi_wide_kernel(KiviWideArgs A) {
   extern __shared__ __align__(16) char lds[];
@@ -2010,25 +2162,16 @@ __global__ __launch_bounds__(Wide<BITS>::kThreads, 1) void kivi_wide_kernel(Kivi
   typedef typename std::conditional<kNorm, QTileRawN<BITS>, QTileRaw>::type Raw;
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const uint32_t head = SPLIT ? blockIdx.x / (uint32_t)A.n_splits : blockIdx.x;
-  const uint32_t split = SPLIT ? blockIdx.x - head * (uint32_t)A.n_splits : 0u;
+  const uint32_t head = wide_head<SPLIT>(A);
   half8 qB[4];
   lean_prologue<KiviWideArgs, PACK>(A.c, head, lane, qB);
   char* slot = lds + Wd::kSlots + wave * kSlotBytes;
   int* ctr = reinterpret_cast<int*>(lds + Wd::kCtr);
   const int nwt = A.nwt;
-  SlotRanges R = A.c.R;
-  int first = A.first;
-  if constexpr (VAR) {
-    const int len = max((int)((cint32*)A.lens)[head / (uint32_t)A.KVH], 0);
-    R = sparse_ranges(len, A.window, A.sink, KVDEC_LAYOUT_LINEAR);
-    first = min((R.vb - A.sink) / kTile, nwt);
-  }
-  // this workgroup's items: window-old groups g0 .. g1 - 1, then (`tail`:
-  // the head's last split) the sink group as item g1
-  const int g1 = SPLIT ? min((int)(split + 1) * A.per_split + A.first, nwt) : nwt;
-  const int g0 = SPLIT ? min(max((int)split * A.per_split + A.first, first), g1) : first;
-  const bool tail = !SPLIT || (int)split == A.n_splits - 1;
+  const WideShare share = wide_share<SPLIT, VAR>(A, head);
+  const SlotRanges R = share.R;
+  const int g0 = share.g0, g1 = share.g1;
+  const bool tail = share.tail;
   const int n_q = tail ? g1 + 1 : g1;
   const QTensors Tw = q_tensors(A.winq, A.win_code_bytes, A.win_meta_bytes);
   const QTensors Ts = q_sink_tensors<BITS>(A.sinkq, head, A.sink);
@@ -2110,8 +2253,8 @@ __global__ __launch_bounds__(Wide<BITS>::kThreads, 1) void kivi_wide_kernel(Kivi
   if constexpr (kNorm) q_state_unshift(qs, v_field);
   publish_q<false, PACK, BITS>(qs, slot, lane);
 
-  // merge: one thread per (head, 4 channels) over the 16 quantized partials
-  // (remainders already folded in) and the 4 fp16 partials
+  // merge: one thread per (head, 4 channels) over the waves' quantized partials
+  // (remainders already folded in) and the 4 residual ones
   __syncthreads();
   const int e = threadIdx.x;
   if (e >= A.c.G * 32) return;
@@ -2145,6 +2288,14 @@ __global__ __launch_bounds__(Wide<BITS>::kThreads, 1) void kivi_wide_kernel(Kivi
       const float f = __builtin_amdgcn_exp2f(mw[p] - M);
       L += lw[j] * f;
       acc += ow[j] * f;
+    }
+  }
+  if constexpr (kNorm) {
+    if (any_nan(L, acc)) {
+      const PlainState ps = wide_plain<SPLIT, VAR, BITS, E>(hn, ch);
+      M = ps.m;
+      L = ps.l;
+      acc = ps.o;
     }
   }
   if constexpr (SPLIT) {
@@ -2720,9 +2871,10 @@ bool valid_attn_dtype(int dtype) { return dtype == KVDEC_F16 || dtype == KVDEC_F
 // 31-bit offsets.  Measured per step in a graph: B=8, W=1024, 4-bit bf16
 // 13.3 us, 2-bit bf16 12.3; W=128 7.6; B=32, W=2944 31.9 (2-bit fp16: 29.1);
 // the generic kernel dequantizes value by value into fp32 products (4 bits, B=8,
-// W=1024: 51.2 us).  At 8 bits an inf zero
-// point, which those caches can hold, would turn an infinite key into NaN, so
-// they stay there.
+// W=1024: 51.2 us).  Other widths stay there: their codes are not the exact
+// fp8 values that codes_f16 widens.  What the factored products cannot give
+// (infinite zero points and scales, which caches of any width can hold) the
+// kernel's merge computes again in fp32 (wide_plain).
 template <int BITS, int E>
 int kivi_decode_wide(const void* q, const void* k_res, const void* v_res, const void* const* kivi, void* o,
                      const int32_t* lens, int64_t B, int32_t H, int32_t KVH, int64_t seq_len, int32_t window,

@@ -1159,9 +1159,7 @@ __device__ __forceinline__ int q_normalize(half8 (&qB)[4]) {
       top = max(top, max(u & 0x7FFFu, (u >> 16) & 0x7FFFu));
     }
   // the head's four lanes n, n + 16, n + 32, n + 48 (and n + 8 .. hold copies)
-  top = max(top, (uint32_t)__shfl_xor((int)top, 16));
-  top = max(top, (uint32_t)__shfl_xor((int)top, 32));
-  const int e = (int)(top >> kMant) - kBias;
+  const int e = (int)((uint32_t)group_max((float)top) >> kMant) - kBias;
 #pragma unroll
   for (int c = 0; c < 4; ++c) {
     const u32x4 u = as_u4(qB[c]);

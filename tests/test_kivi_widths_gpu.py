@@ -101,6 +101,52 @@ def test_heads_stand_alone(bits, dt, odd, device):
     o = _attend(q.to(device), _upload(hc, dt, device), 163840, W, S, R, bits)
     rest = [h for h in range(H) if h != 2]
     _check(o[:, rest], ref[:, rest], dt)
+    if odd == "nan":
+        assert o[:, 2].isnan().all()
+
+
+def _same(o, ref, dt):
+    """_check where the oracle is finite, the same infinities where not."""
+    got, fin = o.double().cpu().numpy(), np.isfinite(ref)
+    assert np.array_equal(got[~fin], ref[~fin])
+    _check(torch.where(torch.from_numpy(fin).to(o.device), o, torch.zeros_like(o)), np.where(fin, ref, 0.0), dt)
+
+
+@pytest.mark.parametrize("bits,dt", [(4, "fp16"), (4, "bf16"), (2, "bf16")])
+@pytest.mark.parametrize("what", ["k_zero", "k_scale", "v_zero", "v_scale", "v_residual"])
+def test_infinities_in_the_cache(bits, dt, what, device):
+    """A nearly constant channel far from 0 has an infinite zero point once
+    quantized: its 32 keys are -inf, weight 0 under a positive query.  Infinite
+    scales, V zero points and V rows likewise give scale * (code - zero)."""
+    B, H, KVH, S, W, R = 2, 16, 2, 4, 448, 128
+    kc, vc = randn((B, KVH, S + W, 128), 71), randn((B, KVH, S + W, 128), 72)
+    if what == "k_zero":
+        kc[:, :, S + 32:S + 64, 40] = -20000 + 0.05 * randn((B, KVH, 32), 73)
+    hc = O.build_quantized_kv_cache(kc, vc, residual_size=R, sink=S, bits=bits)
+    hc["k_residual"], hc["v_residual"] = (
+        torch.from_numpy(x[:, :, -R:]).to(DT[dt]).float().numpy() for x in (kc, vc))
+    if what == "k_zero":
+        assert (hc["k_win_zero"][:, :, 1, 40] == np.inf).all()
+    elif what == "k_scale":
+        hc["k_win_scale"][:, :, 1, 40], hc["k_win_zero"][:, :, 1, 40] = np.inf, 20
+    elif what == "v_zero":
+        hc["v_win_zero"][:, :, 37, 2] = np.inf
+    elif what == "v_scale":
+        hc["v_win_scale"][:, :, 37, 2], hc["v_win_zero"][:, :, 37, 2] = np.inf, -1
+    else:
+        hc["v_residual"][:, :, 3, 7] = np.inf
+    q = torch.from_numpy(randn((B, H, 128), 74))
+    q[..., 40] = q[..., 40].abs() + 0.1
+    q = q.to(DT[dt])
+    c = _upload(hc, dt, device)
+    say(f"kivi bits={bits} {dt} infinite {what}")
+    for L in (163840, S + W - 20):
+        ref = O.quantized_attention_masked(q.float().numpy(), hc, L, W, SCALE, sink=S, residual_size=R, bits=bits)
+        assert not np.isnan(ref).any() and np.isinf(ref).any() == (what[0] == "v")
+        _same(_attend(q.to(device), c, L, W, S, R, bits), ref, dt)
+    lens = np.array([S + W - 20, 90000], dtype=np.int32)
+    ref = O.quantized_attention_varlen(q.float().numpy(), hc, lens, W, SCALE, sink=S, residual_size=R, bits=bits)
+    _same(_attend(q.to(device), c, dev(lens, device), W, S, R, bits), ref, dt)
 
 
 @pytest.mark.parametrize("bits", [2, 4])
