@@ -2443,7 +2443,7 @@ __global__ __launch_bounds__(64 * kMergeWaves) void merge_kernel(AttnCommon P) {
       const int s = s0 + kMergeWaves * j;
       const size_t u = base + (size_t)(s < S ? s : 0) * P.G;
       a[j] = *reinterpret_cast<const float2v*>(wo + u * kHeadDim);
-      ms[j] = s < S ? wm[u] : -INFINITY;
+      ms[j] = wm[u];
       ls[j] = wl[u];
     }
   };
@@ -2458,7 +2458,8 @@ __global__ __launch_bounds__(64 * kMergeWaves) void merge_kernel(AttnCommon P) {
     if (s0 != wave) fetch(s0);
 #pragma unroll
     for (int j = 0; j < kIn; ++j) {
-      const float f = __builtin_amdgcn_exp2f(ms[j] - M);   // 0 past the last split
+      if (s0 + kMergeWaves * j >= S) break;   // past the last split (wave-uniform)
+      const float f = __builtin_amdgcn_exp2f(ms[j] - M);
       L += ls[j] * f;
       acc += a[j] * f;
     }

@@ -68,3 +68,26 @@ def test_any_workspace(held, device):
     assert rc == 0
     assert_nearly_rounded(host(o), O.quantized_attention_masked(q, hc, 163840, W, SCALE, sink=S))
     assert bool((ws[nbytes // 4:] == 7.0).all())
+
+
+@pytest.mark.parametrize("token", [0, 700, 1279])
+def test_infinite_partials(token, device):
+    """An infinite V row in the first, a middle and the last window-old split
+    of a 4-bit call reaches its channels as that infinity, and no others."""
+    import _kvdec as K
+    from quant_kernel import sparse_decode_attention_quantized
+    B, H, KVH, S, R, bits = 1, 8, 1, 4, 128, 4
+    W = R + 32 * 40
+    assert K.lib.kvdec_num_splits(K.KIND_KIVI_SPLIT, B, KVH, W - R) == 5
+    kc, vc, q = randn((B, KVH, S + W, 128), 81), randn((B, KVH, S + W, 128), 82), randn((B, H, 128), 83)
+    hc = O.build_quantized_kv_cache(kc, vc, residual_size=R, sink=S, bits=bits)
+    hc = {k: v.astype(np.float16) if k.endswith("residual") else v for k, v in hc.items()}
+    hc["v_win_zero"][:, :, token, 1] = np.inf
+    q = q.astype(np.float16)
+    say(f"kivi 4-bit split, infinite V of token {token}")
+    o = host(sparse_decode_attention_quantized(dev(q, device), *[dev(hc[k], device) for k in O.CACHE_KEYS],
+                                               seq_len=163840, window=W, sink=S, bits=bits))
+    ref = O.quantized_attention_masked(q, hc, 163840, W, SCALE, sink=S, bits=bits)
+    assert (ref[..., 32:64] == -np.inf).all() and (o[..., 32:64] == -np.inf).all()
+    rest = np.r_[0:32, 64:128]
+    assert_nearly_rounded(o[..., rest], ref[..., rest])
