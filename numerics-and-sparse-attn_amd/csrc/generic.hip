@@ -498,9 +498,9 @@ __global__ __launch_bounds__(64 * kGMergeWaves) void generic_merge_kernel(GArgs 
     acc += part[w][lane];
     L += part_l[w];
   }
-  const float inv = L > 0.f ? 1.0f / L : 0.f;   // row = b * H + head
-  store_o(A.o, A.dt, row * kHeadDim + 2 * lane, acc[0] * inv);
-  store_o(A.o, A.dt, row * kHeadDim + 2 * lane + 1, acc[1] * inv);
+  // row = b * H + head; no valid slot: zeros (L may be NaN)
+  store_o(A.o, A.dt, row * kHeadDim + 2 * lane, L == 0.f ? 0.f : acc[0] / L);
+  store_o(A.o, A.dt, row * kHeadDim + 2 * lane + 1, L == 0.f ? 0.f : acc[1] / L);
 }
 
 int gstatus() {

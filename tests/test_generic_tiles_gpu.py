@@ -84,6 +84,16 @@ def test_nan_reaches_the_output(L, at, device):
     assert dense_decode_attention(q, k, v, L).isnan().all()
 
 
+@pytest.mark.parametrize("L", [4007, 4039, 4331])
+def test_split_sums_are_divided_once(L, device):
+    """Equal logits over rows of ones, split: n / n is 1, n * (1 / n) is not."""
+    from dense_kernel import dense_decode_attention
+    assert np.float32(L) * (np.float32(1) / np.float32(L)) != 1
+    q, v = torch.zeros((1, 16, 128), device=device), torch.ones((1, 2, L, 128), device=device)
+    print(f"fp32 dense of ones L={L}", flush=True)
+    assert (dense_decode_attention(q, v, v, seq_len=L) == 1).all()
+
+
 @pytest.mark.parametrize("bits,group", [(8, 1), (8, 2), (5, 4), (8, 32), (4, 2), (3, 4), (4, 64), (2, 4), (1, 8),
                                         (1, 128)])
 @pytest.mark.parametrize("q_dt,res_dt", [("fp16", "fp16"), ("fp32", "bf16")])
