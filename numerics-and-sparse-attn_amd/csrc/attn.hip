@@ -446,6 +446,18 @@ __device__ __forceinline__ float4v row4(const _Float16* p) {
   }
 }
 
+// The kernel's arguments, read again through a pointer the compiler cannot see
+// through: kept from the kernel's start for a rare path, they would spill.
+template <class Args>
+__device__ __forceinline__ Args kernargs_again() {
+  typedef __attribute__((address_space(4))) const Args CArgs;
+  CArgs* ka = (CArgs*)__builtin_amdgcn_kernarg_segment_ptr();
+  asm volatile("" : "+s"(ka));
+  Args a;
+  __builtin_memcpy(&a, (const void*)ka, sizeof a);
+  return a;
+}
+
 // x of lane L ^ N, N < 32 (no lane address to keep in a register).
 template <int N>
 __device__ __forceinline__ float swap_lane(float x) {
@@ -481,10 +493,25 @@ __device__ __forceinline__ void plain_slots(Fetch&& fetch, int lo, int hi, const
   }
 }
 
+// Slots lo .. hi - 1 of the rows (row_bytes apart) at k and v.
+template <int E>
+__device__ __forceinline__ PlainState plain_rows(const char* k, const char* v, size_t row_bytes, int lo, int hi,
+                                                 const SlotRanges& R, const _Float16* q, int ch, float scale_log2) {
+  PlainState st;
+  auto fetch = [&](int s, float4v& kr, float4v& vr) {
+    const size_t at = (size_t)s * row_bytes + 8 * ch;
+    kr = row4<E>(reinterpret_cast<const _Float16*>(k + at));
+    vr = row4<E>(reinterpret_cast<const _Float16*>(v + at));
+  };
+  plain_slots(fetch, lo, hi, R, row4<E>(q + 4 * ch), scale_log2, st);
+  return st;
+}
+
 // Barrier, then combine the waves' published partials into the output (one
 // split) or the split's fp32 partial (`unit` of pairs * n_splits).
-template <int E>
-__device__ __forceinline__ void merge_out(const AttnCommon& P, char* lds, int64_t pair, size_t unit) {
+// redo(hn, ch): a NaN result of bf16 rows in plain fp32.
+template <int E, class Redo>
+__device__ __forceinline__ void merge_out(const AttnCommon& P, char* lds, int64_t pair, size_t unit, Redo&& redo) {
   __syncthreads();
   const float* sh_m = reinterpret_cast<const float*>(lds + kLdsM);
   const float* sh_l = reinterpret_cast<const float*>(lds + kLdsL);
@@ -514,6 +541,14 @@ __device__ __forceinline__ void merge_out(const AttnCommon& P, char* lds, int64_
     const float f = __builtin_amdgcn_exp2f(mw[w] - M);
     L += lw[w] * f;
     acc += ow[w] * f;
+  }
+  if constexpr (E == kEltBf16) {
+    if (any_nan(L, acc)) {
+      const PlainState ps = redo(hn, ch);
+      M = ps.m;
+      L = ps.l;
+      acc = ps.o;
+    }
   }
   if (P.n_splits == 1) {
     const float inv = L > 0.f ? 1.0f / L : 0.f;   // L == 0: a sequence of length 0
@@ -592,6 +627,14 @@ struct RowsSrc {
     if (it.n > 0) it.rot = (int)((uint64_t)pair % (uint64_t)it.n);
     it.R = P.R;
     f16_queue(P, it, P.R, wave, lane, ctr, sync, st);
+  }
+
+  __device__ __forceinline__ PlainState plain(int64_t pair, int split, const AttnCommon& P, int hn, int ch) const {
+    const size_t off = (size_t)pair * rows * kHeadDim;
+    const int lo = split * P.tiles_per_split * kTile;
+    return plain_rows<E>(reinterpret_cast<const char*>(k + off), reinterpret_cast<const char*>(v + off), kRowBytes,
+                         lo, min(lo + P.tiles_per_split * kTile, rows), P.R,
+                         P.q + ((size_t)pair * P.G + hn) * kHeadDim, ch, P.scale_log2);
   }
 };
 
@@ -705,6 +748,15 @@ struct PagedSrc {
     it.n = max(0, min(P.tiles_per_split, tiles - it.tile0));
     it.R = R;
     f16_queue(P, it, R, wave, lane, ctr, sync, st);
+  }
+
+  // (the calls of this type: the sparse rule over a cache without a table)
+  __device__ __forceinline__ PlainState plain(int64_t pair, int split, const AttnCommon& P, int hn, int ch) const {
+    const int64_t b = pair / P.KVH, at = b * page_bytes + (pair - b * P.KVH) * head_bytes;
+    const SlotRanges R = sparse_ranges(max((int)((cint32*)lens)[b], 0), window, sink, layout);
+    const int lo = split * P.tiles_per_split * kTile;
+    return plain_rows<E>(k + at, v + at, row_bytes, lo, min(lo + P.tiles_per_split * kTile, rows), R,
+                         P.q + ((size_t)pair * P.G + hn) * kHeadDim, ch, P.scale_log2);
   }
 };
 
@@ -1113,7 +1165,19 @@ __global__ __launch_bounds__(kThreads, 1) void attn_kernel(AttnCommon P, Src S) 
   WaveState st;
   wave_state_init(st);
   S.process(pair, split, P, wave, lane, ctr, sync, st);
-  merge_out<src_elt<Src>::value>(P, lds, pair, blockIdx.x);
+  merge_out<src_elt<Src>::value>(P, lds, pair, blockIdx.x, [](int hn, int ch) {
+    if constexpr (src_elt<Src>::value == kEltBf16) {
+      struct Args {
+        AttnCommon P;
+        Src S;
+      };
+      const Args A = kernargs_again<Args>();
+      return A.S.plain((int64_t)(blockIdx.x / (unsigned)A.P.n_splits), (int)(blockIdx.x % (unsigned)A.P.n_splits),
+                       A.P, hn, ch);
+    } else {
+      return PlainState();
+    }
+  });
   if constexpr (has_arrive<Src>::value) S.arrive(pair, P);
 }
 
@@ -1241,8 +1305,11 @@ static_assert(LeanLds<kWaves>::kL == kLdsL && LeanLds<kWaves>::kSlots == kLdsSlo
 // published partials into the fp16 output rows of this KV head.  The waves
 // of bit mask SKIP (never wave 0) have had their partials combined into
 // another's.
-template <int NW = kWaves, unsigned SKIP = 0, int E = kEltF16>
-__device__ __forceinline__ void lean_merge(const LeanCommon& C, const char* lds, uint32_t head) {
+struct NoRedo {
+  __device__ __forceinline__ PlainState operator()(int, int) const { return PlainState(); }
+};
+template <int NW = kWaves, unsigned SKIP = 0, int E = kEltF16, class Redo = NoRedo>
+__device__ __forceinline__ void lean_merge(const LeanCommon& C, const char* lds, uint32_t head, Redo&& redo = Redo()) {
   typedef LeanLds<NW> Lds;
   static_assert((SKIP & 1u) == 0, "wave 0's partial is always read");
   __syncthreads();
@@ -1272,6 +1339,13 @@ __device__ __forceinline__ void lean_merge(const LeanCommon& C, const char* lds,
     const float f = __builtin_amdgcn_exp2f(mw[w] - M);
     L += lw[w] * f;
     acc += ow[w] * f;
+  }
+  if constexpr (E == kEltBf16) {   // (redo: as in merge_out)
+    if (any_nan(L, acc)) {
+      const PlainState ps = redo(hn, ch);
+      L = ps.l;
+      acc = ps.o;
+    }
   }
   const float inv = L > 0.f ? 1.0f / L : 0.f;
   store_out4<E>(C.o + ((size_t)head * C.G + hn) * kHeadDim + 4 * ch, acc * inv);
@@ -1446,7 +1520,12 @@ __global__ __launch_bounds__(kThreads, 1) void f16_lean_kernel(F16LeanArgs A) {
   }
   lean_publish_ml(A.c.G, st, lds, lane, wave);
   lean_publish_f(A.c.G, st, slot, lane);
-  lean_merge<kWaves, 0u, E>(A.c, lds, head);
+  lean_merge<kWaves, 0u, E>(A.c, lds, head, [](int hn, int ch) {
+    const F16LeanArgs A = kernargs_again<F16LeanArgs>();
+    const size_t off = (size_t)blockIdx.x * A.rows * kHeadDim;
+    return plain_rows<E>(reinterpret_cast<const char*>(A.k + off), reinterpret_cast<const char*>(A.v + off), kRowBytes,
+                         0, A.rows, A.c.R, A.c.q + ((size_t)blockIdx.x * A.c.G + hn) * kHeadDim, ch, A.c.scale_log2);
+  });
 }
 
 // The fused KIVI decode with an fp16 residual of at most 128 rows (4 tiles;
@@ -2125,16 +2204,10 @@ __device__ __forceinline__ void kivi_slot4(const KiviWideArgs& A, uint32_t head,
   }
 }
 
-// The workgroup's slots for query head hn in plain fp32 (plain_slots).  The
-// kernel's arguments are read again, through a pointer the compiler cannot see
-// through: kept from the kernel's start, they would spill its registers.
+// The workgroup's slots for query head hn in plain fp32 (plain_slots).
 template <bool SPLIT, bool VAR, int BITS, int E>
 __device__ __forceinline__ PlainState wide_plain(int hn, int ch) {
-  typedef __attribute__((address_space(4))) const KiviWideArgs Args;
-  Args* ka = (Args*)__builtin_amdgcn_kernarg_segment_ptr();
-  asm volatile("" : "+s"(ka));
-  KiviWideArgs A;
-  __builtin_memcpy(&A, (const void*)ka, sizeof A);
+  const KiviWideArgs A = kernargs_again<KiviWideArgs>();
   const uint32_t head = wide_head<SPLIT>(A);
   const WideShare w = wide_share<SPLIT, VAR>(A, head);
   const float4v q = row4<E>(A.c.q + ((size_t)head * A.c.G + hn) * kHeadDim + 4 * ch);

@@ -111,3 +111,46 @@ def test_logits_far_below_zero(L, device):
     # equal logits: the mean of V
     want = v.double().mean(2, keepdim=True).expand(1, 2, 8, 128).reshape(1, 16, 128).numpy()
     _check(o, want)
+
+
+def _check_infinite(o, ref):
+    got, fin = o.double().cpu().numpy(), np.isfinite(ref)
+    assert np.array_equal(got[~fin], ref[~fin]) and (~fin).any()
+    _check(torch.where(torch.from_numpy(fin).to(o.device), o, torch.zeros_like(o)), np.where(fin, ref, 0.0))
+
+
+@pytest.mark.parametrize("H,KVH", [(32, 2), (3, 1)])
+@pytest.mark.parametrize("L,at", [(20, 3), (500, 499), (515, 512), (9000, 0), (9000, 4700), (9000, 8999)])
+def test_infinite_value_rows(H, KVH, L, at, device):
+    """An attended infinity in V is that infinity in its channel's output."""
+    from dense_kernel import dense_decode_attention
+    q, k, v = _bf16((2, H, 128), 17), _bf16((2, KVH, L, 128), 18), _bf16((2, KVH, L, 128), 19)
+    v[:, :, at, 5], v[:, 0, at, 77] = float("inf"), float("-inf")
+    say(f"dense bf16 H={H} L={L} infinite V at {at}")
+    o = dense_decode_attention(q.to(device), k.to(device), v.to(device), seq_len=L)
+    _check_infinite(o, O.dense_attention(q.float().numpy(), k.float().numpy(), v.float().numpy(), SCALE))
+
+
+@pytest.mark.parametrize("W", [29, 512, 1500])
+@pytest.mark.parametrize("layout", ["linear", "ring"])
+def test_infinite_sparse_rows(W, layout, device):
+    """The same under the sink and window rule, NaN in the slots it masks."""
+    from sparse_kernel import sparse_decode_attention
+    B, H, KVH, S = 3, 24, 8, 4
+    q, k, v = _bf16((B, H, 128), 20), _bf16((B, KVH, S + W, 128), 21), _bf16((B, KVH, S + W, 128), 22)
+    v[:, :, 1, 9] = float("inf")
+    f = [x.float().numpy() for x in (q, k, v)]
+    lay = 0 if layout == "linear" else 1
+    for L in (2, S + W // 2, 100000):
+        valid = O.slot_validity(L, W, S, lay)
+        kd, vd = k.clone(), v.clone()
+        kd[:, :, ~torch.from_numpy(valid)] = float("nan")
+        vd[:, :, ~torch.from_numpy(valid)] = float("nan")
+        say(f"sparse bf16 {layout} W={W} L={L} infinite V")
+        o = sparse_decode_attention(q.to(device), kd.to(device), vd.to(device), seq_len=L, window=W, sink=S,
+                                    layout=layout)
+        _check_infinite(o, O.masked_attention(*f, valid, SCALE))
+    lens = np.array([2, S + W // 3, S + W + 9], dtype=np.int32)
+    o = sparse_decode_attention(q.to(device), k.to(device), v.to(device), seq_len=dev(lens, device), window=W,
+                                sink=S, layout=layout)
+    _check_infinite(o, O.sparse_attention_varlen(*f, lens, W, S, SCALE, layout=lay))
