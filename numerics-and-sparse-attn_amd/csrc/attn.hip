@@ -423,7 +423,8 @@ __device__ __forceinline__ Shares share_splits(const AttnCommon& P, int lane) {
 // result once more, from the cache in fp32 as the generic kernel does, slot by
 // slot: the half wave that holds a query head's output (lane c of 32: channels
 // 4c .. 4c + 3) steps all of its workgroup's slots.  Finite calls pay one
-// comparison of the merged values.
+// comparison of the merged values.  A KIVI workgroup whose scales lie too far
+// apart for two fp16 parts (q_tile_stage_n's `far`) goes the same way.
 // ---------------------------------------------------------------------------
 struct PlainState {
   float m = kMaxSentinel, l = 0.f;
@@ -2253,7 +2254,10 @@ __global__ __launch_bounds__(Wide<BITS>::kThreads, 1) void kivi_wide_kernel(Kivi
     const bool sk = i == g1;
     load_q_group(sk ? Ts : Tw, sk ? 0u : head * (uint32_t)nwt + (uint32_t)i, i < n_q, lane, X);
   };
-  if (threadIdx.x == 0) *ctr = g0 + Wd::kQWaves;
+  if (threadIdx.x == 0) {
+    *ctr = g0 + Wd::kQWaves;
+    if constexpr (kNorm) ctr[1] = 0;
+  }
   Raw X;
   int i = n_q;
   if (wave < Wd::kQWaves) {
@@ -2294,11 +2298,12 @@ __global__ __launch_bounds__(Wide<BITS>::kThreads, 1) void kivi_wide_kernel(Kivi
   QState qs;
   q_state_init(qs);
   int v_field = 0;
+  uint64_t far = 0;   // kNorm: lanes that saw scales too far apart
   // stages X and returns its slack; `f` is the staged tile's logit factor
   auto stage = [&](int slot0, int xlim, float& f) {
     if constexpr (kNorm) {
       int k;
-      q_tile_stage_n<BITS>(X, slot, lane, slot0, xlim, R, k, v_field, qs);
+      q_tile_stage_n<BITS>(X, slot, lane, slot0, xlim, R, k, v_field, qs, far);
       f = __builtin_ldexpf(sl2, -k);
       return kRescaleSlack;
     } else {
@@ -2323,7 +2328,10 @@ __global__ __launch_bounds__(Wide<BITS>::kThreads, 1) void kivi_wide_kernel(Kivi
     q_tile_body<false, true, PACK, BITS>(slot, qB, 0, A.sink, R, f, slack, st, qs, lane);
   }
   wide_publish_ml<BITS>(A.c.G, st, lds, lane, wave);
-  if constexpr (kNorm) q_state_unshift(qs, v_field);
+  if constexpr (kNorm) {
+    q_state_unshift(qs, v_field);
+    if (far != 0 && lane == 0) ctr[1] = 1;
+  }
   publish_q<false, PACK, BITS>(qs, slot, lane);
 
   // merge: one thread per (head, 4 channels) over the waves' quantized partials
@@ -2364,7 +2372,7 @@ __global__ __launch_bounds__(Wide<BITS>::kThreads, 1) void kivi_wide_kernel(Kivi
     }
   }
   if constexpr (kNorm) {
-    if (any_nan(L, acc)) {
+    if (ctr[1] != 0 || any_nan(L, acc)) {
       const PlainState ps = wide_plain<SPLIT, VAR, BITS, E>(hn, ch);
       M = ps.m;
       L = ps.l;

@@ -1073,17 +1073,24 @@ __device__ __forceinline__ float q_tile_stage(const QTileRaw& raw, char* slot, i
   return __ballot(!(fmaxf((float)vs[0], (float)vs[1]) <= kSlackVScale)) ? 0.0f : kRescaleSlack;
 }
 
-// The staging of a tile whose Q operand is scaled to less than 2^15 in
+// The staging of a tile whose Q operand is scaled to less than 2^8 in
 // magnitude (q_normalize), with powers of two taken out of its scales: K scales
-// come to [2^-1, 1) at their largest (k_exp: the tile's logits are 2^k_exp too
+// come to [2^6, 2^7) at their largest (k_exp: the tile's logits are 2^k_exp too
 // large), V scales to at most 2^7 over all of the wave's tiles so far (v_field:
 // the largest exponent field seen; a tile with a larger one rescales the
 // accumulators), so that neither product's exact remainder falls into fp16's
 // subnormal range, for wide codes and small scales alike, and P' < 2^15 with
 // the softmax's slack.  (The 2-bit fp16 path scales Q alone: its remainders
 // below 2^-24 cost less than its codes' 0..3 carry into a result of order 1.)
+// The two parts end at 2^-25 whatever the scale: a product 2^-s of the largest
+// its head's |q| and the tile's scales allow (2^14) has s - 38 bits behind its
+// point.  `far` collects the tiles in which that leaves less than about 2^-22
+// of a head's largest term: a K scale more than kKSpan exponents below the
+// tile's largest (a head's largest |q| may stand on it), or a V scale other
+// than 0 more than kVSpan below v_field.
 // Tokens of a tile that is not fully valid lose their V scale and zero: a slot
 // never written may hold any bits.
+constexpr int kKSpan = 16, kVSpan = 9;
 // The largest exponent field (0..31) of fp16 magnitudes over the wave.
 __device__ __forceinline__ int max_field(uint32_t h2) {
   const int el = (int)(max(h2 & 0x7FFFu, (h2 >> 16) & 0x7FFFu) >> 10);
@@ -1102,9 +1109,11 @@ __device__ __forceinline__ uint32_t scale_pk(uint32_t h2, int k) {
 }
 template <int BITS>
 __device__ __forceinline__ void q_tile_stage_n(const QTileRawN<BITS>& X, char* slot, int lane, int slot0, int xlim,
-                                               const SlotRanges& R, int& k_exp, int& v_field, QState& qs) {
+                                               const SlotRanges& R, int& k_exp, int& v_field, QState& qs, uint64_t& far) {
   typedef QSlot<BITS> Lay;
-  k_exp = 14 - max_field(X.ks);
+  const int kf = max_field(X.ks), k_least = max(kf - kKSpan, 0) << 10;
+  k_exp = 21 - kf;
+  far |= __ballot((int)min(X.ks & 0x7FFFu, (X.ks >> 16) & 0x7FFFu) < k_least);
 #pragma unroll
   for (int i = 0; i < kQPieces<BITS>; ++i) {
     const int krow = 8 * i + (lane >> 3);
@@ -1128,6 +1137,9 @@ __device__ __forceinline__ void q_tile_stage_n(const QTileRawN<BITS>& X, char* s
     for (int b = 0; b < 8; ++b) qs.O[b] = qs.O[b] * down;
     v_field = vf;
   }
+  // (0 - 1 wraps round to the largest)
+  const uint32_t v_least = max((uint32_t)max(v_field - kVSpan, 0) << 10, 1u) - 1u;
+  far |= __ballot(min((vs & 0x7FFFu) - 1u, ((vs >> 16) & 0x7FFFu) - 1u) < v_least);
   vs = scale_pk(vs, v_shift(v_field));
   *reinterpret_cast<uint16_t*>(slot + Lay::kVS + g0 * 64 + 2 * tok) = (uint16_t)vs;
   *reinterpret_cast<uint16_t*>(slot + Lay::kVS + (g0 + 1) * 64 + 2 * tok) = (uint16_t)(vs >> 16);
@@ -1142,14 +1154,14 @@ __device__ __forceinline__ void q_state_unshift(QState& qs, int v_field) {
 }
 
 // The Q operand of element type E as fp16, each query head scaled by its own
-// power of two 2^-e, which brings that head's largest |q| to [2^14, 2^15);
+// power of two 2^-e, which brings that head's largest |q| to [2^7, 2^8);
 // returns the lane's head's e (heads share nothing: one that is far larger than
 // the others, or not finite, must not reach them).  Exact for every channel
-// within 2^-28 of the head's largest (bf16's 8 bits: 2^-31), the rest off by at
-// most 2^-39 of it.
+// within 2^-21 of the head's largest (bf16's 8 bits: 2^-24), the rest off by at
+// most 2^-32 of it.
 template <int E>
 __device__ __forceinline__ int q_normalize(half8 (&qB)[4]) {
-  constexpr int kMant = E == kEltBf16 ? 7 : 10, kBias = E == kEltBf16 ? 141 : 29;
+  constexpr int kMant = E == kEltBf16 ? 7 : 10, kBias = E == kEltBf16 ? 134 : 22;
   uint32_t top = 0;
 #pragma unroll
   for (int c = 0; c < 4; ++c)

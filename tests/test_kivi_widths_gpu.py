@@ -168,6 +168,55 @@ def test_channels_far_apart(bits, device):
     _check(o, ref, "bf16")
 
 
+def _relative(o, ref, dt):
+    """Half an ulp plus 1e-5 of the head's largest output (2^-25: fp16's own
+    spacing below its normal range)."""
+    got, top = o.double().cpu().numpy(), np.abs(ref).max(-1, keepdims=True)
+    ulp = 2.0 ** (np.floor(np.log2(np.maximum(np.abs(ref), 1e-30))) - (11 if dt == "fp16" else 8))
+    assert (np.abs(got - ref) - ulp - 1e-5 * top).max() <= (2.0**-25 if dt == "fp16" else 0.0)
+
+
+@pytest.mark.parametrize("bits,dt", [(4, "fp16"), (4, "bf16"), (2, "bf16")])
+@pytest.mark.parametrize("span", [8, 16, 17, 18, 24])
+def test_key_scales_far_apart(bits, dt, span, device):
+    """Every other channel's keys 2^span the others', its query as much smaller."""
+    B, H, KVH, S, W, R = 1, 16, 2, 4, 448, 128
+    big = torch.arange(128) % 2 == 0
+    lo, hi = 2.0 ** -(span // 2), 2.0 ** (span - span // 2)
+    kc, vc, q = (torch.from_numpy(randn(n, i)) for n, i in
+                 (((B, KVH, S + W, 128), 91), ((B, KVH, S + W, 128), 92), ((B, H, 128), 93)))
+    kc = torch.where(big, kc * hi, kc * lo).to(DT[dt])
+    q = (torch.where(big, q / hi, q / lo) * 2).to(DT[dt])
+    vc = vc.to(DT[dt])
+    hc = O.build_quantized_kv_cache(kc.float().numpy(), vc.float().numpy(), residual_size=R, sink=S, bits=bits)
+    hc["k_residual"], hc["v_residual"] = (x[:, :, -R:].float().numpy() for x in (kc, vc))
+    ref = O.quantized_attention_masked(q.float().numpy(), hc, 163840, W, SCALE, sink=S, residual_size=R, bits=bits)
+    say(f"kivi bits={bits} {dt} key scales 2^{span} apart")
+    _relative(_attend(q.to(device), _upload(hc, dt, device), 163840, W, S, R, bits), ref, dt)
+
+
+@pytest.mark.parametrize("bits,dt", [(4, "fp16"), (4, "bf16"), (2, "bf16")])
+@pytest.mark.parametrize("span", [8, 10, 12, 20, 24])
+def test_value_scales_far_apart(bits, dt, span, device):
+    """Two tokens of weight 0 whose values are 2^span the others', and two whose
+    values are 0."""
+    B, H, KVH, S, W, R = 1, 16, 2, 4, 448, 128
+    kc, vc, q = (torch.from_numpy(randn(n, i)) for n, i in
+                 (((B, KVH, S + W, 128), 94), ((B, KVH, S + W, 128), 95), ((B, H, 128), 96)))
+    q[..., 40] = 4
+    out = [S + 5, S + 200]
+    kc[:, :, out, 40] = -300
+    vc *= 2.0**-10
+    vc[:, :, out] *= 2.0**span
+    vc[:, :, [S + 9, S + 100]] = 0
+    kc, vc, q = (x.to(DT[dt]) for x in (kc, vc, q))
+    hc = O.build_quantized_kv_cache(kc.float().numpy(), vc.float().numpy(), residual_size=R, sink=S, bits=bits)
+    hc["k_residual"], hc["v_residual"] = (x[:, :, -R:].float().numpy() for x in (kc, vc))
+    ref = O.quantized_attention_masked(q.float().numpy(), hc, 163840, W, SCALE, sink=S, residual_size=R, bits=bits)
+    say(f"kivi bits={bits} {dt} value scales 2^{span} apart")
+    _relative(_attend(q.to(device), _upload(hc, dt, device), 163840, W, S, R, bits), ref, dt)
+
+
 @pytest.mark.parametrize("bits,dt", [(4, "fp16"), (2, "bf16")])
 def test_slots_never_written(bits, dt, device):
     """NaN patterns in every quantized byte and residual row of slots past the
