@@ -14,6 +14,7 @@ from __future__ import annotations
 
 import ctypes
 import os
+import warnings
 
 # torch must load its bundled HIP runtime before libkvdec.so is opened: both
 # carry the SONAME libamdhip64.so.7, and whichever is loaded first is the one
@@ -110,18 +111,35 @@ def _load() -> ctypes.CDLL:
 lib = _load()
 
 
+class _Checked:
+    """Stands in for the native fast path where it cannot run: None to every
+    call, so that each goes through its wrapper's checks and ctypes."""
+
+    def __getattr__(self, name):
+        return lambda *args: None
+
+
 def _load_host():
     """The wrappers' native fast path (csrc/host.cpp), bound to the library
     loaded above: each function makes a whole call, or returns None for a call
-    that the wrapper itself has to check (and refuse, or convert)."""
+    that the wrapper itself has to check (and refuse, or convert).  It is tied
+    to the torch it was compiled against; under another one the wrappers run
+    the same kernels without it (with a warning: small calls take longer)."""
+    rebuild = f"build it with `python {os.path.join(_HERE, 'build.py')}` (or __graft_entry__.build())"
     try:
         import _kvdec_host
     except ModuleNotFoundError as e:
-        raise ImportError(
-            f"_kvdec_host.so is missing: build it with `python {os.path.join(_HERE, 'build.py')}` "
-            "(or __graft_entry__.build())") from e
-    _kvdec_host.bind(LIB_PATH, check)
-    return _kvdec_host
+        raise ImportError(f"_kvdec_host.so is missing: {rebuild}") from e
+    except ImportError as e:
+        why = str(e)
+    else:
+        built, here = _kvdec_host.torch_version, torch.__version__.split("+")[0]
+        if built == here:
+            _kvdec_host.bind(LIB_PATH, check)
+            return _kvdec_host
+        why = f"compiled against torch {built}, this is {here}"
+    warnings.warn(f"_kvdec_host.so cannot be used ({why}): {rebuild}", RuntimeWarning, stacklevel=2)
+    return _Checked()
 
 
 class KvdecLaunchError(RuntimeError):

@@ -21,6 +21,7 @@
 #include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/generated/variable_factories.h>
 #include <torch/csrc/autograd/python_variable.h>
+#include <torch/version.h>
 
 #include <algorithm>
 #include <climits>
@@ -493,4 +494,8 @@ PyModuleDef module = {PyModuleDef_HEAD_INIT, "_kvdec_host", nullptr, -1, methods
 
 }  // namespace
 
-PyMODINIT_FUNC PyInit__kvdec_host() { return PyModule_Create(&module); }
+PyMODINIT_FUNC PyInit__kvdec_host() {
+  PyObject* m = PyModule_Create(&module);
+  if (m && PyModule_AddStringConstant(m, "torch_version", TORCH_VERSION)) Py_CLEAR(m);
+  return m;
+}

@@ -5,6 +5,7 @@ negative codes before any HIP call."""
 import ctypes
 import os
 import re
+import sys
 
 import pytest
 
@@ -485,6 +486,18 @@ def test_dequant_tile_validation():
     assert K.lib.kvdec_dequant_k_tile(FAKE, FAKE, FAKE, FAKE, 0, 0, 1, 1, 1, 128, 128, None) == E["SHAPE"]
     assert K.lib.kvdec_dequant_v_tile(FAKE, FAKE, FAKE, FAKE, 0, 0, 1, 1, 128, 128, None) == E["SHAPE"]
     assert K.lib.kvdec_dequant_v_tile(FAKE, FAKE, FAKE, FAKE, 0, 32, 1, 1, 100, 128, None) == E["DGROUP"]
+
+
+@pytest.mark.parametrize("body", ["raise ImportError('undefined symbol: x')", "torch_version = '1.0.0'"])
+def test_fast_path_of_another_torch(body, tmp_path, monkeypatch):
+    """A fast path that cannot be loaded, or was compiled against another
+    torch, leaves every call to the wrappers, with a warning."""
+    (tmp_path / "_kvdec_host.py").write_text(body)
+    monkeypatch.syspath_prepend(str(tmp_path))
+    monkeypatch.delitem(sys.modules, "_kvdec_host", raising=False)
+    with pytest.warns(RuntimeWarning, match="_kvdec_host.so cannot be used"):
+        host = K._load_host()
+    assert host.sparse(None, None, None, 1, 2, 3, 0, 0.1) is None and host.build() is None
 
 
 def test_python_wrappers_reject_cpu_tensors():
