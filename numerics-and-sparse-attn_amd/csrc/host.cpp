@@ -342,14 +342,18 @@ PyObject* step_attend(PyObject*, PyObject* const* a, Py_ssize_t n) {
     return none();
   for (int i = 0; i < 6; ++i)
     if (!to_i32(a[9 + i], geo[i])) return none();
-  const Tensor* t[14];
+  // the cache's tensors, held until the launch: the dict lends them, and a
+  // thread may replace an entry while the GIL is released
+  Tensor t[14];
   for (int i = 0; i < 14; ++i) {
     PyObject* x = PyDict_GetItem(a[0], keys[i]);
-    if (!x || !(t[i] = gpu_tensor(x))) return none();
+    const Tensor* g = x ? gpu_tensor(x) : nullptr;
+    if (!g) return none();
+    t[i] = *g;
   }
-  if (t[0]->dim() != 4) return none();
-  const c10::Device dev = t[0]->device();
-  const int64_t B = t[0]->size(0), KVH = t[0]->size(1), D = t[0]->size(3), H = q->size(1);
+  if (t[0].dim() != 4) return none();
+  const c10::Device dev = t[0].device();
+  const int64_t B = t[0].size(0), KVH = t[0].size(1), D = t[0].size(3), H = q->size(1);
   const Tensor* tok[2];
   for (int i = 0; i < 2; ++i)
     if (!(tok[i] = gpu_tensor(a[2 + i])) || tok[i]->scalar_type() != at::kHalf || !tok[i]->is_contiguous() ||
@@ -361,10 +365,10 @@ PyObject* step_attend(PyObject*, PyObject* const* a, Py_ssize_t n) {
     if (!(st[i] = gpu_tensor(a[5 + i])) || st[i]->device() != dev) return none();
   if (!shaped(*q, {B, H, D}) || q->device() != dev || !fits_i32(KVH)) return none();
   const void* parts[12];
-  for (int i = 0; i < 12; ++i) parts[i] = ptr(*t[2 + i]);
+  for (int i = 0; i < 12; ++i) parts[i] = ptr(t[2 + i]);
   int32_t* state[4];
   for (int i = 0; i < 4; ++i) state[i] = (int32_t*)st[i]->data_ptr();
-  void* rings[2] = {t[0]->data_ptr(), t[1]->data_ptr()};
+  void* rings[2] = {t[0].data_ptr(), t[1].data_ptr()};
   Tensor o;
   int rc;
   {

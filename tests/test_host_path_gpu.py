@@ -2,6 +2,8 @@
 what the checked Python path gives, and every call that path refuses it leaves
 alone, so that the error is the same."""
 
+import threading
+
 import numpy as np
 import pytest
 import torch
@@ -110,6 +112,33 @@ def test_stream_step_same_as_checked_path(monkeypatch):
             outs = [c.step_attend(q, kn * (i + 1), vn, active=active) for i in range(34)]
             return [outs, c.t, c.appended, c.ring]
         _both(monkeypatch, steps)
+
+
+def test_stream_step_while_entries_are_replaced():
+    """The step holds the cache's tensors: another thread may put copies of the
+    parts it only reads in their place."""
+    k, v, q = _randn(2, 2, 300, 128), _randn(2, 2, 300, 128), _randn(2, 16, 128)
+    kn, vn = _randn(2, 2, 128), _randn(2, 2, 128)
+
+    def steps(replace):
+        c = kivi_stream.KiviStreamBatch.from_prefill(k, v, window=192)
+        stop = threading.Event()
+
+        def work():
+            while not stop.is_set():
+                for n in list(c.t):
+                    if "_sink_" in n:
+                        c.t[n] = c.t[n].clone()
+        t = threading.Thread(target=work)
+        if replace:
+            t.start()
+        try:
+            return torch.stack([c.step_attend(q, kn * (i + 1), vn) for i in range(200)])
+        finally:
+            stop.set()
+            if replace:
+                t.join()
+    assert torch.equal(steps(False), steps(True))
 
 
 def test_calls_left_to_the_checks(monkeypatch):
