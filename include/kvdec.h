@@ -168,8 +168,8 @@ int kvdec_sparse_decode_varlen(const void* q, const void* k_cache, const void* v
  *            token pf*p+j in bits j*bits .. j*bits + bits - 1
  *   scale, zero : [B, KVH, N/group, D] fp16
  *   1 <= bits <= 8, N % group == 0, group % pf == 0 (whole bytes per group).
- *   bits of 1, 2, 4 or 8 with group == 32 (D even, tensors on 16-byte
- *   boundaries) is the fast path, anything else a generic kernel.
+ *   bits of 1, 2, 4 or 8 with group == 32 (D even; other than 2 bits: tensors
+ *   on 16-byte boundaries) is the fast path, anything else a generic kernel.
  *   QMAX = 2^bits - 1; codes are bit-exact to the
  *   IEEE-float32 closed form s = (mx - mn) / QMAX, ... (quant_kernel.py:77-99).
  */

@@ -252,10 +252,10 @@ struct VRaw {
 
 template <typename T>
 __device__ __forceinline__ void v_load(const T* grp, VRaw<T>& r) {
-  const u32x4* p = reinterpret_cast<const u32x4*>(grp);
 #pragma unroll
   for (int i = 0; i < VRaw<T>::kW / 4; ++i) {
-    const u32x4 v = p[i];
+    u32x4 v;   // (one 16-byte load at any alignment of T: HSA runs in unaligned access mode)
+    __builtin_memcpy(&v, reinterpret_cast<const char*>(grp) + 16 * i, 16);
 #pragma unroll
     for (int j = 0; j < 4; ++j) r.w[4 * i + j] = v[j];
   }
@@ -311,16 +311,18 @@ __device__ __forceinline__ void v_quantize(const VRaw<T>& r, int64_t u, uint8_t*
   else
     codes(std::false_type());
   // streaming (non-temporal) stores: outputs are not read again here
+  uint8_t* p = packed + (size_t)u * (4 * BITS);
   if constexpr (BITS % 4 == 0) {
 #pragma unroll
     for (int i = 0; i < BITS / 4; ++i)
       __builtin_nontemporal_store(u32x4{out[4 * i], out[4 * i + 1], out[4 * i + 2], out[4 * i + 3]},
-                                  reinterpret_cast<u32x4*>(packed) + (size_t)u * (BITS / 4) + i);
+                                  reinterpret_cast<u32x4*>(p) + i);
   } else if constexpr (BITS == 2) {
-    __builtin_nontemporal_store(u32x2{out[0], out[1]}, reinterpret_cast<u32x2*>(packed) + u);
+    typedef u32x2 any_u32x2 __attribute__((aligned(1)));
+    __builtin_nontemporal_store(any_u32x2{out[0], out[1]}, reinterpret_cast<any_u32x2*>(p));
   } else {
     static_assert(BITS == 1, "one 32-bit word");
-    __builtin_nontemporal_store(out[0], reinterpret_cast<uint32_t*>(packed) + u);
+    __builtin_nontemporal_store(out[0], reinterpret_cast<uint32_t*>(p));
   }
   __builtin_nontemporal_store((_Float16)q.s, scale + u);
   __builtin_nontemporal_store((_Float16)q.z, zero + u);
@@ -755,10 +757,11 @@ int launch_quant_generic(bool k, const void* x, int in_dtype, void* packed_u8, v
 
 // Groups of 32 with 1, 2, 4 or 8 bits take the streaming kernels above, which
 // read the input once and divide by Markstein's sequence (bound by the
-// read/write mix); the rest, and tensors that do not allow their accesses (the
-// 2-bit form has always assumed them), the generic ones: K and V of B=8, N=4096,
-// bf16 at 4 bits 236.6 -> 32.3 us (5.4 TB/s of input and output; there two reads
-// of the input, an IEEE division per element and byte stores).
+// read/write mix); the rest, and at 1, 4 and 8 bits tensors that do not allow
+// their accesses, the generic ones: K and V of B=8, N=4096, bf16 at 4 bits 236.6
+// -> 32.3 us (5.4 TB/s of input and output; there two reads of the input, an
+// IEEE division per element and byte stores).  2 bits streams from and to any
+// alignment of the elements.
 bool stream_form(const void* x, const void* p, const void* s, const void* z, int group, int bits) {
   if (group != kGroup || (bits & (bits - 1)) != 0) return false;
   if (bits == 2) return true;

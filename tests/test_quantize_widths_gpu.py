@@ -50,3 +50,28 @@ def test_off_16_byte_boundary(dt, device):
     buf = torch.zeros(x.numel() + 1, dtype=DT[dt], device=device)
     buf[1:] = x.flatten().to(device)
     _compare(buf[1:].view(x.shape), 4, f"quantize 4 bits {dt}, one element off alignment")
+
+
+@pytest.mark.parametrize("dt", ["fp32", "fp16", "bf16"])
+@pytest.mark.parametrize("off", [1, 2, 3])
+def test_two_bits_off_16_byte_boundary(dt, off, device):
+    """2-bit input `off` elements off alignment, codes as many bytes and scales
+    and zeros as many halves off, bit for bit; nothing around them is written."""
+    import _kvdec as K
+    B, KVH, N, D = 1, 2, 64, 128
+    x = torch.from_numpy(randn((B, KVH, N, D), 12 + off)).to(DT[dt])
+    buf = torch.zeros(x.numel() + off, dtype=DT[dt], device=device)
+    buf[off:] = x.flatten().to(device)
+    xd = buf[off:].view(x.shape)
+    _compare(xd, 2, f"quantize 2 bits {dt}, {off} elements off alignment")
+    for fn, ofn in ((K.lib.kvdec_quantize_k, O.quantize_k), (K.lib.kvdec_quantize_v, O.quantize_v)):
+        want = ofn(x.float().numpy(), 32, 2)
+        out = [torch.full((w.size + off + 16,), 77, dtype=torch.uint8 if w.dtype == np.uint8 else torch.float16,
+                          device=device) for w in want]
+        say(f"quantize 2 bits {dt}, outputs {off} off alignment")
+        rc = fn(K.ptr(xd), {"fp32": K.F32, "fp16": K.F16, "bf16": K.BF16}[dt], *[K.ptr(o[off:]) for o in out],
+                B, KVH, N, D, 32, 2, K.stream_of(xd))
+        assert rc == 0
+        for o, w in zip(out, want):
+            np.testing.assert_array_equal(host(o[off:off + w.size]).reshape(w.shape), w)
+            assert (host(o[:off]) == 77).all() and (host(o[off + w.size:]) == 77).all()
