@@ -2160,6 +2160,7 @@ struct WideShare {
 };
 template <bool SPLIT, bool VAR>
 __device__ __forceinline__ WideShare wide_share(const KiviWideArgs& A, uint32_t head) {
+  static_assert(!SPLIT || !VAR, "a split call has one length");
   const int split = SPLIT ? (int)(blockIdx.x - head * (uint32_t)A.n_splits) : 0, nwt = A.nwt;
   WideShare w;
   w.R = A.c.R;
@@ -2170,7 +2171,7 @@ __device__ __forceinline__ WideShare wide_share(const KiviWideArgs& A, uint32_t 
     first = min((w.R.vb - A.sink) / kTile, nwt);
   }
   w.g1 = SPLIT ? min((split + 1) * A.per_split + A.first, nwt) : nwt;
-  w.g0 = SPLIT ? min(max(split * A.per_split + A.first, first), w.g1) : first;
+  w.g0 = SPLIT ? min(split * A.per_split + A.first, w.g1) : first;
   w.tail = !SPLIT || split == A.n_splits - 1;
   return w;
 }
@@ -2805,8 +2806,9 @@ template <int BITS, int E>
 int launch_wide(AttnCommon P, KiviWideArgs A, void* ws, size_t ws_bytes, hipStream_t st) {
   const int64_t groups = A.nwt - A.first;
   const size_t per_split = ws_bytes_for(P.pairs, 2, P.G) / 2;
-  int64_t s = kivi_splits(P.pairs, groups);
-  if (ws == nullptr) s = 1;
+  // the calls that bring a workspace: fp16 at one length
+  constexpr bool kSplit = E == kEltF16;
+  int64_t s = kSplit && !A.lens && ws != nullptr ? kivi_splits(P.pairs, groups) : 1;
   s = std::max<int64_t>(1, std::min<int64_t>(s, (int64_t)(ws_bytes / per_split)));
   const int64_t per = (groups + s - 1) / s;
   s = s > 1 ? (groups + per - 1) / per : 1;
@@ -2817,8 +2819,9 @@ int launch_wide(AttnCommon P, KiviWideArgs A, void* ws, size_t ws_bytes, hipStre
   A.n_splits = P.n_splits;
   A.per_split = (int)per;
   void (*kern)(KiviWideArgs) =
-      s > 1 ? (A.lens ? kivi_wide_kernel<true, true, BITS, E> : kivi_wide_kernel<true, false, BITS, E>)
-            : (A.lens ? kivi_wide_kernel<false, true, BITS, E> : kivi_wide_kernel<false, false, BITS, E>);
+      A.lens ? kivi_wide_kernel<false, true, BITS, E> : kivi_wide_kernel<false, false, BITS, E>;
+  if constexpr (kSplit)
+    if (s > 1) kern = kivi_wide_kernel<true, false, BITS, E>;
   hipLaunchKernelGGL(kern, dim3((unsigned)(P.pairs * s)), dim3(Wide<BITS>::kThreads), Wide<BITS>::kBytes, st, A);
   const int rc = launch_status();
   return rc != KVDEC_OK || s == 1 ? rc : launch_merge<E>(P, st);
