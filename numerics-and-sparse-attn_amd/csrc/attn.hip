@@ -2557,7 +2557,8 @@ __global__ __launch_bounds__(64 * kMergeWaves) void merge_kernel(AttnCommon P) {
     acc += part[w][lane];
     L += part_l[w];
   }
-  const float2v r = L == 0.f ? float2v{0.f, 0.f} : float2v{acc[0] / L, acc[1] / L};   // (L may be NaN)
+  const float d = L == 0.f ? 1.f : L;   // L == 0: acc is 0 (a sequence of length 0); L may be NaN
+  const float2v r = {acc[0] / d, acc[1] / d};
   const uint32_t bits = round_elt4<E>(float4v{r[0], r[1], 0.f, 0.f})[0];
   __builtin_nontemporal_store(bits, reinterpret_cast<uint32_t*>(P.o) + (size_t)row * (kHeadDim / 2) + lane);
 }
