@@ -2599,6 +2599,9 @@ Plan make_plan(int64_t pairs, int64_t n_tiles) {
 // 26.6 -> 14.8, B=16 26.9 -> 22.0; W = 2048: B=16 16.4 -> 15.4.  W = 1024
 // (28 groups) loses by it: B=8 10.8 -> 11.2.  So do KV heads enough for every
 // CU: B=33, W = 4096 51.9 -> 54.7, B=48 55.5 -> 59.1 at 2 splits.
+// 4-bit codes, whose kernel has 12 waves: W = 16384: B=1 104.2 -> 14.7, B=2
+// 104.6 -> 19.0; W = 4096: B=1 31.1 -> 11.3, B=8 31.5 -> 18.3, B=16 33.4 -> 26.7;
+// W = 2048: B=1 18.8 -> 10.9, B=16 20.8 -> 18.7: the same line.
 constexpr int64_t kMinGroupsPerSplit = 8;
 int kivi_splits(int64_t pairs, int64_t groups) {
   const int64_t s = std::min<int64_t>(groups / kMinGroupsPerSplit, kTargetUnits / pairs);

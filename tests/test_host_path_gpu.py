@@ -157,6 +157,17 @@ def test_calls_left_to_the_checks(monkeypatch):
         assert K.host.sparse(q, k, v, 100, 64, 4, 0, 0.1) is None
 
 
+def _same_error(monkeypatch, call):
+    errors = []
+    for skip in (False, True):
+        with monkeypatch.context() as m:
+            m.setattr(K, "host", Recorder(skip))
+            with pytest.raises(Exception) as e:
+                call()
+            errors.append((e.type, str(e.value)))
+    assert errors[0] == errors[1] and errors[0][0] is not NameError
+
+
 @pytest.mark.parametrize("change", [
     dict(q=lambda q: q.cpu()), dict(q=lambda q: q.double()), dict(q=lambda q: q[0]), dict(k=lambda k: k.bfloat16()),
     dict(k=lambda k: k[:, :, :67].contiguous()), dict(k=lambda k: k.transpose(1, 2).contiguous().transpose(1, 2)),
@@ -172,11 +183,78 @@ def test_refused_as_before(monkeypatch, change):
     def call():
         return sparse_kernel.sparse_decode_attention(a["q"], a["k"], a["v"], a["seq_len"], a["window"], a["sink"],
                                                      layout=a["layout"])
-    errors = []
-    for skip in (False, True):
-        with monkeypatch.context() as m:
-            m.setattr(K, "host", Recorder(skip))
-            with pytest.raises((ValueError, TypeError)) as e:
-                call()
-            errors.append((e.type, str(e.value)))
-    assert errors[0] == errors[1]
+    _same_error(monkeypatch, call)
+
+
+def _ones(n, dtype=torch.int32):
+    return torch.ones(n, dtype=dtype, device="cuda")
+
+
+def _refused(fn, args, changes):
+    """One case per change of a good call's arguments, all of them refused."""
+    return [pytest.param(fn, args, c, id=f"{fn}-{i}") for i, c in enumerate(changes)]
+
+
+_ROWS = dict(q=lambda: _randn(1, 16, 128), k=lambda: _randn(1, 2, 68, 128), v=lambda: _randn(1, 2, 68, 128))
+_STRIDED = dict(k=lambda k: k.transpose(1, 2).contiguous().transpose(1, 2))
+
+
+@pytest.mark.parametrize("fn,args,change", [
+    *_refused("dense", dict(_ROWS, seq_len=68), [
+        dict(q=lambda q: q.cpu()), dict(q=lambda q: q.double()), dict(q=lambda q: q[0]),
+        dict(q=lambda q: q[:, :15].contiguous()), dict(k=lambda k: k.bfloat16()), dict(v=lambda v: v[:, :1].contiguous()),
+        dict(k=lambda k: k[:, :, :67].contiguous()), dict(seq_len=67), dict(seq_len=0),
+        dict(seq_len=lambda n: _ones(3)), dict(seq_len=lambda n: _ones(1, torch.int64)), _STRIDED,
+        dict(q=lambda q: q.float(), k=lambda k: k.float(), v=lambda v: v.float(), seq_len=lambda n: _ones(1))]),
+    *_refused("paged", dict(q=lambda: _randn(2, 16, 128), k_pages=lambda: _randn(9, 16, 2, 128),
+                            v_pages=lambda: _randn(9, 16, 2, 128), block_table=lambda: _ones(8).view(2, 4),
+                            seq_lens=lambda: _lens(5, 61), max_seq_len=64), [
+        dict(q=lambda q: q.bfloat16()), dict(k_pages=lambda k: k.float()), dict(v_pages=lambda v: v[:, :8].contiguous()),
+        dict(k_pages=lambda k: _randn(9, 12, 2, 128), v_pages=lambda v: _randn(9, 12, 2, 128)),
+        dict(block_table=lambda t: t.long()), dict(block_table=lambda t: t[:1]), dict(block_table=lambda t: t.t()),
+        dict(seq_lens=lambda n: n.long()), dict(seq_lens=lambda n: n[:1]), dict(max_seq_len=65), dict(kv_layout="DHN")]),
+    *_refused("kivi", dict(q=lambda: _randn(1, 16, 128), seq_len=900, window=192), [
+        dict(q=lambda q: q.cpu()), dict(q=lambda q: q.double()), dict(q=lambda q: q[:, :15].contiguous()),
+        dict(window=193), dict(window=0), dict(seq_len=0), dict(sink=0), dict(sink=40), dict(residual_size=0),
+        dict(residual_size=96), dict(bits=9), dict(bits=3), dict(bits=4), dict(group_size=64), dict(group_size=33),
+        dict(seq_len=lambda n: _ones(2)), dict(seq_len=lambda n: _ones(1, torch.int64)),
+        dict(k_cache=lambda k: k[:, :, 1:].contiguous()), dict(v_cache=lambda v: v.float()),
+        dict(k_sink_scale=lambda x: x.float()), dict(v_win_packed=lambda x: x[:, :, ::2]),
+        dict(k_win_zero=lambda x: x[:, :1].contiguous())]),
+    *_refused("quantize_k", dict(x=lambda: _randn(1, 2, 64, 128)), [
+        dict(x=lambda x: x[:, :, :63].contiguous()), dict(x=lambda x: x.cpu()), dict(x=lambda x: x.double()),
+        dict(x=lambda x: x[0]), dict(bits=0), dict(bits=9), dict(group_size=0), dict(group_size=-32), dict(group_size=24),
+        dict(group_size=2)]),
+    *_refused("quantize_v", dict(x=lambda: _randn(1, 2, 64, 128)), [
+        dict(x=lambda x: x[..., :120].contiguous()), dict(x=lambda x: x.cpu()), dict(x=lambda x: x.double()),
+        dict(x=lambda x: x[0]), dict(bits=0), dict(bits=9), dict(group_size=0), dict(group_size=24), dict(group_size=2)]),
+    *_refused("build", dict(k=lambda: _randn(1, 2, 196, 128), v=lambda: _randn(1, 2, 196, 128)), [
+        dict(k=lambda k: k[:, :, :195].contiguous(), v=lambda v: v[:, :, :195].contiguous()),
+        dict(k=lambda k: k.cpu()), dict(k=lambda k: k.bfloat16()), dict(v=lambda v: v[:, :1].contiguous()),
+        dict(k=lambda k: k.double(), v=lambda v: v.double()), dict(k=lambda k: k[0]), dict(sink=0), dict(sink=33),
+        dict(residual_size=0), dict(residual_size=100), dict(k=lambda k: k[:, :, :4].contiguous(),
+                                                             v=lambda v: v[:, :, :4].contiguous()),
+        dict(residual_dtype=torch.bfloat16)]),
+    *_refused("step_attend", dict(q=lambda: _randn(2, 16, 128), k_new=lambda: _randn(2, 2, 128),
+                                  v_new=lambda: _randn(2, 2, 128)), [
+        dict(q=lambda q: q.cpu()), dict(q=lambda q: q.bfloat16()), dict(q=lambda q: q[:1]),
+        dict(q=lambda q: q[:, :15].contiguous()), dict(k_new=lambda k: k[:1]), dict(k_new=lambda k: k.float()),
+        dict(v_new=lambda v: v.cpu()), dict(active=lambda a: _ones(3))]),
+])
+def test_other_entries_refuse_as_before(monkeypatch, fn, args, change):
+    a = {n: x() if callable(x) else x for n, x in args.items()}
+    if fn == "kivi":
+        t = quant_kernel.build_quantized_kv_cache(_randn(1, 2, 196, 128), _randn(1, 2, 196, 128))
+        a.update(k_cache=t["k_residual"], v_cache=t["v_residual"], **{n: t[n] for n in quant_kernel._KIVI_ORDER})
+    if fn == "step_attend":
+        a["self"] = kivi_stream.KiviStreamBatch.from_prefill(_randn(2, 2, 300, 128), _randn(2, 2, 300, 128), window=192)
+    for n, x in change.items():
+        a[n] = x(a.get(n)) if callable(x) else x
+    entry = {"dense": dense_kernel.dense_decode_attention, "paged": paged_kernel.paged_decode_attention,
+             "kivi": quant_kernel.sparse_decode_attention_quantized, "build": quant_kernel.build_quantized_kv_cache,
+             "quantize_k": lambda x, **kw: quant_kernel.quantize_k_cache(x, **kw),
+             "quantize_v": lambda x, **kw: quant_kernel.quantize_v_cache(x, **kw),
+             "step_attend": kivi_stream.KiviStreamBatch.step_attend}[fn]
+    if fn == "build":
+        a["k_compacted"], a["v_compacted"] = a.pop("k"), a.pop("v")
+    _same_error(monkeypatch, lambda: entry(**a))

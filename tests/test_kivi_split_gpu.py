@@ -1,7 +1,7 @@
-"""The wide KIVI decode over few KV heads, split over the GPU, and at
-per-sequence lengths: window-old group counts around the kernel's limits and
-uneven splits, steady state and ramp-up (some splits with no valid group),
-every workspace size, against the fp64 oracle."""
+"""The wide KIVI decode over few KV heads, split over the GPU, and (in one
+pass) at per-sequence lengths: window-old group counts around the kernel's and
+the plan's limits and uneven splits, steady state and ramp-up (fewer groups than
+the workspace was planned for), every workspace size, against the fp64 oracle."""
 
 import numpy as np
 import pytest
@@ -30,11 +30,14 @@ def _attend(q, c, L, W, S, device):
 
 
 @pytest.mark.parametrize("B,H,KVH", [(1, 64, 8), (3, 8, 8), (1, 12, 2), (40, 16, 2)])
-@pytest.mark.parametrize("groups,S", [(12, 4), (16, 1), (17, 16), (77, 4)])
-def test_split_over_few_heads(B, H, KVH, groups, S, device):
+@pytest.mark.parametrize("groups,S,splits", [(12, 4, 1), (16, 1, 1), (17, 16, 1), (29, 4, 3), (33, 16, 4), (77, 4, 9)])
+def test_split_over_few_heads(B, H, KVH, groups, S, splits, device):
+    import _kvdec as K
     W = 128 + 32 * groups
-    if B > 4 and groups > 20:
+    if B > 4 and groups > 40:
         pytest.skip("covered by the smaller batches")
+    # (a workgroup per CU: at most 3 splits of 80 KV heads)
+    assert K.lib.kvdec_num_splits(K.KIND_KIVI_SPLIT, B, KVH, W - 128) == min(splits, 256 // (B * KVH))
     q, hc, c = _problem(B, H, KVH, S, W, 40 + groups, device)
     for L in (163840, S + W - 7, S + W // 2, 100, 1):
         say(f"kivi split B={B} H={H} KVH={KVH} groups={groups} S={S} L={L}")

@@ -1,6 +1,7 @@
 """Splits shared out by the sequences' own lengths: lengths of nothing, of one
 token, of tiles' edges and of the whole context together; few and the most
-sequences that share, one more; lengths past the context (clamped)."""
+sequences that share, one more; lengths past the context (clamped).  Each case
+says whether its plan shares (2 to 64 sequences, splits of at least 64 tiles)."""
 
 import pytest
 import torch
@@ -26,20 +27,26 @@ def _check(o, q, k, v, lens):
         assert ((o[b].double() - ref).abs() - half_ulp).max().item() <= 2e-6, (b, n)
 
 
-@pytest.mark.parametrize("B,KVH,L,lens", [
-    (1, 2, 9000, [7001]),
-    (2, 8, 33000, [0, 33000]),
-    (3, 30, 5000, [1, 5000, 33]),
-    (4, 16, 9000, [9000, 9000, 9000, 9000]),
-    (5, 8, 15000, [0, 0, 0, 0, 0]),
-    (5, 8, 15000, [3000, 6000, 9000, 12000, 15000]),
-    (7, 16, 5000, [5000, 31, 32, 33, -5, 2049, 99999]),
-    (30, 8, 4500, None),
-    (64, 2, 4500, None),
-    (65, 2, 4500, None),
+@pytest.mark.parametrize("B,KVH,L,lens,shares", [
+    (1, 2, 9000, [7001], False),
+    (2, 8, 33000, [0, 33000], True),
+    (3, 30, 5000, [1, 5000, 33], False),
+    (3, 30, 6300, [1, 6300, 33], True),
+    (4, 16, 9000, [9000, 9000, 9000, 9000], True),
+    (5, 8, 15000, [0, 0, 0, 0, 0], True),
+    (5, 8, 15000, [3000, 6000, 9000, 12000, 15000], True),
+    (7, 16, 5000, [5000, 31, 32, 33, -5, 2049, 99999], False),
+    (7, 16, 6300, [6300, 31, 32, 33, -5, 2049, 99999], True),
+    (7, 16, 6300, [-2147483648, 2147483647, 1, 0, 6299, 6301, 64], True),
+    (30, 8, 4500, None, True),
+    (64, 2, 4500, None, True),
+    (65, 2, 4500, None, False),
 ])
-def test_dense_lengths(B, KVH, L, lens, device):
+def test_dense_lengths(B, KVH, L, lens, shares, device):
+    import _kvdec as K
     from dense_kernel import dense_decode_attention
+    splits, tiles = K.lib.kvdec_num_splits(K.KIND_DENSE, B, KVH, L), (L + 31) // 32
+    assert shares == (2 <= B <= 64 and splits > 1 and -(-tiles // splits) >= 64)
     g = torch.Generator(device=device).manual_seed(B)
     q = torch.randn((B, 4 * KVH, 128), generator=g, device=device, dtype=torch.float16)
     k, v = (torch.randn((B, KVH, L, 128), generator=g, device=device, dtype=torch.float16) for _ in range(2))
