@@ -1100,6 +1100,12 @@ __device__ __forceinline__ int max_field(uint32_t h2) {
     if (__ballot(el >= e + b)) e += b;
   return e;
 }
+// The fp16 bits of the power of two `span` exponents below the one of `field`
+// (0 where fp16 has none).
+__device__ __forceinline__ int span_bits(int field, int span) {
+  const int f = field - span;
+  return f > 0 ? f << 10 : f > -10 ? 1 << (9 + f) : 0;
+}
 // The power of two that V scales are multiplied by under v_field.
 __device__ __forceinline__ int v_shift(int v_field) { return 21 - v_field; }
 __device__ __forceinline__ uint32_t scale_pk(uint32_t h2, int k) {
@@ -1111,7 +1117,7 @@ template <int BITS>
 __device__ __forceinline__ void q_tile_stage_n(const QTileRawN<BITS>& X, char* slot, int lane, int slot0, int xlim,
                                                const SlotRanges& R, int& k_exp, int& v_field, QState& qs, uint64_t& far) {
   typedef QSlot<BITS> Lay;
-  const int kf = max_field(X.ks), k_least = max(kf - kKSpan, 0) << 10;
+  const int kf = max_field(X.ks), k_least = span_bits(kf, kKSpan);
   k_exp = 21 - kf;
   far |= __ballot((int)min(X.ks & 0x7FFFu, (X.ks >> 16) & 0x7FFFu) < k_least);
 #pragma unroll
@@ -1138,7 +1144,7 @@ __device__ __forceinline__ void q_tile_stage_n(const QTileRawN<BITS>& X, char* s
     v_field = vf;
   }
   // (0 - 1 wraps round to the largest)
-  const uint32_t v_least = max((uint32_t)max(v_field - kVSpan, 0) << 10, 1u) - 1u;
+  const uint32_t v_least = max((uint32_t)span_bits(v_field, kVSpan), 1u) - 1u;
   far |= __ballot(min((vs & 0x7FFFu) - 1u, ((vs >> 16) & 0x7FFFu) - 1u) < v_least);
   vs = scale_pk(vs, v_shift(v_field));
   *reinterpret_cast<uint16_t*>(slot + Lay::kVS + g0 * 64 + 2 * tok) = (uint16_t)vs;

@@ -177,12 +177,15 @@ def _relative(o, ref, dt):
 
 
 @pytest.mark.parametrize("bits,dt", [(4, "fp16"), (4, "bf16"), (2, "bf16")])
-@pytest.mark.parametrize("span", [8, 16, 17, 18, 24])
-def test_key_scales_far_apart(bits, dt, span, device):
-    """Every other channel's keys 2^span the others', its query as much smaller."""
+@pytest.mark.parametrize("span,at", [(8, 4), (16, 8), (17, 8), (18, 9), (24, 12), (17, 15), (20, 17)])
+def test_key_scales_far_apart(bits, dt, span, at, device):
+    """Every other channel's keys 2^span the others' (2^-at), its query as much
+    smaller; at the low ends the small scales are subnormal fp16."""
+    if dt == "fp16" and at > 12:
+        pytest.skip("no fp16 query makes so small a key count")
     B, H, KVH, S, W, R = 1, 16, 2, 4, 448, 128
     big = torch.arange(128) % 2 == 0
-    lo, hi = 2.0 ** -(span // 2), 2.0 ** (span - span // 2)
+    lo, hi = 2.0**-at, 2.0 ** (span - at)
     kc, vc, q = (torch.from_numpy(randn(n, i)) for n, i in
                  (((B, KVH, S + W, 128), 91), ((B, KVH, S + W, 128), 92), ((B, H, 128), 93)))
     kc = torch.where(big, kc * hi, kc * lo).to(DT[dt])
@@ -196,17 +199,17 @@ def test_key_scales_far_apart(bits, dt, span, device):
 
 
 @pytest.mark.parametrize("bits,dt", [(4, "fp16"), (4, "bf16"), (2, "bf16")])
-@pytest.mark.parametrize("span", [8, 10, 12, 20, 24])
-def test_value_scales_far_apart(bits, dt, span, device):
-    """Two tokens of weight 0 whose values are 2^span the others', and two whose
-    values are 0."""
+@pytest.mark.parametrize("span,at", [(8, 10), (10, 10), (12, 10), (20, 10), (24, 10), (14, 18)])
+def test_value_scales_far_apart(bits, dt, span, at, device):
+    """Two tokens of weight 0 whose values are 2^span the others' (2^-at), and
+    two whose values are 0."""
     B, H, KVH, S, W, R = 1, 16, 2, 4, 448, 128
     kc, vc, q = (torch.from_numpy(randn(n, i)) for n, i in
                  (((B, KVH, S + W, 128), 94), ((B, KVH, S + W, 128), 95), ((B, H, 128), 96)))
     q[..., 40] = 4
     out = [S + 5, S + 200]
     kc[:, :, out, 40] = -300
-    vc *= 2.0**-10
+    vc *= 2.0**-at
     vc[:, :, out] *= 2.0**span
     vc[:, :, [S + 9, S + 100]] = 0
     kc, vc, q = (x.to(DT[dt]) for x in (kc, vc, q))
