@@ -425,6 +425,9 @@ __device__ __forceinline__ Shares share_splits(const AttnCommon& P, int lane) {
 // 4c .. 4c + 3) steps all of its workgroup's slots.  Finite calls pay one
 // comparison of the merged values.  A KIVI workgroup whose scales lie too far
 // apart for two fp16 parts (q_tile_stage_n's `far`) goes the same way.
+// Bound by the latency of one wave's loads, eight slots at a time: with a NaN in
+// one query head, KIVI B=8, W=1024, 4-bit bf16 12.7 -> 261 us, bf16 dense B=4,
+// L=16411 45 -> 394 (four slots, each with its own waits: 389 and 577).
 // ---------------------------------------------------------------------------
 struct PlainState {
   float m = kMaxSentinel, l = 0.f;
@@ -459,37 +462,53 @@ __device__ __forceinline__ Args kernargs_again() {
   return a;
 }
 
-// x of lane L ^ N, N < 32 (no lane address to keep in a register).
-template <int N>
-__device__ __forceinline__ float swap_lane(float x) {
-  return __builtin_bit_cast(float, __builtin_amdgcn_ds_swizzle(__builtin_bit_cast(int, x), N << 10 | 0x1f));
+// Adds x of lane L ^ N, N < 32, to each x (no lane address to keep in a
+// register; all the swaps of a step are on their way before the first sum).
+template <int N, int K>
+__device__ __forceinline__ void half_wave_sum(float (&x)[K]) {
+  float y[K];
+#pragma unroll
+  for (int j = 0; j < K; ++j)
+    y[j] = __builtin_bit_cast(float, __builtin_amdgcn_ds_swizzle(__builtin_bit_cast(int, float(x[j])), N << 10 | 0x1f));
+#pragma unroll
+  for (int j = 0; j < K; ++j) x[j] += y[j];
 }
 
-// Slots lo .. hi - 1, four in flight; fetch(slot, k, v) reads the lane's
+// Slots lo .. hi - 1, eight in flight; fetch(slot, k, v) reads the lane's
 // channels of one slot in [lo, hi).
 template <class Fetch>
 __device__ __forceinline__ void plain_slots(Fetch&& fetch, int lo, int hi, const SlotRanges& R, float4v q,
                                             float scale_log2, PlainState& st) {
-  constexpr int kIn = 4;
+  constexpr int kIn = 8;
   for (int s0 = lo; s0 < hi; s0 += kIn) {
     float4v k[kIn], v[kIn];
 #pragma unroll
     for (int j = 0; j < kIn; ++j) fetch(min(s0 + j, hi - 1), k[j], v[j]);
+    float x[kIn], m = st.m;
+#pragma unroll
+    for (int j = 0; j < kIn; ++j)
+      x[j] = fmaf(q[3], k[j][3], fmaf(q[2], k[j][2], fmaf(q[1], k[j][1], q[0] * k[j][0])));
+    half_wave_sum<16>(x);
+    half_wave_sum<8>(x);
+    half_wave_sum<4>(x);
+    half_wave_sum<2>(x);
+    half_wave_sum<1>(x);
+#pragma unroll
+    for (int j = 0; j < kIn; ++j) {
+      x[j] = s0 + j < hi && slot_valid(R, s0 + j) ? x[j] * scale_log2 : -INFINITY;
+      m = fmaxf(m, x[j]);
+    }
+    const float alpha = exp2f(st.m - m);
+    st.m = m;
+    st.l *= alpha;
+    st.o *= alpha;
 #pragma unroll
     for (int j = 0; j < kIn; ++j) {
       const bool ok = s0 + j < hi && slot_valid(R, s0 + j);
-      float d = fmaf(q[3], k[j][3], fmaf(q[2], k[j][2], fmaf(q[1], k[j][1], q[0] * k[j][0])));
-      d += swap_lane<16>(d);
-      d += swap_lane<8>(d);
-      d += swap_lane<4>(d);
-      d += swap_lane<2>(d);
-      d += swap_lane<1>(d);
-      const float x = ok ? d * scale_log2 : -INFINITY, m = fmaxf(st.m, x);
-      const float alpha = exp2f(st.m - m), p = exp2f(x - m);
-      st.l = fmaf(st.l, alpha, p);
+      const float p = exp2f(x[j] - m);
+      st.l += p;
 #pragma unroll
-      for (int e = 0; e < 4; ++e) st.o[e] = fmaf(p, ok ? v[j][e] : 0.f, st.o[e] * alpha);
-      st.m = m;
+      for (int e = 0; e < 4; ++e) st.o[e] = fmaf(p, ok ? v[j][e] : 0.f, st.o[e]);
     }
   }
 }
@@ -2176,29 +2195,18 @@ __device__ __forceinline__ WideShare wide_share(const KiviWideArgs& A, uint32_t 
   return w;
 }
 
-// K and V of slot s of KV head `head`, channels 4 ch .. 4 ch + 3, in fp32.
-template <int BITS, int E>
-__device__ __forceinline__ void kivi_slot4(const KiviWideArgs& A, uint32_t head, int s, int ch, float4v& k,
-                                           float4v& v) {
+// K and V of a region's token `tok` (over all its KV heads), channels 4 ch ..
+// 4 ch + 3, in fp32.
+template <int BITS>
+__device__ __forceinline__ void quant_token4(const QRegion& Q, size_t tok, int ch, float4v& k, float4v& v) {
   constexpr int kPf = 8 / BITS;
-  const int win = kTile * A.nwt;
-  if (s >= A.sink + win) {
-    const size_t at = ((size_t)head * A.res_rows + (s - A.sink - win)) * kHeadDim + 4 * ch;
-    k = row4<E>(A.kres + at);
-    v = row4<E>(A.vres + at);
-    return;
-  }
-  const bool sk = s < A.sink;
-  const QRegion Q = sk ? A.sinkq : A.winq;
-  const int t = sk ? s : s - A.sink;                             // token of the region
-  const size_t tok = (size_t)head * (sk ? kTile : win) + t;      // over all heads
-  const uint32_t kc = *reinterpret_cast<const uint32_t*>(Q.kp + tok / kPf * kHeadDim + 4 * ch) >> (t % kPf * BITS);
+  constexpr uint32_t kMask = (1u << BITS) - 1u;
+  const uint32_t kc = *reinterpret_cast<const uint32_t*>(Q.kp + tok / kPf * kHeadDim + 4 * ch) >> (tok % kPf * BITS);
   const uint8_t* vp = Q.vp + tok * (kHeadDim / kPf) + 4 * ch / kPf;
   const uint32_t vc = BITS == 4 ? *reinterpret_cast<const uint16_t*>(vp) : *vp;
   const size_t km = tok / kTile * kHeadDim + 4 * ch, vm = tok * (kHeadDim / kTile) + ch / 8;
   const float4v ks = row4<kEltF16>(Q.ks + km), kz = row4<kEltF16>(Q.kz + km);
   const float vs = (float)Q.vs[vm], vz = (float)Q.vz[vm];
-  constexpr uint32_t kMask = (1u << BITS) - 1u;
 #pragma unroll
   for (int e = 0; e < 4; ++e) {
     k[e] = ks[e] * ((float)((kc >> (8 * e)) & kMask) - kz[e]);
@@ -2214,14 +2222,23 @@ __device__ __forceinline__ PlainState wide_plain(int hn, int ch) {
   const WideShare w = wide_share<SPLIT, VAR>(A, head);
   const float4v q = row4<E>(A.c.q + ((size_t)head * A.c.G + hn) * kHeadDim + 4 * ch);
   PlainState st;
-  auto step = [&](int lo, int hi) {
-    plain_slots([&](int s, float4v& k, float4v& v) { kivi_slot4<BITS, E>(A, head, s, ch, k, v); }, lo, hi, w.R, q,
-                A.c.scale_log2, st);
+  // slots lo .. hi - 1, slot s being token tok0 + s - lo of region Q
+  auto quantized = [&](const QRegion& Q, size_t tok0, int lo, int hi) {
+    plain_slots([&](int s, float4v& k, float4v& v) { quant_token4<BITS>(Q, tok0 + (s - lo), ch, k, v); }, lo, hi, w.R,
+                q, A.c.scale_log2, st);
   };
+  const size_t win0 = (size_t)head * kTile * A.nwt;
+  quantized(A.winq, win0 + kTile * w.g0, A.sink + kTile * w.g0, A.sink + kTile * w.g1);
+  if (!w.tail) return st;
+  quantized(A.sinkq, (size_t)head * kTile, 0, A.sink);
   const int res0 = A.sink + kTile * A.nwt;
-  step(A.sink + kTile * w.g0, A.sink + kTile * w.g1);
-  if (w.tail) step(res0, res0 + A.res_rows);
-  if (w.tail) step(0, A.sink);
+  plain_slots(
+      [&](int s, float4v& k, float4v& v) {
+        const size_t at = ((size_t)head * A.res_rows + (s - res0)) * kHeadDim + 4 * ch;
+        k = row4<E>(A.kres + at);
+        v = row4<E>(A.vres + at);
+      },
+      res0, res0 + A.res_rows, w.R, q, A.c.scale_log2, st);
   return st;
 }
 
