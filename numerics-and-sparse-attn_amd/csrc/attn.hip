@@ -2542,7 +2542,7 @@ __global__ __launch_bounds__(64 * kMergeWaves) void merge_kernel(AttnCommon P) {
       const int s = s0 + kMergeWaves * j;
       const size_t u = base + (size_t)(s < S ? s : 0) * P.G;
       a[j] = *reinterpret_cast<const float2v*>(wo + u * kHeadDim);
-      ms[j] = wm[u];
+      ms[j] = s < S ? wm[u] : -INFINITY;
       ls[j] = wl[u];
     }
   };
@@ -2557,10 +2557,21 @@ __global__ __launch_bounds__(64 * kMergeWaves) void merge_kernel(AttnCommon P) {
     if (s0 != wave) fetch(s0);
 #pragma unroll
     for (int j = 0; j < kIn; ++j) {
-      if (s0 + kMergeWaves * j >= S) break;   // past the last split (wave-uniform)
-      const float f = __builtin_amdgcn_exp2f(ms[j] - M);
+      const float f = __builtin_amdgcn_exp2f(ms[j] - M);   // 0 past the last split
       L += ls[j] * f;
       acc += a[j] * f;
+    }
+  }
+  // 0 times split 0's partial, where that one is infinite, is no zero: again
+  // without the places past the last split
+  if (__any(!(acc[0] == acc[0]) || !(acc[1] == acc[1]))) {
+    L = 0.f;
+    acc = float2v{0.f, 0.f};
+    for (int s = wave; s < S; s += kMergeWaves) {
+      const size_t u = base + (size_t)s * P.G;
+      const float f = __builtin_amdgcn_exp2f(wm[u] - M);
+      L += wl[u] * f;
+      acc += *reinterpret_cast<const float2v*>(wo + u * kHeadDim) * f;
     }
   }
   __shared__ float2v part[kMergeWaves][64];
