@@ -2986,7 +2986,8 @@ bool valid_attn_dtype(int dtype) { return dtype == KVDEC_F16 || dtype == KVDEC_F
 // groups of at most kPackGroup heads, a residual of at most 128 rows and a sink
 // of at most 16 tokens, when every tensor allows its 16-byte accesses and
 // 31-bit offsets.  Measured per step in a graph: B=8, W=1024, 4-bit bf16
-// 13.3 us, 2-bit bf16 12.3; W=128 7.6; B=32, W=2944 31.9 (2-bit fp16: 29.1);
+// 12.6 us, 2-bit bf16 12.0; W=128 6.7; B=32, W=2944 4-bit 32 to 33, 2-bit 27 to 29
+// (2-bit fp16: 26);
 // the generic kernel dequantizes value by value into fp32 products (4 bits, B=8,
 // W=1024: 51.2 us).  Other widths stay there: their codes are not the exact
 // fp8 values that codes_f16 widens.  What the factored products cannot give

@@ -1101,10 +1101,9 @@ __device__ __forceinline__ int max_field(uint32_t h2) {
   return e;
 }
 // The fp16 bits of the power of two `span` exponents below the one of `field`
-// (0 where fp16 has none).
-__device__ __forceinline__ int span_bits(int field, int span) {
-  const int f = field - span;
-  return f > 0 ? f << 10 : f > -10 ? 1 << (9 + f) : 0;
+// (0 where fp16 has none; formed as a float, so that no branch does it).
+__device__ __forceinline__ uint32_t span_bits(int field, int span) {
+  return __builtin_bit_cast(uint16_t, (_Float16)__builtin_ldexpf(1.0f, field - 15 - span));
 }
 // The power of two that V scales are multiplied by under v_field.
 __device__ __forceinline__ int v_shift(int v_field) { return 21 - v_field; }
@@ -1117,9 +1116,9 @@ template <int BITS>
 __device__ __forceinline__ void q_tile_stage_n(const QTileRawN<BITS>& X, char* slot, int lane, int slot0, int xlim,
                                                const SlotRanges& R, int& k_exp, int& v_field, QState& qs, uint64_t& far) {
   typedef QSlot<BITS> Lay;
-  const int kf = max_field(X.ks), k_least = span_bits(kf, kKSpan);
+  const int kf = max_field(X.ks);
   k_exp = 21 - kf;
-  far |= __ballot((int)min(X.ks & 0x7FFFu, (X.ks >> 16) & 0x7FFFu) < k_least);
+  const bool k_far = min(X.ks & 0x7FFFu, (X.ks >> 16) & 0x7FFFu) < span_bits(kf, kKSpan);
 #pragma unroll
   for (int i = 0; i < kQPieces<BITS>; ++i) {
     const int krow = 8 * i + (lane >> 3);
@@ -1144,8 +1143,8 @@ __device__ __forceinline__ void q_tile_stage_n(const QTileRawN<BITS>& X, char* s
     v_field = vf;
   }
   // (0 - 1 wraps round to the largest)
-  const uint32_t v_least = max((uint32_t)span_bits(v_field, kVSpan), 1u) - 1u;
-  far |= __ballot(min((vs & 0x7FFFu) - 1u, ((vs >> 16) & 0x7FFFu) - 1u) < v_least);
+  const uint32_t v_least = max(span_bits(v_field, kVSpan), 1u) - 1u;
+  far |= __ballot(k_far || min((vs & 0x7FFFu) - 1u, ((vs >> 16) & 0x7FFFu) - 1u) < v_least);
   vs = scale_pk(vs, v_shift(v_field));
   *reinterpret_cast<uint16_t*>(slot + Lay::kVS + g0 * 64 + 2 * tok) = (uint16_t)vs;
   *reinterpret_cast<uint16_t*>(slot + Lay::kVS + (g0 + 1) * 64 + 2 * tok) = (uint16_t)(vs >> 16);
