@@ -2987,12 +2987,12 @@ bool valid_attn_dtype(int dtype) { return dtype == KVDEC_F16 || dtype == KVDEC_F
 // of at most 16 tokens, when every tensor allows its 16-byte accesses and
 // 31-bit offsets.  Measured per step in a graph: B=8, W=1024, 4-bit bf16
 // 12.6 us, 2-bit bf16 12.0; W=128 6.7; B=32, W=2944 4-bit 32 to 33, 2-bit 27 to 29
-// (2-bit fp16: 26);
-// the generic kernel dequantizes value by value into fp32 products (4 bits, B=8,
-// W=1024: 51.2 us).  Other widths stay there: their codes are not the exact
-// fp8 values that codes_f16 widens.  What the factored products cannot give
-// (infinite zero points and scales, which caches of any width can hold) the
-// kernel's merge computes again in fp32 (wide_plain).
+// (2-bit fp16: 26); the generic kernel dequantizes value by value into fp32
+// products (4 bits, B=8, W=1024: 49.7 us).  Other widths stay there: their codes
+// are not the exact fp8 values that codes_f16 widens.  What the factored products
+// cannot give (infinite zero points and scales, which caches of any width can
+// hold, and scales far apart) the kernel's merge computes again in fp32
+// (wide_plain).
 template <int BITS, int E>
 int kivi_decode_wide(const void* q, const void* k_res, const void* v_res, const void* const* kivi, void* o,
                      const int32_t* lens, int64_t B, int32_t H, int32_t KVH, int64_t seq_len, int32_t window,

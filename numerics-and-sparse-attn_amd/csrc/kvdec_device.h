@@ -283,6 +283,8 @@ __device__ __forceinline__ uint32_t tile_valid_bits(const SlotRanges& R, int slo
 // bf16 rows take three bf16 parts, p = pB + pM + pL with 8 bits each (both
 // remainders are exact in fp32): p to ~2^-25, as a third MFMA per product of a
 // path whose time is its memory traffic.
+// (An infinite V is NaN against parts that are zero or negative; the bf16
+// kernels' merges compute a NaN result again in fp32.)
 template <int E = kEltF16>
 struct TileProbs {
   half8 pB, pL;

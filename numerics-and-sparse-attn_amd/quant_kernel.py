@@ -272,8 +272,9 @@ def build_quantized_kv_cache(k_compacted, v_compacted, residual_size=RESIDUAL_SI
     -> fp32 is exact, so the codes equal the quantizers' on those copies).
     The residual keeps the input dtype, as in the reference, unless
     residual_dtype says otherwise (torch.float16 turns an fp32 or bf16 cache
-    into what the fp16 fused decode reads; a bf16 or fp32 residual takes the
-    generic fp32 kernel).  A window shorter than residual_size
+    into what the fp16 fused decode reads; a bf16 residual runs on the matrix
+    cores under a bf16 query, a residual of another type than the query's or of
+    fp32 takes the generic fp32 kernel).  A window shorter than residual_size
     (undefined in the reference, whose slicing would then put sink slots into
     the residual) keeps the whole window as the residual and has no
     window-old part.
