@@ -1084,12 +1084,12 @@ __device__ __forceinline__ float q_tile_stage(const QTileRaw& raw, char* slot, i
 // subnormal range, for wide codes and small scales alike, and P' < 2^15 with
 // the softmax's slack.  (The 2-bit fp16 path scales Q alone: its remainders
 // below 2^-24 cost less than its codes' 0..3 carry into a result of order 1.)
-// The two parts end at 2^-25 whatever the scale: a product 2^-s of the largest
-// its head's |q| and the tile's scales allow (2^14) has s - 38 bits behind its
-// point.  `far` collects the tiles in which that leaves less than about 2^-22
-// of a head's largest term: a K scale more than kKSpan exponents below the
-// tile's largest (a head's largest |q| may stand on it), or a V scale other
-// than 0 more than kVSpan below v_field.
+// The two parts end at 2^-25 whatever the scale, so a product that lies 2^-s
+// below the 2^15 that its head's |q| and the tile's scales allow keeps 40 - s
+// bits.  `far` collects the tiles in which that may leave a head's largest term
+// fewer than about 22: a K scale more than kKSpan exponents below the tile's
+// largest (the head's largest |q| may stand on it), or a V scale other than 0
+// more than kVSpan below v_field.
 // Tokens of a tile that is not fully valid lose their V scale and zero: a slot
 // never written may hold any bits.
 constexpr int kKSpan = 16, kVSpan = 9;
